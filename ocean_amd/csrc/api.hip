@@ -504,60 +504,62 @@ int dev_nrm(H* h, const double2* p, double* v) {
 // ---------------------------------------------------------------------------
 // GMRES helpers
 // ---------------------------------------------------------------------------
-// <W_i|v1>, <W_i|v2> for i < m: partials [blk][i][4].  Eight W rows per pass with
-// all their loads in flight; the 32 sums of a pass reduce by one butterfly per
-// wave and one LDS round across the waves.
-__global__ __launch_bounds__(kBlock) void k_multidot2(const int* __restrict__ skip,
+// <W_i|v1>, <W_i|v2> for i < m: partials [i][4][eb].  Workgroup (row group, b) takes
+// eight rows of W over the elements of slice b, all its loads in flight; the 32 sums
+// reduce by one butterfly per wave and one LDS round across the waves.  The rows are
+// spread over the grid (not looped over in the workgroup), so that a short vector,
+// whose eb slices cannot fill the device, still runs its m rows at once: averages over
+// solves of up to 80 rows at 3 120 elements 11.3 -> 4.5 us, up to 100 rows at 131 072
+// elements 21.4 -> 18.4 us (4.8 TB/s; 34 us at 90 rows).
+constexpr int kDotRows = 8, kDotThreads = 256;
+__global__ __launch_bounds__(kDotThreads) void k_multidot2(const int* __restrict__ skip,
                                                       const double2* const* __restrict__ Wl, int m,
                                                       const double2* __restrict__ v1,
-                                                      const double2* __restrict__ v2, size_t n,
+                                                      const double2* __restrict__ v2, size_t n, int eb,
                                                       double* __restrict__ part) {
   if (*skip) return;
-  constexpr int R = 8;
-  __shared__ double lds[(kBlock / 64) * 4 * R];
+  constexpr int R = kDotRows;
+  __shared__ double lds[(kDotThreads / 64) * 4 * R];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int i0 = 0; i0 < m; i0 += R) {
-    double v[4 * R];
+  const int i0 = (blockIdx.x / eb) * R, b = blockIdx.x % eb;
+  double v[4 * R];
 #pragma unroll
-    for (int q = 0; q < 4 * R; ++q) v[q] = 0.0;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
-      const double2 b = v1[e], c = v2[e];
-      double2 a[R];
+  for (int q = 0; q < 4 * R; ++q) v[q] = 0.0;
+  const double2* row[R];
 #pragma unroll
-      for (int q = 0; q < R; ++q) a[q] = Wl[min(i0 + q, m - 1)][e];
+  for (int q = 0; q < R; ++q) row[q] = Wl[min(i0 + q, m - 1)];
+  for (size_t e = (size_t)b * blockDim.x + threadIdx.x; e < n; e += (size_t)eb * blockDim.x) {
+    const double2 b1 = v1[e], c1 = v2[e];
+    double2 a[R];
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        v[4 * q + 0] = fma(a[q].x, b.x, v[4 * q + 0]); v[4 * q + 0] = fma(a[q].y, b.y, v[4 * q + 0]);
-        v[4 * q + 1] = fma(a[q].x, b.y, v[4 * q + 1]); v[4 * q + 1] = fma(-a[q].y, b.x, v[4 * q + 1]);
-        v[4 * q + 2] = fma(a[q].x, c.x, v[4 * q + 2]); v[4 * q + 2] = fma(a[q].y, c.y, v[4 * q + 2]);
-        v[4 * q + 3] = fma(a[q].x, c.y, v[4 * q + 3]); v[4 * q + 3] = fma(-a[q].y, c.x, v[4 * q + 3]);
-      }
+    for (int q = 0; q < R; ++q) a[q] = row[q][e];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      v[4 * q + 0] = fma(a[q].x, b1.x, v[4 * q + 0]); v[4 * q + 0] = fma(a[q].y, b1.y, v[4 * q + 0]);
+      v[4 * q + 1] = fma(a[q].x, b1.y, v[4 * q + 1]); v[4 * q + 1] = fma(-a[q].y, b1.x, v[4 * q + 1]);
+      v[4 * q + 2] = fma(a[q].x, c1.x, v[4 * q + 2]); v[4 * q + 2] = fma(a[q].y, c1.y, v[4 * q + 2]);
+      v[4 * q + 3] = fma(a[q].x, c1.y, v[4 * q + 3]); v[4 * q + 3] = fma(-a[q].y, c1.x, v[4 * q + 3]);
     }
-    int owner = 0;
-    const double tot = og::wave_multi_sum<double, 4 * R>(v, lane, &owner);
-    if ((lane & (64 / (4 * R) - 1)) == 0) lds[wid * 4 * R + owner] = tot;
-    __syncthreads();
-    if (threadIdx.x < 4 * R) {
-      double sum = 0.0;
-      for (int w = 0; w < nw; ++w) sum += lds[w * 4 * R + threadIdx.x];
-      const int q = threadIdx.x >> 2;
-      if (i0 + q < m) part[((size_t)blockIdx.x * m + i0 + q) * 4 + (threadIdx.x & 3)] = sum;
-    }
-    __syncthreads();
+  }
+  int owner = 0;
+  const double tot = og::wave_multi_sum<double, 4 * R>(v, lane, &owner);
+  if ((lane & (64 / (4 * R) - 1)) == 0) lds[wid * 4 * R + owner] = tot;
+  __syncthreads();
+  if (threadIdx.x < 4 * R && i0 + (int)(threadIdx.x >> 2) < m) {
+    double sum = 0.0;
+    for (int w = 0; w < nw; ++w) sum += lds[w * 4 * R + threadIdx.x];
+    part[(size_t)(4 * i0 + threadIdx.x) * eb + b] = sum;
   }
 }
 
-// out[j] = sum_b part[b*nv + j]: one wave per value, lane-strided partial sums
-// then a butterfly (fixed order, so every run gives the same bits).
-__global__ void k_multifinish(const int* __restrict__ skip, const double* __restrict__ part, int nblk, int nv,
-                              double* __restrict__ out) {
-  // the flag is read with the partials (one round trip) and tested before the store
-  const int sk = *skip;
-  const int lane = threadIdx.x & 63;
-  const int j = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (j >= nv) return;
-  const double s = og::wave_sum_parts(part, nblk, nv, j, lane);
-  if (lane == 0 && !sk) out[j] = s;
+// Element slices of k_multidot2: with the row groups about a thousand workgroups (four
+// per compute unit; 64 slices of 1024 threads took 21.8 against 18.4 us at 131 072
+// elements and 7.9 against 4.5 us at 3 120), at most one per
+// kDotThreads elements and kRedBlocks in all.
+int dot_slices(size_t n, int m) {
+  const int ng = (m + kDotRows - 1) / kDotRows;
+  const size_t full = (n + kDotThreads - 1) / kDotThreads;
+  return (int)std::min<size_t>({full, (size_t)kRedBlocks, (size_t)(1024 / ng)});
 }
 
 // x += sum_i C_i U_i over the cycle's cumulative least-squares coefficients (the sum of
@@ -595,174 +597,258 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const int* __restrict__ 
 // Least-squares step of update_gmres on the device (OCEAN_gmres.f90:241-344).
 // The Gram matrix grows by one bordered row per call (cur = 1, 2, ... after every
 // restart or recycled energy), so its LDL^H factor (no pivoting) grows by one row:
-//   L(j,k) = (C(j,k) - sum_{m<k} L(j,m) conj(L(k,m)) D(m)) / D(k),  k < j = cur-1
-//   D(j)   =  C(j,j) - sum_{k<j} L(j,k) conj(L(j,k)) D(k)
+//   t(k)   = C(j,k) - sum_{m<k} t(m) conj(L(k,m)),  L(j,k) = t(k) / D(k),  k < j = cur-1
+//   D(j)   = C(j,j) - sum_{k<j} L(j,k) conj(L(j,k)) D(k)
 // with D and the strictly lower triangle of L (packed row by row: L(i, k) at
 // i (i - 1) / 2 + k) kept in global memory between calls; then coef = -C^-1 <au|g> by
-// the two triangular solves.  One wave: lane l owns indices l, l + 64, .. (kLsSlots of
-// them), and every triangular sweep is right-looking, so each of its cur steps is
-// one broadcast of the finished value plus one FMA per owned index; the strictly
-// lower triangle of L is staged in LDS (packed rows) when it fits, otherwise read
-// from global memory.  A zero pivot leaves its 1-based index in *info (zhptrf's
-// info) and the coefficients at 0.  The coefficients are also added to the cycle's
-// cumulative ones C (x = x_b + sum_i C_i U_i, formed when the basis is replaced).
-constexpr int kLsSlots = 4;
-constexpr int kMaxGmresDepth = 64 * kLsSlots;
-constexpr int kLsPacked = 3916;  // LDS-staged rows 1 .. cur-2: (cur-2)(cur-1)/2 entries, cur <= 90
+// the two triangular solves.  One workgroup: its waves sum the eb partials of
+// k_multidot2 (a fixed order, so every run gives the same bits) and stage L in LDS
+// (packed rows: column k over consecutive rows falls on distinct banks, a row is
+// contiguous); then one wave runs the sweeps, lane l owning indices l, l + 64, ...
+// What bounds it is the serial chain of the sweeps.  Row j of the factor and the
+// forward solve take the same columns of L in the same order, so they share one
+// sweep; a step of it is four lane reads and two dependent FMAs per value, with the
+// columns of L loaded four steps ahead and the divisions by D outside of the chain
+// (t = L D is what the sweep carries).  Averages over solves of up to 80 rows at 3 120
+// elements: 31.3 + 3.9 us in two kernels -> 9.5 us; up to 100 rows at 131 072: 40.1 + 4.9
+// -> 12.7 us (5 us at 8 rows, 15 at 64, 26 at 100).
+// A zero pivot leaves its 1-based index in *info (zhptrf's info) and the coefficients
+// at 0.  The coefficients are also added to the cycle's cumulative ones C
+// (x = x_b + sum_i C_i U_i, formed when the basis is replaced).
+constexpr int kMaxGmresDepth = 256;
 
-__device__ __forceinline__ double2 ls_bcast(const double2 (&v)[kLsSlots], int k) {
-  const int q = k >> 6, src = k & 63;
-  double2 s = v[0];
-#pragma unroll
-  for (int i = 1; i < kLsSlots; ++i)
-    if (q == i) s = v[i];
-  return make_double2(__shfl(s.x, src, 64), __shfl(s.y, src, 64));
+__device__ __forceinline__ double lane_read(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ double2 lane_read(double2 v, int l) {
+  return make_double2(lane_read(v.x, l), lane_read(v.y, l));
 }
 
-__global__ __launch_bounds__(64) void k_ls_update(int* __restrict__ skip, const double* __restrict__ fin,
-                                                  double2* __restrict__ L, double* __restrict__ D,
-                                                  double2* __restrict__ coef, double2* __restrict__ C, int cur,
-                                                  int depth, int* __restrict__ info) {
-  // every input is loaded before the flag is tested, so the flag, the Gram column
-  // and the stored factor arrive in one round trip
-  const int sk = *skip;
-  __shared__ double2 Ls[kLsPacked];
-  __shared__ double Dl[kMaxGmresDepth];
-  const int lane = threadIdx.x;
+// The sweeps of one wave for cur <= 64 NS.  Lat(i, k, ok) = L(i, k), k < i < j, or 0
+// where ok is not set; fin the 4 cur
+// sums (<au_k|au_j>, <au_k|g>), Dl the pivots of rows 0 .. j - 1.
+template <int NS, typename Lf>
+__device__ __forceinline__ void ls_sweeps(Lf Lat, const double* fin, const double* Dl, double2* __restrict__ L,
+                                          double* __restrict__ D, double2* __restrict__ coef,
+                                          double2* __restrict__ C, int cur, int* __restrict__ skip,
+                                          int* __restrict__ info) {
+  constexpr int P = NS == 1 ? 4 : NS == 2 ? 2 : 1;  // columns (rows in the backward sweep) of L loaded ahead
+  const int lane = threadIdx.x & 63;
   const int j = cur - 1;
-  const int npk = j * (j - 1) / 2;  // strictly lower rows 1 .. j - 1, packed row by row
-  const bool in_lds = npk <= kLsPacked;
-  // C(j, k) = conj(<au_k|au_j>) for k < j (the lower triangle of the Hermitian
-  // matrix whose upper column j holds <au_k|au_j>); C(j, j) = |au_j|^2; the
-  // right-hand side -<au_i|g>; D(0 .. j-1)
-  double2 t[kLsSlots], lj[kLsSlots], r[kLsSlots];
-  double dv[kLsSlots];
+  // C(j, k) = conj(<au_k|au_j>) for k < j (the lower triangle of the Hermitian matrix
+  // whose upper column j holds <au_k|au_j>); C(j, j) = |au_j|^2; the right-hand side
+  // -<au_i|g>
+  double2 t[NS], r[NS], c0[NS];
+  double d[NS];
 #pragma unroll
-  for (int q = 0; q < kLsSlots; ++q) {
+  for (int q = 0; q < NS; ++q) {
     const int i = lane + 64 * q;
     t[q] = i < j ? make_double2(fin[4 * i], -fin[4 * i + 1]) : make_double2(0.0, 0.0);
     r[q] = i < cur ? make_double2(-fin[4 * i + 2], -fin[4 * i + 3]) : make_double2(0.0, 0.0);
-    dv[q] = i < j ? D[i] : 0.0;
-    lj[q] = make_double2(0.0, 0.0);
+    d[q] = i < j ? Dl[i] : 1.0;
+    c0[q] = i < cur ? C[i] : make_double2(0.0, 0.0);
   }
-  // rows 1 .. j - 1 of L (contiguous in the packed layout); row j is formed here and
-  // kept in registers.  The first four loads per lane are issued with the others.
-  double2 v0[4];
+  const double cjj = fin[4 * j];
+  // forward: after step k, t(k) and r(k) are final and update every later index
 #pragma unroll
-  for (int q = 0; q < 4; ++q) v0[q] = L[min(lane + 64 * q, max(npk - 1, 0))];
-  if (sk) return;
-  if (in_lds) {
+  for (int kb = 0; kb < NS; ++kb) {
+    const int k0 = 64 * kb, k1 = min(j, k0 + 64);
+    double2 X[P][NS], Y[P][NS];
+    auto cols = [&](double2 (&B)[P][NS], int k) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (lane + 64 * q < npk) Ls[lane + 64 * q] = v0[q];
-    for (int e0 = lane + 4 * 64; e0 < npk; e0 += 4 * 64) {
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int q = kb; q < NS; ++q) {
+          const int i = lane + 64 * q;
+          B[p][q] = Lat(i, k + p, i > k + p && i < j && k + p < k1);
+        }
+    };
+    auto step = [&](const double2 (&B)[P][NS], int k) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const int src = (k + p) & 63;
+        const double2 tk = lane_read(t[kb], src), rk = lane_read(r[kb], src);
+#pragma unroll
+        for (int q = kb; q < NS; ++q) {
+          const double2 b = B[p][q];
+          t[q].x = fma(-tk.x, b.x, t[q].x); t[q].x = fma(-tk.y, b.y, t[q].x);  // t conj(b)
+          t[q].y = fma(-tk.y, b.x, t[q].y); t[q].y = fma(tk.x, b.y, t[q].y);
+          r[q].x = fma(-rk.x, b.x, r[q].x); r[q].x = fma(rk.y, b.y, r[q].x);   // b r
+          r[q].y = fma(-rk.y, b.x, r[q].y); r[q].y = fma(-rk.x, b.y, r[q].y);
+        }
+      }
+    };
+    cols(X, k0);
+#pragma unroll 1
+    for (int k = k0; k < k1; k += 2 * P) {
+      cols(Y, k + P);
+      step(X, k);
+      cols(X, k + 2 * P);
+      step(Y, k + P);
+    }
+  }
+  // row j of L, its pivot, and the forward solve's last value
+  double2 lj[NS];
+  double ds = 0.0, sx = 0.0, sy = 0.0;
+#pragma unroll
+  for (int q = 0; q < NS; ++q) {
+    const int i = lane + 64 * q;
+    lj[q] = make_double2(0.0, 0.0);
+    if (i < j) {
+      lj[q] = make_double2(t[q].x / d[q], t[q].y / d[q]);
+      L[(size_t)j * (j - 1) / 2 + i] = lj[q];
+      ds += (lj[q].x * lj[q].x + lj[q].y * lj[q].y) * d[q];
+      sx += lj[q].x * r[q].x - lj[q].y * r[q].y;
+      sy += lj[q].x * r[q].y + lj[q].y * r[q].x;
+    }
+  }
+  const double dj = cjj - og::wave_sum(ds);
+  sx = og::wave_sum(sx);
+  sy = og::wave_sum(sy);
+  int bad = 0;
+#pragma unroll
+  for (int q = NS - 1; q >= 0; --q) {
+    const int i = lane + 64 * q;
+    if (i == j) {
+      d[q] = dj;
+      D[j] = dj;
+      r[q].x -= sx;
+      r[q].y -= sy;
+    }
+    const unsigned long long z = __ballot(i < cur && d[q] == 0.0);
+    if (z) bad = 64 * q + __ffsll((long long)z);
+  }
+  if (bad) {
+    if (lane == 0) {
+      *info = bad;
+      *skip = 2;  // the solve stops here: later enqueued work is dropped
+    }
+    for (int i = lane; i < cur; i += 64) coef[i] = make_double2(0.0, 0.0);
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < NS; ++q)
+    if (lane + 64 * q < cur) { r[q].x /= d[q]; r[q].y /= d[q]; }
+  // backward: L^H coef = r; row j from the registers of its owners
+  auto back = [&](double2& z, double2 l, double2 v) {  // z -= conj(l) v
+    z.x = fma(-l.x, v.x, z.x); z.x = fma(-l.y, v.y, z.x);
+    z.y = fma(-l.x, v.y, z.y); z.y = fma(l.y, v.x, z.y);
+  };
+  {
+    double2 v = r[0];
+#pragma unroll
+    for (int q = 1; q < NS; ++q)
+      if ((j >> 6) == q) v = r[q];
+    v = lane_read(v, j & 63);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) back(r[q], lj[q], v);
+  }
+#pragma unroll
+  for (int kb = NS - 1; kb >= 0; --kb) {
+    const int k0 = max(64 * kb, 1), k1 = min(j - 1, 64 * kb + 63);
+    double2 X[P][NS], Y[P][NS];
+    auto rows = [&](double2 (&B)[P][NS], int k) {
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int q = 0; q <= kb; ++q) {
+          const int i = lane + 64 * q;
+          B[p][q] = Lat(k - p, i, i < k - p && k - p >= k0);
+        }
+    };
+    auto step = [&](const double2 (&B)[P][NS], int k) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const double2 v = lane_read(r[kb], (k - p) & 63);
+#pragma unroll
+        for (int q = 0; q <= kb; ++q) back(r[q], B[p][q], v);
+      }
+    };
+    rows(X, k1);
+#pragma unroll 1
+    for (int k = k1; k >= k0; k -= 2 * P) {
+      rows(Y, k - P);
+      step(X, k);
+      rows(X, k - 2 * P);
+      step(Y, k - P);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NS; ++q) {
+    const int i = lane + 64 * q;
+    if (i < cur) {
+      coef[i] = r[q];
+      C[i] = make_double2(c0[q].x + r[q].x, c0[q].y + r[q].y);
+    }
+  }
+}
+
+// LDS of k_ls_update: the sums, the pivots and, where it fits, the packed factor (up to
+// 141 rows in 160 KB; past that the sweeps read L from global memory).
+size_t ls_lds(int cur, bool with_L) {
+  const size_t j = (size_t)cur - 1;
+  return (4 * (size_t)cur + cur + (cur & 1)) * sizeof(double) + (with_L ? (j * (j - 1) / 2 + 1) * sizeof(double2) : 0);
+}
+
+constexpr int kLsThreads = 1024;
+
+template <bool kInLds>
+__global__ __launch_bounds__(kLsThreads) void k_ls_update(int* __restrict__ skip, const double* __restrict__ part, int eb,
+                                                    double2* __restrict__ L, double* __restrict__ D,
+                                                    double2* __restrict__ coef, double2* __restrict__ C, int cur,
+                                                    int* __restrict__ info) {
+  extern __shared__ __align__(16) double lsmem[];
+  double* fin = lsmem;                  // [4 cur]
+  double* Dl = fin + 4 * cur;           // [cur], padded to an even count
+  double2* Ls = reinterpret_cast<double2*>(Dl + cur + (cur & 1));
+  const int sk = *skip;  // tested after the loads below are under way
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int j = cur - 1, nv = 4 * cur;
+  const int npk = j * (j - 1) / 2;
+  if constexpr (kInLds) {
+    for (int e0 = threadIdx.x; e0 < npk; e0 += 4 * blockDim.x) {
       double2 v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = L[min(e0 + 64 * q, npk - 1)];
+      for (int q = 0; q < 4; ++q) v[q] = L[min(e0 + q * (int)blockDim.x, npk - 1)];
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (e0 + 64 * q < npk) Ls[e0 + 64 * q] = v[q];
+        if (e0 + q * (int)blockDim.x < npk) Ls[e0 + q * blockDim.x] = v[q];
     }
+    if (threadIdx.x == 0) Ls[npk] = make_double2(0.0, 0.0);
   }
+  for (int e = threadIdx.x; e < j; e += blockDim.x) Dl[e] = D[e];
+  constexpr int V = 8, S = kRedBlocks / 64;  // sums per wave and pass; loads per sum and lane
+  for (int v0 = wid * V; v0 < nv; v0 += nw * V) {
+    double p[S][V], s[V];
 #pragma unroll
-  for (int q = 0; q < kLsSlots; ++q)
-    if (lane + 64 * q < j) Dl[lane + 64 * q] = dv[q];
+    for (int c = 0; c < S; ++c)
+      if (64 * c < eb)
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+          p[c][q] = part[(size_t)min(v0 + q, nv - 1) * eb + min(lane + 64 * c, eb - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      s[q] = 0.0;
+#pragma unroll
+      for (int c = 0; c < S; ++c)
+        if (lane + 64 * c < eb) s[q] += p[c][q];
+    }
+    int owner = 0;
+    const double tot = og::wave_multi_sum<double, V>(s, lane, &owner);
+    if ((lane & (64 / V - 1)) == 0 && v0 + owner < nv) fin[v0 + owner] = tot;
+  }
+  if (sk) return;
   __syncthreads();
-  // The sweeps, compiled once for L staged in LDS and once for L in global memory: a
-  // run-time choice between the two address spaces would make every L read a flat
-  // load that waits on the vector memory counter inside the serial sweeps.
-  auto sweeps = [&](auto in_lds_tag) {
-    constexpr bool kInLds = decltype(in_lds_tag)::value;
-    auto Lat = [&](int i, int k) -> double2 {  // L(i, k), k < i < j
-      if constexpr (kInLds) return Ls[i * (i - 1) / 2 + k];
-      else return L[(size_t)i * (i - 1) / 2 + k];
-    };
-    // row j: after step k, t(k) is final and L(j, k) = t(k) / D(k) updates every t(kk), kk > k
-    double dsum = 0.0;
-    for (int k = 0; k < j; ++k) {
-      const double2 tk = ls_bcast(t, k);
-      const double dk = Dl[k];
-      const double2 a = make_double2(tk.x / dk, tk.y / dk);
-      if (lane == 0) dsum -= (a.x * a.x + a.y * a.y) * dk;
-  #pragma unroll
-      for (int q = 0; q < kLsSlots; ++q) {
-        const int kk = lane + 64 * q;
-        if (kk == k) lj[q] = a;
-        if (kk > k && kk < j) {
-          const double2 b = Lat(kk, k);
-          // a * conj(b) * d
-          t[q].x -= (a.x * b.x + a.y * b.y) * dk;
-          t[q].y -= (a.y * b.x - a.x * b.y) * dk;
-        }
-      }
-    }
-  #pragma unroll
-    for (int q = 0; q < kLsSlots; ++q) {
-      const int k = lane + 64 * q;
-      if (k < j) L[(size_t)npk + k] = lj[q];  // row j at j (j - 1) / 2
-    }
-    if (lane == 0) {
-      const double dj = fin[4 * j] + dsum;
-      D[j] = dj;
-      Dl[j] = dj;
-    }
-    __syncthreads();
-    int bad = 0;
-    for (int k = 0; k <= j; ++k)
-      if (Dl[k] == 0.0) { bad = k + 1; break; }
-    if (bad) {
-      if (lane == 0) {
-        *info = bad;
-        *skip = 2;  // the solve stops here: later enqueued work is dropped
-      }
-      for (int i = lane; i < cur; i += 64) coef[i] = make_double2(0.0, 0.0);
-      return;
-    }
-    // coef = -C^-1 rvec: L y = -rvec, then D, then L^H coef = y (row j of L from the
-    // registers of its owners)
-    for (int k = 0; k < cur; ++k) {
-      const double2 v = ls_bcast(r, k);
-      const double2 ljk = ls_bcast(lj, k);
-  #pragma unroll
-      for (int q = 0; q < kLsSlots; ++q) {
-        const int i = lane + 64 * q;
-        if (i > k && i < cur) {
-          const double2 l = i == j ? ljk : Lat(i, k);
-          r[q].x -= l.x * v.x - l.y * v.y;
-          r[q].y -= l.x * v.y + l.y * v.x;
-        }
-      }
-    }
-  #pragma unroll
-    for (int q = 0; q < kLsSlots; ++q) {
-      const int i = lane + 64 * q;
-      if (i < cur) { r[q].x /= Dl[i]; r[q].y /= Dl[i]; }
-    }
-    for (int k = cur - 1; k > 0; --k) {
-      const double2 v = ls_bcast(r, k);
-  #pragma unroll
-      for (int q = 0; q < kLsSlots; ++q) {
-        const int i = lane + 64 * q;
-        if (i < k) {
-          const double2 l = k == j ? lj[q] : Lat(k, i);  // conj(l) * v
-          r[q].x -= l.x * v.x + l.y * v.y;
-          r[q].y -= l.x * v.y - l.y * v.x;
-        }
-      }
-    }
-  #pragma unroll
-    for (int q = 0; q < kLsSlots; ++q) {
-      const int i = lane + 64 * q;
-      if (i < cur) {
-        coef[i] = r[q];
-        double2 ci = C[i];
-        ci.x += r[q].x; ci.y += r[q].y;
-        C[i] = ci;
-      }
-    }
+  if (wid != 0) return;
+  auto Lat = [&](int i, int k, bool ok) -> double2 {
+    if constexpr (kInLds) return Ls[ok ? i * (i - 1) / 2 + k : npk];  // a zero past the factor
+    else return ok ? L[(size_t)i * (i - 1) / 2 + k] : make_double2(0.0, 0.0);
   };
-  if (in_lds) sweeps(std::true_type{});
-  else sweeps(std::false_type{});
+  if (cur <= 64) ls_sweeps<1>(Lat, fin, Dl, L, D, coef, C, cur, skip, info);
+  else if (cur <= 128) ls_sweeps<2>(Lat, fin, Dl, L, D, coef, C, cur, skip, info);
+  else ls_sweeps<4>(Lat, fin, Dl, L, D, coef, C, cur, skip, info);
 }
 
 // pcdiv = (E - (h1_r + i(h1_i + g))) / ((E - h1)^2 + g^2)  (OCEAN_psi_min_set_prec, :2907-2994)
@@ -818,7 +904,7 @@ __global__ void k_axpy_gated(const int* __restrict__ skip, double ar, double ai,
 // next action's projection.  (A last-workgroup-to-arrive finish inside the kernels
 // serialised a device-scope atomic per workgroup.)
 __device__ __forceinline__ void resid_part(double (&v)[3], double* __restrict__ part) {
-  __shared__ double lds[4 * 3];
+  __shared__ double lds[16 * 3];  // one slot per wave, up to 1024 threads
   og::block_sum<3>(v, lds);
   if (threadIdx.x == 0) {
     part[3 * blockIdx.x] = v[0]; part[3 * blockIdx.x + 1] = v[1]; part[3 * blockIdx.x + 2] = v[2];
@@ -873,63 +959,72 @@ __global__ __launch_bounds__(kBlock) void k_pc_apply(GmCtl* __restrict__ c, doub
   resid_part(v, part);
 }
 
-// ax += sum_i c_i AU_i (update_gmres, OCEAN_gmres.f90:336-341; eight rows per step
-// with their loads in flight, the sum in i order), then in the same pass the residual
-// step: g = ax - rhs, |g|^2, the next basis vector unext = g . pc (nullable) and the
-// partials of <rhs|unext>; k_resid_fin (kResU) forms <rhs|x> from the cumulative
-// coefficients C (already holding this update) without forming x.
-__global__ __launch_bounds__(kBlock) void k_axpy_resid(GmCtl* __restrict__ c, const double2* const* __restrict__ AUl,
-                                                       const double2* __restrict__ coef, int m,
-                                                       double2* __restrict__ ax, const double2* __restrict__ rhs,
-                                                       double2* __restrict__ g, const double2* __restrict__ pc,
-                                                       double2* __restrict__ unext, size_t n,
-                                                       double* __restrict__ part) {
+// ax += sum_i c_i AU_i (update_gmres, OCEAN_gmres.f90:336-341), then in the same pass
+// the residual step: g = ax - rhs, |g|^2, the next basis vector unext = g . pc
+// (nullable) and the partials of <rhs|unext>; k_resid_fin (kResU) forms <rhs|x> from
+// the cumulative coefficients C (already holding this update) without forming x.
+// A workgroup of 1024 threads takes 1024 / RS elements at a time, its waves in RS
+// groups that each sum a contiguous share of the rows (eight loads in flight per
+// wave); the shares are added in LDS in order.  With the rows of an element on one
+// thread the kernel waited on m / 8 dependent rounds of loads with one wave per SIMD:
+// averages over solves of up to 80 rows at 3 120 elements 9.4 -> 5.8 us, up to 100 rows
+// at 131 072 elements 19.1 us as before (36 us at 90 rows, 5.2 TB/s).
+constexpr int kAxThreads = 1024;
+template <int RS>
+__global__ __launch_bounds__(kAxThreads) void k_axpy_resid(GmCtl* __restrict__ c,
+                                                           const double2* const* __restrict__ AUl,
+                                                           const double2* __restrict__ coef, int m,
+                                                           double2* __restrict__ ax, const double2* __restrict__ rhs,
+                                                           double2* __restrict__ g, const double2* __restrict__ pc,
+                                                           double2* __restrict__ unext, size_t n,
+                                                           double* __restrict__ part) {
+  constexpr int EPB = kAxThreads / RS, R = 8;
+  __shared__ double2 red[RS][EPB];
   // the flag is read with the first loads and tested before the first store
   const int done = c->done;
-  constexpr int R = 8;
+  const int el = threadIdx.x % EPB;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x / EPB);
+  const int ch = (m + RS - 1) / RS, ia = s * ch, ib = min(m, ia + ch);
   double v[3] = {0, 0, 0};
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  const double2 z = make_double2(0.0, 0.0);
-  // two elements (e0 and e0 + stride, the grid-stride order) per step, so that twice
-  // the rows are in flight
-  for (size_t e0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e0 < n; e0 += 2 * stride) {
-    const size_t e1 = e0 + stride;
-    const bool has1 = e1 < n;
-    double2 av0 = ax[e0], av1 = has1 ? ax[e1] : z;
-    for (int i0 = 0; i0 < m; i0 += R) {
-      double2 a0[R], a1[R];
+  for (size_t e0 = (size_t)blockIdx.x * EPB; e0 < n; e0 += (size_t)gridDim.x * EPB) {
+    const size_t e = e0 + el;
+    const size_t ec = e < n ? e : n - 1;
+    double2 av = make_double2(0.0, 0.0), bv = av, pv = av;
+    if (s == 0) {
+      av = ax[ec];
+      bv = rhs[ec];
+      if (unext) pv = pc[ec];
+    }
+    double2 sum = make_double2(0.0, 0.0);
+    for (int i0 = ia; i0 < ib; i0 += R) {
+      double2 a[R];
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const double2* row = AUl[min(i0 + q, m - 1)];
-        a0[q] = row[e0];
-        a1[q] = has1 ? row[e1] : z;
-      }
+      for (int q = 0; q < R; ++q) a[q] = AUl[min(i0 + q, ib - 1)][ec];
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        if (i0 + q < m) {
-          const double2 ci = coef[i0 + q];
-          av0.x += ci.x * a0[q].x; av0.y += ci.x * a0[q].y;
-          av0.x += -ci.y * a0[q].y; av0.y += ci.y * a0[q].x;
-          av1.x += ci.x * a1[q].x; av1.y += ci.x * a1[q].y;
-          av1.x += -ci.y * a1[q].y; av1.y += ci.y * a1[q].x;
-        }
-      }
+      for (int q = 0; q < R; ++q)
+        if (i0 + q < ib) og::cfma(sum, coef[i0 + q], a[q]);
     }
     if (done) return;
+    red[s][el] = sum;
+    __syncthreads();
+    if (s == 0 && e < n) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const size_t e = h ? e1 : e0;
-      if (h && !has1) break;
-      const double2 av = h ? av1 : av0;
+      for (int q = 0; q < RS; ++q) {
+        const double2 w = red[q][el];
+        av.x += w.x;
+        av.y += w.y;
+      }
       ax[e] = av;
-      const double2 b = resid_g(e, av, rhs, g, v[0]);
+      const double2 gv = make_double2(av.x - bv.x, av.y - bv.y);
+      g[e] = gv;
+      v[0] = fma(gv.x, gv.x, v[0]); v[0] = fma(gv.y, gv.y, v[0]);
       if (unext) {
-        const double2 gv = make_double2(av.x - b.x, av.y - b.y);
-        const double2 uv = og::cmul(gv, pc[e]);
+        const double2 uv = og::cmul(gv, pv);
         unext[e] = uv;
-        dot_term(b, uv, v[1], v[2]);
+        dot_term(bv, uv, v[1], v[2]);
       }
     }
+    __syncthreads();
   }
   if (done) return;
   resid_part(v, part);
@@ -2234,10 +2329,10 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   // g = ax - rhs with x materialised, its sums and (with check) the stopping test of
   // iteration it
   double* rpart = part + (size_t)kRedBlocks * 4 * depth + 4 * (size_t)depth;
-  auto fin_of = [&](int it, int check, int mode, int m, int slot) -> GmFin {
+  auto fin_of = [&](int it, int check, int mode, int m, int slot, int nblk = kRedBlocks) -> GmFin {
     GmFin F{};
     F.c = ctl; F.part = rpart; F.C = dC; F.rU = dRU; F.ffff = ffff;
-    F.nblk = kRedBlocks; F.it = it; F.check = check; F.mode = mode; F.m = m; F.slot = slot;
+    F.nblk = nblk; F.it = it; F.check = check; F.mode = mode; F.m = m; F.slot = slot;
     return F;
   };
   auto resid = [&](int it, int check) -> int {
@@ -2250,14 +2345,26 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   // of iteration rit, and unext (nullable) receives the next basis vector U[cur];
   // without, the update ends a cycle: x is materialised (ax is recomputed from it)
   auto update = [&](int cur, int rit = -1, int check = 0, double2* unext = nullptr) -> int {
-    k_multidot2<<<kRedBlocks, kBlock, 0, st>>>(skip, (const double2* const*)dlist, cur, AU[cur - 1], g, nv, part);
-    double* fin = part + (size_t)kRedBlocks * 4 * depth;
-    k_multifinish<<<(4 * cur + 3) / 4, 256, 0, st>>>(skip, part, kRedBlocks, 4 * cur, fin);
-    k_ls_update<<<1, 64, 0, st>>>(skip, fin, dL, dD, dcoef, dC, cur, depth, info);
+    const int eb = dot_slices(nv, cur);
+    k_multidot2<<<eb * ((cur + kDotRows - 1) / kDotRows), kDotThreads, 0, st>>>(
+        skip, (const double2* const*)dlist, cur, AU[cur - 1], g, nv, eb, part);
+    const size_t sm = ls_lds(cur, true);
+    if (sm <= h->lds_max) {
+      OG_TRY(lds_opt_in(k_ls_update<true>, sm));
+      k_ls_update<true><<<1, kLsThreads, sm, st>>>(skip, part, eb, dL, dD, dcoef, dC, cur, info);
+    } else {
+      k_ls_update<false><<<1, kLsThreads, ls_lds(cur, false), st>>>(skip, part, eb, dL, dD, dcoef, dC, cur, info);
+    }
     if (rit >= 0) {
-      k_axpy_resid<<<kRedBlocks, kBlock, 0, st>>>(ctl, (const double2* const*)dlist, dcoef, cur, ax, rhs, g, pc,
-                                                  unext, nv, rpart);
-      const GmFin F = fin_of(rit, check, kResU, cur, unext ? cur : -1);
+      // 16 row groups of 64 elements while kRedBlocks workgroups cover the vector in one
+      // pass, else 4 groups of 256 (measured, 45 rows, 4 / 16 groups: 3 120 elements
+      // 6.3 / 5.6 us, 16 384 6.4 / 5.7, 32 768 6.5 / 7.4, 131 072 20.6 / 33.4)
+      const bool wide = nv <= (size_t)kRedBlocks * (kAxThreads / 16);
+      const size_t epb = kAxThreads / (wide ? 16 : 4);
+      const int nblk = (int)std::min<size_t>(kRedBlocks, (nv + epb - 1) / epb);
+      (wide ? k_axpy_resid<16> : k_axpy_resid<4>)<<<nblk, kAxThreads, 0, st>>>(
+          ctl, (const double2* const*)dlist, dcoef, cur, ax, rhs, g, pc, unext, nv, rpart);
+      const GmFin F = fin_of(rit, check, kResU, cur, unext ? cur : -1, nblk);
       if (ride && check && unext) {
         // the next kernel is the next iteration's projection: the finish rides on it
         pend = F;

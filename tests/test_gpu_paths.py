@@ -141,6 +141,26 @@ def test_gmres_deep_restarts(depth):
     assert np.abs(got[:, 4] - ref[:, 4]).max() <= tol, (got[:, 4], ref[:, 4])
 
 
+@pytest.mark.parametrize("nb,depth,rows", [(8, 256, 142), (5, 256, 129), (2, 70, 0)])
+def test_gmres_recycled_basis_past_the_lds_factor(nb, depth, rows):
+    """Recycled solves whose basis passes 64 and 128 rows (one, two and four indices per
+    lane in the least-squares sweeps) and, at 8 bands, the 141 rows whose factor fits
+    the LDS; 2 bands: fewer unknowns than one wave.  Both solves stop at |g|^2 < ffff,
+    so -Im<b|x> f of each is within f |b| sqrt(ffff) / Gamma of the solution's."""
+    inp = synth.make_inputs(nb=nb, kmesh=(2, 2, 2), xmesh=(3, 3, 3), lc=0, seed=61)
+    P = to_problem(inp)
+    E = np.array([12.0, 12.1, 12.3, 12.5])
+    ffff, gam = 1e-16, 0.1
+    ref = orc.gmres_do_recycle(P, inp.psi0, E, gam, 13.605, ffff, depth, inp.kpref)
+    with core.OceanGPU.from_inputs(inp) as g:
+        got = g.gmres(inp.psi0, E, gam, 13.605, ffff, depth)
+    print(ref[:, [2, 4, 5]], got[:, [2, 4, 5]], flush=True)
+    assert ref[-1, 5] >= rows
+    bnorm = np.linalg.norm(inp.allow * inp.psi0)
+    tol = 2 * inp.kpref * bnorm * np.sqrt(ffff) / (gam * core.EV2HARTREE)
+    assert np.abs(got[:, 2] - ref[:, 2]).max() <= tol
+
+
 def test_nan_in_start_vector_stops_at_first_iteration():
     inp = synth.make_inputs(nb=8, kmesh=(2, 2, 2), xmesh=(3, 3, 3), lc=0, seed=62)
     psi = inp.psi0.copy()
