@@ -116,7 +116,7 @@ struct ActArgs {
   const double2* energy;
   const double* allow;
   const double2* cproj;       // [s][k][p][n]
-  double2* apart;             // [a*P+p][k]
+  double2* apart;             // [nm][a*P+p] multiplet partials
   double2* amp;               // [a*P+p]
   const double2* Kmat;        // (na P)^2
   double2* hmult;             // [a*P+p]
@@ -128,8 +128,9 @@ struct ActArgs {
                               // right-hand side a / na0 (na = na0 for one right-hand side)
   int ldu, ldT, ldphi;
   int flags;
-  int px;                     // projection x-tiles (blockDim.x x-points each)
-  int bstage;                 // FP64 matrix-core projection: A psi of the k staged in LDS
+  int px;                     // projection x-tiles per k (one wave tile per wave)
+  int tput;                   // projection: phi tiles go out through LDS (one spin, where it fits)
+  int nm, nmb;                // multiplet workgroups per spin and 16 projectors, and in all
   int G, ncol, nfft, nred;    // transform: columns per strip, strips, reduction workgroups
   int K1, K2, K3;
   int XC, JR;                 // adjoint: phi' chunk, alphas per reduction round
@@ -166,442 +167,317 @@ __device__ __forceinline__ int find_problem(const int* __restrict__ off, int np,
   return lo;
 }
 
-__device__ __forceinline__ void mproj_k(const double2* __restrict__ c, const double2* __restrict__ psi,
-                                        const double* __restrict__ allow, double2* __restrict__ apart,
-                                        int nb, int nk, int na, int ns, int P, int k, int s, int c0,
-                                        int cstep);
+// ---------------------------------------------------------------------------
+// Multiplet projection partials: amplitude (a, p) = sum_{k,n} c(n,k,p) (A psi)(n,k,a)
+//   OCEAN_multiplet.f90:1730-1783 (no conjugation)
+// as an FP64 matrix-core GEMM (M = 16 projectors, N = the 2 nalpha real columns of a
+// spin, K = bands and k).  Workgroup blk = (s, projector tile, m): its waves take units
+// of one k and up to 64 bands, m nw + w first and nm nw apart, with kB steps of four
+// bands in flight; their sums are added in LDS in wave order into apart[m].  These
+// workgroups come first in the projection's grid, so that they run beside the u
+// stream: at the end of the slab workgroups (a butterfly of 16 sums per alpha and
+// wave, after the slab) the same sums cost 5 us of a 31 us FP32 projection at 64
+// bands, 31 of 163 us at the L2,3 edge with 128 bands; here 4 and 8.
+// ---------------------------------------------------------------------------
+template <int NA>
+constexpr int mult_lds_per_wave() { return ((2 * NA + 15) / 16) * 4 * 64 * (int)sizeof(double); }
+
+template <int NA>
+__device__ __forceinline__ void mult_body(const double2* __restrict__ c, const double2* __restrict__ psi,
+                                          const double* __restrict__ allow, double2* __restrict__ apart, int nb,
+                                          int nk, int na, int ns, int P, int nm, int blk, double* red) {
+  constexpr int NT = (2 * NA + 15) / 16, kB = NT == 1 ? 8 : 4;
+  const int npt = (P + 15) >> 4;
+  const int s = blk / (nm * npt), pt = (blk / nm) % npt, m = blk % nm;
+  const int astep = (ns == 2) ? 2 : 1;
+  const int acnt = (ns == 2) ? na / 2 : na;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int i = lane & 15, kk = lane >> 4;
+  const bool im = i & 1;
+  const int nch = (nb + 63) >> 6, units = nk * nch;
+  og_d4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = og_d4{0, 0, 0, 0};
+  for (int un = m * nw + w; un < units; un += nm * nw) {
+    const int k = un / nch, n00 = (un - k * nch) * 64, n1 = min(nb, n00 + 64);
+    const double2* cb = c + ((size_t)(s * nk + k) * P + min(16 * pt + i, P - 1)) * nb;
+    for (int n0 = n00; n0 < n1; n0 += 4 * kB) {
+      double2 cv[kB], pv[kB][NT];
+      double mv[kB][NT];
+#pragma unroll
+      for (int q = 0; q < kB; ++q) {
+        const int n = min(n0 + 4 * q + kk, nb - 1);
+        cv[q] = ld_stream(cb + n);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int j = min((16 * t + i) >> 1, acnt - 1);
+          const size_t off = ((size_t)(s + j * astep) * nk + k) * nb + n;
+          pv[q][t] = psi[off];
+          mv[q][t] = allow[off];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < kB; ++q) {
+        // rows past the unit's bands contribute zeros on both sides
+        const bool ok = n0 + 4 * q + kk < n1;
+        const double cx = ok ? cv[q].x : 0.0, cy = ok ? cv[q].y : 0.0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const double pr = ok ? pv[q][t].x * mv[q][t] : 0.0, pi = ok ? pv[q][t].y * mv[q][t] : 0.0;
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cx, im ? pi : pr, acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(cy, im ? pr : -pi, acc[t], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[((w * NT + t) * 4 + r) * 64 + lane] = acc[t][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NT * 256; e += blockDim.x) {
+    const int l = e & 63, r = (e >> 6) & 3, t = e >> 8;
+    double v = 0.0;
+    for (int q = 0; q < nw; ++q) v += red[((q * NT + t) * 4 + r) * 64 + l];
+    const int G = 16 * t + (l & 15), p = 16 * pt + Mf<double>::row(l >> 4, r);
+    if ((G >> 1) < acnt && p < P)
+      reinterpret_cast<double*>(apart + (size_t)m * na * P + (s + (G >> 1) * astep) * P + p)[G & 1] = v;
+  }
+}
+
+template <int NA>
+__global__ __launch_bounds__(kBlock) void k_mproj(const double2* __restrict__ c, const double2* __restrict__ psi,
+                                                  const double* __restrict__ allow, double2* __restrict__ apart,
+                                                  int nb, int nk, int na, int ns, int P, int nm) {
+  __shared__ double red[mult_lds_per_wave<NA>() / 8 * (kBlock / 64)];
+  mult_body<NA>(c, psi, allow, apart, nb, nk, na, ns, P, nm, blockIdx.x, red);
+}
 
 // ---------------------------------------------------------------------------
 // Projection: phi(k,x,a) = sum_n u(n,k,x) (A psi)(n,k,a)
-//   long_range.f90:897-906 (no conjugation of u).  Grid (ceil(nx/256), nk, ns).
-// With fg set, the slab workgroups of each k also form its multiplet projection
-// partials (a 16-KB read of c beside the 512-KB u slab), so the multiplet term needs
-// no launch or stream of its own.
+//   long_range.f90:897-906 (no conjugation of u).
+// Per (k, s) a GEMM on the matrix cores in the precision of the stored u, M = x, N = the
+// 2 nalpha real columns (G = 2 a + re/im), K = bands with the complex parts unrolled:
+// lane l supplies u(n, x) for x = l % 16, n = l / 16 and, from A psi staged in LDS as
+// Bs[n][a], column l % 16 of B; columns past 2 nalpha compute values nobody stores.
+// Each wave takes one tile of kProjNL loads: 16 x points each in FP64, 32 in FP32 (a
+// 16-byte load holds u(n, x) and u(n, x + 1), which feed an even and an odd tile), with
+// a ring of kProjD steps of four bands in registers, so that kProjD - 1 are in flight
+// while one is multiplied.  It is bound by HBM: reading u alone runs at 6.5-7 TB/s and
+// writing phi beside it adds about a byte's read time per two thirds of a byte.  256
+// threads: at 512 the tail of the grid is coarser (L2,3 edge, 128 bands, 213 -> 222 us
+// FP64, 125 -> 142 FP32).  Phi goes out through a wave-private LDS transpose as whole
+// contiguous rows (118 -> 115 us there in FP32).  Against streaming FMAs below six
+// alphas and matrix-core forms with one load per step and k-strided stores above,
+// at 512 k points (us before -> after):
+//   64 bands, 512 x, 4 alphas: FP64 50 -> 50, FP32 31 -> 27 (100 bands: FP64 46 -> 37)
+//   64 bands, 512 x, 12 / 24 alphas: FP64 66 -> 63 / 128 -> 93, FP32 (24) 66 -> 53
+//   128 bands, 1000 x, 12 alphas: FP64 221 -> 213, FP32 163 -> 125
+//   64 k points, 16 bands, 216 x, 4 alphas: FP64 8.1 -> 4.4
 // ---------------------------------------------------------------------------
-// FP32 projection on the matrix cores, for many alphas (L2,3 edges), where the FMA
-// count per byte of u would otherwise bound the streaming loop.  Per (k, s) it is the
-// real GEMM phi[x][c] = sum_{n, r} U[x][(n, r)] B[(n, r)][c] with the complex parts
-// unrolled: r = re/im part of u(n, x), columns c < acnt the real parts of phi(x, a),
-// c - acnt the imaginary parts, so B[(n, re)] = (psi_r, psi_i), B[(n, im)] =
-// (-psi_i, psi_r) of A psi(n, a).  v_mfma_f32_16x16x4f32: lane l supplies
-// U[x(l % 16)][k = l / 16] and B[k = l / 16][c = l % 16] and receives D[4 (l / 16) + r]
-// [l % 16] in register r.  Each lane loads 16 bytes, u(n, x) and u(n, x + 1), which
-// feed two tiles (even and odd x) of 16 x points; one wave covers 32 x points, four
-// band rows per step, and all column tiles (two for acnt <= 12, three for 24).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-// floats per half B row (the part multiplying re u, then the part multiplying im u)
-// and per row: halves of 32 (48 for three column tiles) and 16 floats of pad, so
-// the four band rows one instruction reads start 16 or 48 banks apart (no conflicts)
-template <int NA> constexpr int proj_bhalf() { return NA > 12 ? 48 : 32; }
-template <int NA> constexpr int proj_brow() { return 2 * proj_bhalf<NA>() + 16; }
-template <int NA>
-__device__ __forceinline__ void proj_mfma_body(const ActArgs<float2>& A, int bx, int k, int s) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int kBRow = proj_brow<NA>(), HW = proj_bhalf<NA>();
-  float* bt = reinterpret_cast<float*>(smem);  // [nb4][kBRow]: B rows (n, re) then (n, im)
-  const int nb = A.nb, nk = A.nk, na = A.na, ns = A.ns;
+constexpr int kProjNL = 2;  // loads per step and wave (one: 222 -> 244 us, 130 -> 151 us at the L2,3 edge)
+constexpr int kProjD = 4;   // ring steps (three: equal to 1 us; six at three waves per SIMD: slower)
+
+template <typename T2> struct ProjLoad;
+template <> struct ProjLoad<double2> {
+  using F = double2;
+  static constexpr int X = 16;  // x points per load
+};
+template <> struct ProjLoad<float2> {
+  using F = float4;
+  static constexpr int X = 32;
+};
+// x points per wave
+template <typename T2> constexpr int proj_xt() { return ProjLoad<T2>::X * kProjNL; }
+
+template <typename T2, int NA>
+__device__ __forceinline__ void proj_body(const ActArgs<T2>& A, int bx, int k, int s, unsigned char* smem) {
+  using T = typename Scalar<T2>::T;
+  using M = Mf<T>;
+  using V = typename M::V;
+  using F = typename ProjLoad<T2>::F;
+  constexpr int NT = (2 * NA + 15) / 16, NL = kProjNL, D = kProjD, XL = ProjLoad<T2>::X;
+  constexpr int Q = sizeof(T) == 8 ? 1 : 2;  // matrix-core tiles per load
+  const int nb = A.nb, nk = A.nk, nx = A.nx, na = A.na, ns = A.ns;
   const int astep = (ns == 2) ? 2 : 1;
   const int acnt = (ns == 2) ? na / 2 : na;
-  const int nb4 = (nb + 3) & ~3;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int xb = (bx * (int)(blockDim.x >> 6) + wave) * 32;
-  const bool xon = xb < A.nx;  // waves past nx stay for the multiplet partials after the slab
-  const int m16 = lane & 15, kq = lane >> 4;
-  // x + 1 <= xb + 31 < nx + 31 < ldu: the pair stays inside the padded row
-  const float2* ub = A.u + ((size_t)(s * nk + k) * nb) * A.ldu + min(xb, A.nx - 1) + 2 * m16;
-  // batches of kS four-row steps, double-buffered: the loads of batch b + 1 are
-  // issued before the products of batch b, so each wave keeps HBM busy while its
-  // matrix-core work runs.  The first batch is issued before the B staging below,
-  // so the slab stream starts while psi and allow are read.
-  // (four at 24 alphas: 84.5 -> 66.8 us at nb 64, 111 instead of 133 VGPRs, so two
-  // 512-thread workgroups fit a CU)
-  constexpr int kS = NA > 12 ? 4 : 8;
-  const int nfull = nb / (4 * kS);
-  float4 qa[kS], qb[kS];
-  auto load_batch = [&](float4* q, int b) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int i = lane & 15, kk = lane >> 4;
+  const bool im = i & 1;
+  const int S = (nb + 3) >> 2;  // steps of four bands; B rows past nb are zero
+  T2* Bs = reinterpret_cast<T2*>(smem);
+  const int x0 = (bx * nw + w) * XL * NL;
+  const bool on = x0 < nx;
+  const T2* __restrict__ ub = A.u + (size_t)(s * nk + k) * nb * A.ldu;
+  int xo[NL];
 #pragma unroll
-    for (int i = 0; i < kS; ++i) q[i] = ld_stream4(ub + (size_t)(b * 4 * kS + 4 * i + kq) * A.ldu);
+  for (int l = 0; l < NL; ++l)
+    xo[l] = sizeof(T) == 8 ? min(x0 + 16 * l + i, nx - 1) : min(x0 + 32 * l + 2 * i, A.ldu - 2);
+  int ln = kk;
+  auto load = [&](F(&f)[NL]) {
+    const T2* row = ub + (size_t)min(ln, nb - 1) * A.ldu;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      if constexpr (sizeof(T) == 8) f[l] = ld_stream(row + xo[l]);
+      else f[l] = ld_stream4(row + xo[l]);
+    }
+    ln += 4;
   };
-  if (xon && nfull > 0) load_batch(qa, 0);
-  // each (n, alpha) element is read once (kF loads in flight per thread) and fills
-  // its four B entries; columns past 2 acnt and rows past nb are zero.  (Bands
-  // fastest over the threads, which makes the reads contiguous, measured slower:
-  // its LDS writes land four banks apart, 52.5 -> 61.4 us at nb 64 and 12 alphas.)
-  const int nel = nb4 * acnt;
-  constexpr int kF = 8;
+  // the first steps of the stream are in flight while A psi is staged
+  F f[D][NL];
+  if (on) {
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) load(f[d]);
+  }
+  const int nel = 4 * S * acnt;
+  constexpr int kF = 4;
   for (int i0 = threadIdx.x; i0 < nel; i0 += kF * blockDim.x) {
     double2 pv[kF];
     double mv[kF];
 #pragma unroll
-    for (int f = 0; f < kF; ++f) {
-      const int i = i0 + f * blockDim.x;
-      const int n = i / acnt, c = i - n * acnt;
-      pv[f] = make_double2(0.0, 0.0);
-      mv[f] = 0.0;
-      if (i < nel && n < nb) {
-        const size_t off = ((size_t)(s + c * astep) * nk + k) * nb + n;
-        pv[f] = A.psi[off];
-        mv[f] = A.allow[off];
-      }
-    }
-#pragma unroll
-    for (int f = 0; f < kF; ++f) {
-      const int i = i0 + f * blockDim.x;
-      if (i < nel) {
-        const int n = i / acnt, c = i - n * acnt;
-        float* row = bt + n * kBRow;
-        const float pr = (float)(pv[f].x * mv[f]), pim = (float)(pv[f].y * mv[f]);
-        row[c] = pr;
-        row[HW + c] = -pim;
-        row[acnt + c] = pim;
-        row[HW + acnt + c] = pr;
-      }
-    }
-  }
-  const int nz = HW - 2 * acnt;
-  for (int i = threadIdx.x; i < nb4 * nz; i += blockDim.x) {
-    const int n = i / nz, c = 2 * acnt + (i - n * nz);
-    bt[n * kBRow + c] = 0.f;
-    bt[n * kBRow + HW + c] = 0.f;
-  }
-  __syncthreads();
-  if (xon) {
-    constexpr int NT = (2 * NA + 15) / 16;  // column tiles (2 acnt <= 16 fits one)
-    f32x4 ce[NT], co[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) { ce[t] = f32x4{0, 0, 0, 0}; co[t] = f32x4{0, 0, 0, 0}; }
-    // one four-row step: tile t takes re(u) x B(n, re) + im(u) x B(n, im); the four
-    // chains are interleaved so that dependent products are NT * 2 issues apart
-    auto step = [&](const float4& q, const float* br) {
-      float b[NT], c[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) { b[t] = br[16 * t]; c[t] = br[HW + 16 * t]; }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        ce[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x, b[t], ce[t], 0, 0, 0);
-        co[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.z, b[t], co[t], 0, 0, 0);
-      }
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        ce[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.y, c[t], ce[t], 0, 0, 0);
-        co[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w, c[t], co[t], 0, 0, 0);
-      }
-    };
-    auto use_batch = [&](const float4* q, int b) {
-#pragma unroll
-      for (int i = 0; i < kS; ++i) step(q[i], bt + (b * 4 * kS + 4 * i + kq) * kBRow + m16);
-    };
-    for (int b = 0; b < nfull; b += 2) {
-      if (b + 1 < nfull) load_batch(qb, b + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      use_batch(qa, b);
-      if (b + 1 < nfull) {
-        if (b + 2 < nfull) load_batch(qa, b + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        use_batch(qb, b + 1);
-      }
-    }
-    // remaining rows, four at a time; rows past nb read zero B rows (nb4 covers them)
-    for (int n0 = nfull * 4 * kS; n0 < nb; n0 += 4) {
-      const float4 q = ld_stream4(ub + (size_t)min(n0 + kq, nb - 1) * A.ldu);
-      step(q, bt + (n0 + kq) * kBRow + m16);
-    }
-    // D[4 kq + r][m16]: x = xb + 2 (4 kq + r) (+1 for the odd tile), column 16 t + m16
-    float* ph = reinterpret_cast<float*>(A.phi + (size_t)k * A.ldphi);
-    auto put = [&](const f32x4& d, int t, int odd) {
-      const int c = 16 * t + m16;
-      if (c >= 2 * acnt) return;
-      const int j = c < acnt ? c : c - acnt, part = c < acnt ? 0 : 1;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int x = xb + 2 * (4 * kq + r) + odd;
-        if (x < A.nx) ph[2 * ((size_t)x * na + s + j * astep) + part] = d[r];
-      }
-    };
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      put(ce[t], t, 0);
-      put(co[t], t, 1);
-    }
-  }
-}
-
-template <typename T2, int NA>
-__device__ __forceinline__ void proj_body(const ActArgs<T2>& A, int bx, int k, int s) {
-  if constexpr (sizeof(T2) == 8 && NA >= 6) {
-    proj_mfma_body<NA>(A, bx, k, s);
-    return;
-  }
-  using T = typename Scalar<T2>::T;
-  extern __shared__ __align__(16) unsigned char smem[];
-  T2* ps = reinterpret_cast<T2*>(smem);  // [acnt][nb]
-  const int nb = A.nb, nk = A.nk, na = A.na, ns = A.ns;
-  const int astep = (ns == 2) ? 2 : 1;
-  const int acnt = (ns == 2) ? na / 2 : na;
-  // 16 bytes per lane and row: one x point in FP64, two adjacent ones in FP32 (the
-  // row stride ldu is even, so the pair is 16-byte aligned)
-  constexpr int VX = sizeof(T) == 8 ? 1 : 2;
-  const int x = (bx * blockDim.x + threadIdx.x) * VX;
-  const bool on = x < A.nx;  // threads past nx stay for the multiplet partials after the slab
-  const T2* ub = A.u + ((size_t)(s * nk + k) * nb) * A.ldu + min(x, (A.nx - 1) & ~(VX - 1));
-  // Batches of kB band rows: all kB loads are issued before the first use, so
-  // each wave keeps kB row segments in flight (8 KB per wave in FP64; FP32 runs
-  // half as many threads per workgroup and keeps 16 KB per wave in flight).
-  // Full batches carry no per-row predicate: with one, the compiler sinks the FP32
-  // loads into per-row branches and waits on each row in turn.
-  constexpr int kB = VX == 1 ? 8 : 16;
-  auto load_row = [&](int n, T2* dst) {
-    const T2* row = ub + (size_t)n * A.ldu;
-    if constexpr (VX == 1) {
-      dst[0] = ld_stream(row);
-    } else {
-      const float4 q = ld_stream4(reinterpret_cast<const float2*>(row));
-      dst[0] = cmake<T2>(q.x, q.y);
-      dst[VX - 1] = cmake<T2>(q.z, q.w);
-    }
-  };
-  // the first batch is in flight while A psi is staged
-  T2 uv0[kB][VX];
-  const bool pre = on && nb >= kB;
-  if (pre) {
-#pragma unroll
-    for (int i = 0; i < kB; ++i) load_row(i, uv0[i]);
-  }
-  // A psi of this k in LDS, with up to kF loads in flight per thread
-  constexpr int kF = 4;
-  for (int i0 = threadIdx.x; i0 < acnt * nb; i0 += kF * blockDim.x) {
-    double2 pv[kF];
-    double mv[kF];
-#pragma unroll
-    for (int f = 0; f < kF; ++f) {
-      const int i = min(i0 + f * (int)blockDim.x, acnt * nb - 1);
-      const int j = i / nb, n = i - j * nb;
+    for (int q = 0; q < kF; ++q) {
+      const int e = min(i0 + q * (int)blockDim.x, nel - 1);
+      const int j = e / (4 * S), n = min(e - j * 4 * S, nb - 1);
       const size_t off = ((size_t)(s + j * astep) * nk + k) * nb + n;
-      pv[f] = A.psi[off];
-      mv[f] = A.allow[off];
+      pv[q] = A.psi[off];
+      mv[q] = A.allow[off];
     }
 #pragma unroll
-    for (int f = 0; f < kF; ++f) {
-      const int i = i0 + f * blockDim.x;
-      if (i < acnt * nb) ps[i] = cmake<T2>((T)(pv[f].x * mv[f]), (T)(pv[f].y * mv[f]));
+    for (int q = 0; q < kF; ++q) {
+      const int e = i0 + q * (int)blockDim.x;
+      if (e < nel) {
+        const int j = e / (4 * S), n = e - j * 4 * S;
+        Bs[n * acnt + j] = n < nb ? cmake<T2>((T)(pv[q].x * mv[q]), (T)(pv[q].y * mv[q])) : cmake<T2>(0, 0);
+      }
     }
   }
   __syncthreads();
-  if (on) {
-    T2 acc[VX][NA];
-#pragma unroll
-    for (int v = 0; v < VX; ++v)
-#pragma unroll
-      for (int j = 0; j < NA; ++j) acc[v][j] = cmake<T2>(0, 0);
-    auto use_row = [&](int n, const T2* uvr) {
-#pragma unroll
-      for (int j = 0; j < NA; ++j) {
-        const T2 pv = ps[j * nb + n];
-#pragma unroll
-        for (int v = 0; v < VX; ++v) cfma(acc[v][j], uvr[v], pv);
-      }
-    };
-    int n0 = 0;
-    if (pre) {
-#pragma unroll
-      for (int i = 0; i < kB; ++i) use_row(i, uv0[i]);
-      n0 = kB;
-    }
-    for (; n0 + kB <= nb; n0 += kB) {
-      T2 uv[kB][VX];
-#pragma unroll
-      for (int i = 0; i < kB; ++i) load_row(n0 + i, uv[i]);
-      // keep the kB loads together ahead of the arithmetic
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < kB; ++i) use_row(n0 + i, uv[i]);
-    }
-    for (; n0 < nb; ++n0) {
-      T2 uv[VX];
-      load_row(n0, uv);
-      use_row(n0, uv);
-    }
-#pragma unroll
-    for (int v = 0; v < VX; ++v) {
-      if (x + v < A.nx) {
-        T2* out = A.phi + (size_t)k * A.ldphi + (size_t)(x + v) * na;
-#pragma unroll
-        for (int j = 0; j < NA; ++j)
-          if (j < acnt) out[s + j * astep] = acc[v][j];
-      }
-    }
-  }
-}
-
-// M tiles (16 x points each) per wave of the FP64 matrix-core projection
-constexpr int kProjMT64 = 4;
-
-// FP64 projection for many alphas on the matrix cores: per k the GEMM
-// phi[x][(a, c)] = sum_n u(n, k, x) (A psi)(n, k, a) with the complex parts unrolled
-// along K (v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16], B[l / 16][l % 16]
-// and receives D[l / 16 + 4 r][l % 16]).  Each wave covers 16 MT x points (MT M tiles)
-// and all 2 nalpha real columns of its spin, so every u element is read once; A psi
-// is formed per lane from psi and allow (L1/L2 hits).  Single-buffered fragments
-// keep four waves per SIMD, which hide the u stream's latency; double buffering
-// needed 166 VGPRs (three waves) and was slower.
-template <int NA, int MT>
-__device__ __forceinline__ void proj_mf64_body(const ActArgs<double2>& A, int bx, int k, int s) {
-  constexpr int NT = (2 * NA + 15) / 16;
-  const int nb = A.nb, nk = A.nk, nx = A.nx, na = A.na, ns = A.ns;
-  const int astep = (ns == 2) ? 2 : 1;
-  const int acnt = (ns == 2) ? na / 2 : na;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int i = lane & 15, kk = lane >> 4;
-  const int x0 = bx * (int)blockDim.x * MT / 4 + w * 16 * MT;
-  int ja[NT], jc[NT], jl[NT];
-  bool jok[NT];
-  size_t boff[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int G = t * 16 + i;
-    jc[t] = G & 1;
-    jok[t] = (G >> 1) < acnt;
-    jl[t] = min(G >> 1, acnt - 1);
-    ja[t] = s + jl[t] * astep;
-    boff[t] = ((size_t)ja[t] * nk + k) * nb;
-  }
-  // A psi of this k staged once per workgroup (A.bstage; the host sets it when nb acnt
-  // complex values fit the LDS budget): read with bands fastest over the threads, so
-  // every load is a contiguous band row of one alpha, where each wave otherwise loads
-  // 2 NT scattered (alpha, band) pairs per lane and step from L2
-  extern __shared__ __align__(16) unsigned char smem[];
-  double2* Bs = reinterpret_cast<double2*>(smem);  // A psi(n, j) at Bs[n * acnt + j]
-  const bool staged = NA <= 12 && A.bstage != 0;  // not built at 24 alphas (slower there)
-  if (staged) {
-    const int nel = nb * acnt;
-    constexpr int kF = 8;
-    for (int i0 = threadIdx.x; i0 < nel; i0 += kF * blockDim.x) {
-      double2 pv[kF];
-      double mv[kF];
-#pragma unroll
-      for (int f = 0; f < kF; ++f) {
-        const int e = min(i0 + f * (int)blockDim.x, nel - 1);
-        const int j = e / nb, n = e - j * nb;
-        const size_t off = ((size_t)(s + j * astep) * nk + k) * nb + n;
-        pv[f] = A.psi[off];
-        mv[f] = A.allow[off];
-      }
-#pragma unroll
-      for (int f = 0; f < kF; ++f) {
-        const int e = i0 + f * (int)blockDim.x;
-        if (e < nel) {
-          const int j = e / nb, n = e - j * nb;
-          Bs[n * acnt + j] = make_double2(pv[f].x * mv[f], pv[f].y * mv[f]);
-        }
-      }
-    }
-    __syncthreads();
-  }
-  const double2* __restrict__ up = A.u + ((size_t)s * nk + k) * nb * A.ldu;
-  int xr[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) xr[m] = min(x0 + 16 * m + i, nx - 1);
-  og_d4 acc[NT][MT];
+  if (!on) return;
+  V acc[NT][NL * Q];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[t][m] = og_d4{0.0, 0.0, 0.0, 0.0};
-  double2 bA[NT], aA[MT];
-  auto load = [&](int n0, double2 (&bn)[NT], double2 (&an)[MT]) {
-    const int n = min(n0 + kk, nb - 1);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (staged) {
-        bn[t] = Bs[n * acnt + jl[t]];
-      } else {
-        double2 pv = A.psi[boff[t] + n];
-        const double m = A.allow[boff[t] + n];
-        bn[t] = make_double2(pv.x * m, pv.y * m);
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) an[m] = ld_stream(up + (size_t)n * A.ldu + xr[m]);
-  };
-  // C = A B: re: ar br - ai bi, im: ar bi + ai br
-  auto step = [&](int n0, const double2 (&bv)[NT], const double2 (&an)[MT]) {
-    const bool ok = n0 + kk < nb;
-    double2 av[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) av[m] = ok ? an[m] : make_double2(0.0, 0.0);
-    double b0[NT], b1[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      b0[t] = jc[t] ? bv[t].y : bv[t].x;
-      b1[t] = jc[t] ? bv[t].x : -bv[t].y;
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m].x, b0[t], acc[t][m], 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[m].y, b1[t], acc[t][m], 0, 0, 0);
-  };
-  for (int n0 = 0; n0 < nb; n0 += 4) {
-    load(n0, bA, aA);
-    step(n0, bA, aA);
-  }
+    for (int m = 0; m < NL * Q; ++m) acc[t][m] = V{0, 0, 0, 0};
+  const T2* bp[NT];
+  bool jok[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
-    if (!jok[t]) continue;
-    double* __restrict__ out = reinterpret_cast<double*>(A.phi + (size_t)k * A.ldphi + ja[t]) + jc[t];
+    const int G = 16 * t + i;
+    jok[t] = (G >> 1) < acnt;
+    bp[t] = Bs + kk * acnt + min(G >> 1, acnt - 1);
+  }
+  // u B: re: ur br - ui bi, im: ur bi + ui br
+  auto step = [&](const F(&g)[NL], int st) {
+    T b0[NT], b1[NT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int t = 0; t < NT; ++t) {
+      const T2 b = bp[t][4 * st * acnt];
+      b0[t] = im ? b.y : b.x;
+      b1[t] = im ? b.x : -b.y;
+    }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int x = x0 + 16 * m + kk + 4 * r;
-        if (x < nx) out[(size_t)x * na * 2] = acc[t][m][r];
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        acc[t][l * Q] = M::step(g[l].x, b0[t], acc[t][l * Q]);
+        if constexpr (Q == 2) acc[t][l * 2 + 1] = M::step(g[l].z, b0[t], acc[t][l * 2 + 1]);
       }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int l = 0; l < NL; ++l) {
+        acc[t][l * Q] = M::step(g[l].y, b1[t], acc[t][l * Q]);
+        if constexpr (Q == 2) acc[t][l * 2 + 1] = M::step(g[l].w, b1[t], acc[t][l * 2 + 1]);
+      }
+  };
+  int st = 0;
+  for (; st + D <= S; st += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      load(f[(d + D - 1) % D]);
+      __builtin_amdgcn_sched_barrier(0);  // keep the ring's loads ahead of this step's products
+      step(f[d], st + d);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D - 1; ++d)
+    if (st + d < S) step(f[d], st + d);
+  if (A.tput) {
+    T2* tw = reinterpret_cast<T2*>(smem + (((size_t)nel * sizeof(T2) + 15) & ~(size_t)15)) + w * XL * acnt;
+    T* o = reinterpret_cast<T*>(tw);
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const int xl = x0 + XL * l;
+      if (xl >= nx) break;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (jok[t]) {
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[(Q * M::row(kk, r) + q) * 2 * acnt + 16 * t + i] = acc[t][l * Q + q][r];
+        }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const int n16 = min(XL, nx - xl) * acnt * (int)sizeof(T2) / 16;
+      const float4* src = reinterpret_cast<const float4*>(tw);
+      float4* dst = reinterpret_cast<float4*>(A.phi + (size_t)k * A.ldphi + (size_t)xl * na);
+#pragma unroll
+      for (int e = lane; e < XL * NA * (int)sizeof(T2) / 16; e += 64)
+        if (e < n16) dst[e] = src[e];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  } else {
+    T* ph = reinterpret_cast<T*>(A.phi + (size_t)k * A.ldphi);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (!jok[t]) continue;
+      T* o = ph + 2 * (s + ((16 * t + i) >> 1) * astep) + (im ? 1 : 0);
+#pragma unroll
+      for (int m = 0; m < NL * Q; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int x = x0 + XL * (m / Q) + Q * M::row(kk, r) + m % Q;
+          if (x < nx) o[(size_t)x * na * 2] = acc[t][m][r];
+        }
+    }
   }
 }
 
-// Workgroup b of a projection launch: slab tile bx of (k, s).  With the multiplet
-// on, each tile then forms its share (chunks bx, bx + px, ...) of that k's multiplet
-// partials (16 KB of c per k), after its slab so that the stream starts at once.
+// Workgroup b of a projection launch of n: the multiplet workgroups, then slab tile bx of
+// (k, s).  Workgroups are dispatched round-robin over the 8 XCDs; with remap each XCD
+// gets a contiguous range of tiles, so the px tiles of one k (which stage the same A
+// psi) share an L2.
 template <typename T2, int NA>
-__device__ __forceinline__ void proj_dispatch(const ActArgs<T2>& A, int b) {
+__device__ __forceinline__ void proj_dispatch(const ActArgs<T2>& A, int b, int n, bool remap) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (b < A.nmb) {
+    mult_body<NA>(A.cproj, A.psi, A.allow, A.apart, A.nb, A.nk, A.na, A.ns, A.P, A.nm, b,
+                  reinterpret_cast<double*>(smem));
+    return;
+  }
+  b -= A.nmb;
+  n -= A.nmb;
+  if (remap && (n & 7) == 0) b = (b & 7) * (n >> 3) + (b >> 3);
   const int r = b / A.px, bx = b - r * A.px, k = r % A.nk, s = r / A.nk;
-  if constexpr (sizeof(T2) == 16 && NA >= 6)
-    proj_mf64_body<NA, kProjMT64>(A, bx, k, s);
-  else
-    proj_body<T2, NA>(A, bx, k, s);
-  if (A.flags & F_FG) mproj_k(A.cproj, A.psi, A.allow, A.apart, A.nb, A.nk, A.na, A.ns, A.P, k, s, bx, A.px);
+  proj_body<T2, NA>(A, bx, k, s, smem);
 }
 
-// One problem: a 1-D grid of px * nk * ns slab tiles.  Workgroups are dispatched
-// round-robin over the 8 XCDs; the remap gives each XCD a contiguous range of tiles,
-// so the px tiles of one k (which stage the same A psi) share an L2.
-// The FP64 matrix-core form at twelve alphas keeps four waves per SIMD (at most 128
-// VGPRs); at 24 alphas that cap spilled 96 bytes per lane, so it runs at three.
 template <typename T2, int NA>
-constexpr int kProjWaves = (sizeof(T2) == 16 && NA >= 6 && NA <= 12) ? 4 : 1;
-
-template <typename T2, int NA>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kProjWaves<T2, NA>))) void k_proj(
-    const ActArgs<T2> A) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_proj(const ActArgs<T2> A) {
   if (skipped(A)) return;
   if (A.fin.c != nullptr && blockIdx.x == 0) gm_finish(A.fin);
-  int b = blockIdx.x;
-  const int n = gridDim.x;
-  if ((n & 7) == 0) b = (b & 7) * (n >> 3) + (b >> 3);
-  proj_dispatch<T2, NA>(A, b);
+  proj_dispatch<T2, NA>(A, blockIdx.x, gridDim.x, true);
 }
 
 // Many problems: workgroup b belongs to the problem whose range holds it.
 template <typename T2, int NA>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kProjWaves<T2, NA>))) void k_proj_batch(
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_proj_batch(
     const ActArgs<T2>* __restrict__ As, const int* __restrict__ off, int np) {
   const int p = find_problem(off, np, blockIdx.x);
   const ActArgs<T2> A = As[p];
   if (skipped(A)) return;
-  const int local = blockIdx.x - off[p];
-  proj_dispatch<T2, NA>(A, local);
+  proj_dispatch<T2, NA>(A, blockIdx.x - off[p], 0, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -837,7 +713,7 @@ __device__ __forceinline__ void dft_run(const T2* tw, int G, int nk, int L, int 
 
 __device__ void mred_tail(const double2* __restrict__ apart, double2* __restrict__ amp,
                           const double2* __restrict__ K, double2* __restrict__ hmult, int* counter,
-                          int nk, int nj, int nj0, double mul, int r, int nred, double2* lds);
+                          int np, int nj, int nj0, double mul, int r, int nred, double2* lds);
 
 // Strip of G consecutive phi columns (c = x*na + a) per workgroup, all nk rows:
 //   pass 1 (K3, F_+): HBM -> registers -> LDS, with W(x, :) staged beside it
@@ -855,7 +731,7 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
   // the reduction workgroups come first so that they are dispatched first
   const int nred = A.nred, nfft = A.nfft;
   if (blk < nred) {
-    mred_tail(A.apart, A.amp, A.Kmat, A.hmult, A.mcount, A.nk, A.nj, A.na0 * A.P, A.mul, blk, nred,
+    mred_tail(A.apart, A.amp, A.Kmat, A.hmult, A.mcount, A.nm, A.nj, A.na0 * A.P, A.mul, blk, nred,
               reinterpret_cast<double2*>(smem));
     return;
   }
@@ -1018,82 +894,6 @@ __global__ void k_wgrad(const T2* __restrict__ PX, const T2* __restrict__ PY, in
   }
 }
 
-// ---------------------------------------------------------------------------
-// Multiplet projection partials: apart(j = a*P+p, k) = sum_n c(n,k,p) (A psi)(n,k,a)
-//   OCEAN_multiplet.f90:1730-1783 (no conjugation).  One workgroup per (k, s):
-//   one wave per alpha, lanes over bands, 16 projectors per butterfly reduction.
-//   Wave-level only (no barriers), so a workgroup of another kernel can run it.
-// ---------------------------------------------------------------------------
-constexpr int kProjChunk = 8;
-
-__device__ __forceinline__ void mproj_k(const double2* __restrict__ c, const double2* __restrict__ psi,
-                                        const double* __restrict__ allow, double2* __restrict__ apart,
-                                        int nb, int nk, int na, int ns, int P, int k, int s, int c0,
-                                        int cstep) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int astep = (ns == 2) ? 2 : 1;
-  const int acnt = (ns == 2) ? na / 2 : na;
-  const double2* cb = c + ((size_t)s * nk + k) * P * nb;
-  for (int j = wid; j < acnt; j += nw) {
-    const int a = s + j * astep;
-    for (int p0 = c0 * kProjChunk; p0 < P; p0 += cstep * kProjChunk) {
-      double v[2 * kProjChunk];
-#pragma unroll
-      for (int q = 0; q < 2 * kProjChunk; ++q) v[q] = 0.0;
-      for (int n = lane; n < nb; n += 64) {
-        const size_t off = ((size_t)a * nk + k) * nb + n;
-        double2 pv = psi[off];
-        const double m = allow[off];
-        pv.x *= m; pv.y *= m;
-#pragma unroll
-        for (int q = 0; q < kProjChunk; ++q) {
-          if (p0 + q < P) {
-            const double2 cv = cb[(size_t)(p0 + q) * nb + n];
-            v[2 * q] = fma(cv.x, pv.x, v[2 * q]); v[2 * q] = fma(-cv.y, pv.y, v[2 * q]);
-            v[2 * q + 1] = fma(cv.x, pv.y, v[2 * q + 1]); v[2 * q + 1] = fma(cv.y, pv.x, v[2 * q + 1]);
-          }
-        }
-      }
-      int owner = 0;
-      const double tot = wave_multi_sum<double, 2 * kProjChunk>(v, lane, &owner);
-      if ((lane & (64 / (2 * kProjChunk) - 1)) == 0) {
-        const int q = owner >> 1;
-        if (p0 + q < P) {
-          double* dst = reinterpret_cast<double*>(apart + (size_t)(a * P + p0 + q) * nk + k);
-          dst[owner & 1] = tot;
-        }
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_mproj(
-    const double2* __restrict__ c, const double2* __restrict__ psi, const double* __restrict__ allow,
-    double2* __restrict__ apart, int nb, int nk, int na, int ns, int P) {
-  mproj_k(c, psi, allow, apart, nb, nk, na, ns, P, blockIdx.x, blockIdx.y, 0, 1);
-}
-
-// amp(j) = sum_k apart(j, k) for j in [j0, j1): one wave per amplitude, fixed order.
-__device__ __forceinline__ void mred_sum(const double2* __restrict__ apart, double2* __restrict__ amp,
-                                         int nk, int j0, int j1) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int j = j0 + wid; j < j1; j += nw) {
-    const double2* row = apart + (size_t)j * nk;
-    double sx = 0.0, sy = 0.0;
-    for (int k0 = lane; k0 < nk; k0 += 8 * 64) {
-      double2 v[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = row[min(k0 + i * 64, nk - 1)];
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (k0 + i * 64 < nk) { sx += v[i].x; sy += v[i].y; }
-    }
-    sx = wave_sum(sx);
-    sy = wave_sum(sy);
-    if (lane == 0) amp[j] = make_double2(sx, sy);
-  }
-}
-
 // h(i) = mul * sum_j K(i, j) amp(j): direct -mpm a plus exchange X a
 // (OCEAN_multiplet.f90:1812-1936); one wave per row, coalesced rows of K.  With
 // several right-hand sides K is block diagonal over blocks of nj0 amplitudes and a
@@ -1114,26 +914,55 @@ __device__ __forceinline__ void mred_matvec(const double2* __restrict__ K, const
 // Stand-alone reduction (used when the long-range term is off): one workgroup.
 __global__ __launch_bounds__(1024) void k_mred(
     const double2* __restrict__ apart, const double2* __restrict__ K, double2* __restrict__ hmult,
-    int nk, int nj, int nj0, double mul) {
+    int np, int nj, int nj0, double mul) {
   __shared__ double2 amp[kMaxAlpha * 64];
-  mred_sum(apart, amp, nk, 0, nj);
+  for (int j = threadIdx.x; j < nj; j += blockDim.x) {
+    double2 a = make_double2(0.0, 0.0);
+    for (int m = 0; m < np; ++m) {
+      const double2 v = apart[(size_t)m * nj + j];
+      a.x += v.x;
+      a.y += v.y;
+    }
+    amp[j] = a;
+  }
   __syncthreads();
   mred_matvec(K, amp, hmult, nj, nj0, mul);
 }
 
-// Reduction run by nred extra workgroups of another kernel's grid, one wave per
-// amplitude: workgroup r sums amplitudes [r*kRedPerBlock, ...) over k into amp
-// (global); the last workgroup to finish (device-scope counter) applies K, four
-// rows per wave at a time with all their loads in flight.  The counter returns
-// to zero for the next launch.  Loads are batched throughout: the whole tail is
-// a few memory latencies, so it hides under the kernel it rides on.
+// Reduction run by nred extra workgroups of another kernel's grid: workgroup r sums
+// amplitudes [r*kRedPerBlock, ...) over the np <= kMultBlocks partials into amp
+// (global), one load per thread and a fixed-order tree; the last workgroup to finish
+// (device-scope counter) applies K, four rows per wave at a time with all their loads
+// in flight.  The counter returns to zero for the next launch.  Loads are batched
+// throughout: the whole tail is a few memory latencies, so it hides under the kernel
+// it rides on.
 constexpr int kRedPerBlock = 4;
 
 __device__ void mred_tail(const double2* __restrict__ apart, double2* __restrict__ amp,
                           const double2* __restrict__ K, double2* __restrict__ hmult, int* counter,
-                          int nk, int nj, int nj0, double mul, int r, int nred, double2* lds) {
+                          int np, int nj, int nj0, double mul, int r, int nred, double2* lds) {
+  static_assert(kMultBlocks * kRedPerBlock == kBlock, "one partial per thread");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  mred_sum(apart, amp, nk, r * kRedPerBlock, min(nj, (r + 1) * kRedPerBlock));
+  {
+    const int j = r * kRedPerBlock + (threadIdx.x & 3), m = threadIdx.x >> 2;
+    double2 v = make_double2(0.0, 0.0);
+    if (j < nj && m < np) v = apart[(size_t)m * nj + j];
+#pragma unroll
+    for (int off = 4; off < 64; off <<= 1) {
+      v.x += __shfl_xor(v.x, off, 64);
+      v.y += __shfl_xor(v.y, off, 64);
+    }
+    if (lane < kRedPerBlock) lds[wid * kRedPerBlock + lane] = v;
+    __syncthreads();
+    if (threadIdx.x < kRedPerBlock && j < nj) {
+      double2 a = make_double2(0.0, 0.0);
+      for (int q = 0; q < nw; ++q) {
+        a.x += lds[q * kRedPerBlock + threadIdx.x].x;
+        a.y += lds[q * kRedPerBlock + threadIdx.x].y;
+      }
+      amp[j] = a;
+    }
+  }
   __threadfence();
   __syncthreads();
   __shared__ int is_last;

@@ -166,9 +166,16 @@ struct BandSide {
   int nx, ldu, ldT, ldphi;
 };
 
+// Multiplet workgroups per spin and projector tile: a unit (one k, up to 64 bands) per
+// wave, at most kMultBlocks (one load per thread sums them; 128 measured equal).
+int mult_blocks(const H* h, int nw) {
+  const int units = h->nk * ((h->nb + 63) / 64);
+  return std::min(og::kMultBlocks, (units + nw - 1) / nw);
+}
+
 // Fill the kernel arguments and launch geometry of one problem.  The
 // multiplet term rides on the long-range kernels when both are on: its partials
-// in the last x-tile workgroup of k_proj, its k-sum and K apply in workgroups
+// in workgroups prepended to k_proj, their sum and the K apply in workgroups
 // prepended to k_fft_w; both only read psi, so one stream carries the action.
 template <typename T2, int NA>
 int make_args(const H* h, const double2* in, double2* out, int flags, const Tiles& t, const T2* u,
@@ -193,23 +200,21 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   const bool lr = (flags & og::F_LR) != 0, fg = (flags & og::F_FG) != 0;
   // projection
   if (t.proj < 64 || t.proj > 512 || (t.proj & 63)) return OCEAN_GPU_ERR_ARG;
-  // FP32 streaming workgroups cover two x points per thread; the FP32 matrix-core
-  // form (many alphas) covers 32 per wave and stages B as nb4 rows of proj_brow floats
-  const bool mf = sizeof(T) == 4 && NA >= 6;
-  const bool mf64 = sizeof(T) == 8 && NA >= 6;
-  const int xper = mf ? 32 * (t.proj / 64) : mf64 ? 16 * og::kProjMT64 * (t.proj / 64)
-                                                  : t.proj * (sizeof(T) == 4 ? 2 : 1);
-  a.px = (nx + xper - 1) / xper;
-  // the FP64 matrix-core form (many alphas) forms A psi per lane and stages nothing
-  g.sm_proj = mf ? (size_t)((nb + 3) & ~3) * og::proj_brow<NA>() * sizeof(float)
-              : mf64 ? 0 : (size_t)acnt * nb * sizeof(T2);
-  // the FP64 matrix-core form stages A psi (nb acnt complex) where it fits 64 KB, up to
-  // twelve alphas (measured: L2,3 232 -> 222 us; at 24 alphas 121 -> 133 us)
-  if (mf64 && NA <= 12 && (size_t)nb * acnt * sizeof(double2) <= 65536) {
-    a.bstage = 1;
-    g.sm_proj = (size_t)nb * acnt * sizeof(double2);
+  // A psi of the k (nb rounded up to the steps of four, nalpha complex) in LDS, and beside
+  // it the phi tiles on their way out: contiguous rows on one spin only, and where both
+  // fit (24 alphas with more than about 340 bands: straight from the registers)
+  const int nw = t.proj / 64;
+  a.px = (nx + og::proj_xt<T2>() * nw - 1) / (og::proj_xt<T2>() * nw);
+  g.sm_proj = ((size_t)((nb + 3) & ~3) * acnt * sizeof(T2) + 15) & ~(size_t)15;
+  const size_t tp = (size_t)nw * og::ProjLoad<T2>::X * acnt * sizeof(T2);
+  a.tput = ns == 1 && (na & 1) == 0 && g.sm_proj + tp <= h->lds_max;
+  if (a.tput) g.sm_proj += tp;
+  a.nm = mult_blocks(h, nw);
+  if (lr && fg) {
+    a.nmb = a.nm * ((h->P + 15) / 16) * ns;
+    g.sm_proj = std::max(g.sm_proj, (size_t)nw * og::mult_lds_per_wave<NA>());
   }
-  g.nblk_proj = a.px * nk * ns;
+  g.nblk_proj = a.nmb + a.px * nk * ns;
   // transform
   a.ncol = nx * na;
   const int cap = (int)(57344 / sizeof(T2)) / nk;
@@ -280,16 +285,12 @@ template <> struct StateOf<float2> {
   static const float* W(const H* h) { return h->W32; }
 };
 
-// A handle's tiles for one precision: FP32 streaming projection threads take two x
-// points each, so half as many threads keep the x points per workgroup of FP64; the
-// FP32 matrix-core form for many alphas (32 x points per wave) takes twice as many.
-template <typename T2, int NA>
+// A handle's tiles for one precision (an FP32 projection takes any workgroup that the
+// handle accepts, up to the kernel's 512 threads).
+template <typename T2>
 Tiles tiles_for(const H* h) {
   Tiles t = h->tiles;
-  if (sizeof(typename og::Scalar<T2>::T) == 4) {
-    if (NA < 6) t.proj = std::max(64, t.proj / 2);
-    else t.proj = std::min(512, 2 * t.proj);  // fewer, wider workgroups per k share the B staging
-  }
+  if (sizeof(typename og::Scalar<T2>::T) == 4) t.proj = std::min(512, t.proj);
   return t;
 }
 
@@ -299,7 +300,7 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
            const og::GmFin* fin) {
   og::ActArgs<T2> a;
   Geom<T2> g;
-  const Tiles tl = tiles_for<T2, NA>(h);
+  const Tiles tl = tiles_for<T2>(h);
   OG_TRY((make_args<T2, NA>(h, in, out, flags, tl, u, uT, phi, W, a, g)));
   a.skip = skip;
   if (axmy) {
@@ -331,10 +332,13 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
     OG_CHECK(hipEventRecord(ev[2], h->stream));
   }
   if ((flags & og::F_FG) && !(flags & og::F_LR)) {
-    og::k_mproj<<<dim3(h->nk, h->ns), kBlock, 0, h->stream>>>(h->cproj, in, h->allow, h->apart, h->nb,
-                                                             h->nk, h->na, h->ns, h->P);
-    OG_CHECK(hipGetLastError());
-    og::k_mred<<<1, 1024, 0, h->stream>>>(h->apart, h->Kmat, h->hmult, h->nk, a.nj, h->na0 * h->P, a.mul);
+    const int nm = mult_blocks(h, kBlock / 64);
+    if (h->P > 0) {
+      og::k_mproj<NA><<<nm * ((h->P + 15) / 16) * h->ns, kBlock, 0, h->stream>>>(
+          h->cproj, in, h->allow, h->apart, h->nb, h->nk, h->na, h->ns, h->P, nm);
+      OG_CHECK(hipGetLastError());
+    }
+    og::k_mred<<<1, 1024, 0, h->stream>>>(h->apart, h->Kmat, h->hmult, nm, a.nj, h->na0 * h->P, a.mul);
     OG_CHECK(hipGetLastError());
   }
   if (ev) OG_CHECK(hipEventRecord(ev[3], h->stream));
@@ -380,7 +384,7 @@ int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev,
   flags &= ~og::F_FG;
   og::ActArgs<double2> a, ab;
   Geom<double2> g, gb;
-  const Tiles tl = tiles_for<double2, NA>(h);
+  const Tiles tl = tiles_for<double2>(h);
   OG_TRY((make_args<double2, NA>(h, in, out, flags, tl, nullptr, nullptr, h->phi64, h->W64, a, g)));
   a.phs = h->obf_phs;
   const BandSide bs{h->no, h->ldu_o, h->ldT_o, h->ldb};
@@ -394,6 +398,7 @@ int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev,
   }
   const int nk = h->nk, nx = h->nx, no = h->no;
   if (ev) OG_CHECK(hipEventRecord(ev[0], h->stream));
+  OG_TRY(lds_opt_in(og::k_proj<double2, NA>, gb.sm_proj));
   og::k_proj<double2, NA><<<gb.nblk_proj, tl.proj, gb.sm_proj, h->stream>>>(ab);
   OG_CHECK(hipGetLastError());
   if (ev) OG_CHECK(hipEventRecord(ev[1], h->stream));
@@ -1464,7 +1469,7 @@ int ocean_gpu_load_mult(ocean_gpu_handle* h, const double* mpcr, const double* m
   OG_TRY(dmalloc(&h->mcount, (size_t)1));
   OG_CHECK(hipMemset(h->mcount, 0, sizeof(int)));
   OG_TRY(dmalloc(&h->Kmat, Kd.size()));
-  OG_TRY(dmalloc(&h->apart, (size_t)nk * njt));
+  OG_TRY(dmalloc(&h->apart, (size_t)og::kMultBlocks * njt));
   OG_TRY(dmalloc(&h->hmult, (size_t)njt));
   OG_TRY(dmalloc(&h->Smat, S.size()));
   OG_CHECK(hipMemcpy(h->cproj, c.data(), c.size() * sizeof(double2), hipMemcpyHostToDevice));
@@ -2559,9 +2564,10 @@ int grad_t(H* h, int nE, const double2* xs, const double2* ys, const std::vector
       const auto* W = StateOf<T2>::W(h);
       for (int side = 0; side < 2 && rc == 0; ++side) {
         T2* P = side == 0 ? PX : PY;
-        const Tiles tl = tiles_for<T2, NA>(h);
+        const Tiles tl = tiles_for<T2>(h);
         rc = make_args<T2, NA>(h, side == 0 ? x : y, nullptr, og::F_LR, tl, u, StateOf<T2>::uT(h), P, W, a, g);
         if (rc) break;
+        if ((rc = lds_opt_in(og::k_proj<T2, NA>, g.sm_proj))) break;
         og::k_proj<T2, NA><<<g.nblk_proj, tl.proj, g.sm_proj, h->stream>>>(a);
         const size_t tile = (size_t)h->nk * a.G;
         const size_t smf = (3 * (size_t)g.lmax + tile + tile / 8 + 1) * sizeof(T2);
@@ -2915,7 +2921,6 @@ int ocean_gpu_batch_create(ocean_gpu_handle* const* hs, int32_t n, ocean_gpu_bat
       return g.prec == key.prec && g.NA == key.NA && g.lmax == key.lmax;
     });
     if (it == b->groups.end()) {
-      if (key.prec != OCEAN_GPU_FP64 && key.NA < 6) key.tiles.proj = Tiles{}.proj / 2;  // same x per workgroup
       b->groups.push_back(key);
       it = b->groups.end() - 1;
     }
@@ -3027,9 +3032,7 @@ int ocean_gpu_batch_autotune(ocean_gpu_batch* b, int32_t reps) {
 }
 
 // One problem's tiles by the batch autotuner on a batch of that problem alone (the
-// batched kernels run the single-problem bodies).  The single-problem launch derives
-// its FP32 projection workgroup from the handle's tile (tiles_for), so the pick is
-// stored in the handle's convention.
+// batched kernels run the single-problem bodies).
 int ocean_gpu_autotune(ocean_gpu_handle* h, int32_t reps) {
   if (!h || reps <= 0) return OCEAN_GPU_ERR_ARG;
   ocean_gpu_batch* b = nullptr;
@@ -3037,9 +3040,7 @@ int ocean_gpu_autotune(ocean_gpu_handle* h, int32_t reps) {
   int rc = ocean_gpu_batch_autotune(b, reps);
   if (rc == 0 && b->groups.size() == 1) {
     const B::Group& gr = b->groups[0];
-    Tiles t = gr.tiles;
-    if (gr.prec == OCEAN_GPU_MIXED) t.proj = gr.NA < 6 ? 2 * t.proj : std::max(64, t.proj / 2);
-    h->tiles = t;
+    h->tiles = gr.tiles;
   }
   ocean_gpu_batch_destroy(b);
   return rc;

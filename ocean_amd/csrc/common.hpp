@@ -32,6 +32,7 @@ namespace og {
 constexpr int kBlock = 256;      // threads per workgroup for streaming kernels
 constexpr int kRedBlocks = 256;  // fixed partial count: deterministic reductions
 constexpr int kMaxAlpha = 12;    // nalpha <= 4 (2 lc + 1) with lc <= 1
+constexpr int kMultBlocks = 64;  // most multiplet workgroups (partials per amplitude) of a projection
 constexpr int kMaxDim = 24;      // largest k-mesh edge handled by the LDS DFT
 
 // Tile shapes of the action kernels (defaults; the autotuner picks per batch group).
@@ -45,6 +46,30 @@ struct Tiles {
 
 // accumulator of one 16x16x4 FP64 matrix-core instruction (four rows per lane)
 typedef double __attribute__((ext_vector_type(4))) og_d4;
+typedef float __attribute__((ext_vector_type(4))) og_f4;  // and of the FP32 one
+
+// One 16x16x4 matrix-core step in either precision, and the output row of a lane's
+// r-th accumulator: the f64 form returns rows l/16 + 4r, the f32 form 4(l/16) + r
+// (both measured on gfx950).
+template <typename T> struct Mf;
+template <> struct Mf<double> {
+  using V = og_d4;
+  static __device__ __forceinline__ V step(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int kk, int r) { return kk + 4 * r; }
+  static __device__ __forceinline__ int kk_of(int row) { return row & 3; }
+  static __device__ __forceinline__ int r_of(int row) { return row >> 2; }
+};
+template <> struct Mf<float> {
+  using V = og_f4;
+  static __device__ __forceinline__ V step(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int kk, int r) { return 4 * kk + r; }
+  static __device__ __forceinline__ int kk_of(int row) { return row >> 2; }
+  static __device__ __forceinline__ int r_of(int row) { return row & 3; }
+};
 
 // complex helpers (double2 / float2 as interleaved complex)
 template <typename T2> struct Scalar;
@@ -210,7 +235,7 @@ struct ocean_gpu_handle {
   // multiplet state
   double2* cproj = nullptr; // [s][k][p][n]
   double2* Kmat = nullptr;  // (P*na)^2, h_i = sum_j K[i*(P*na)+j] a_j, i=(a*P+p)
-  double2* apart = nullptr; // [a*P+p][k] projection partials
+  double2* apart = nullptr; // [kMultBlocks][a*P+p] multiplet projection partials
   double2* amp = nullptr;   // [a*P+p]   summed over k
   double2* hmult = nullptr; // [a*P+p]   = mul K amp
   int* mcount = nullptr;    // arrival counter of the reduction workgroups (rests at 0)

@@ -31,32 +31,6 @@ __device__ __forceinline__ MfCol mf_col(int G, int na, int nk) {
   return r;
 }
 
-
-typedef float __attribute__((ext_vector_type(4))) og_f4;
-
-// One 16x16x4 matrix-core step in either precision, and the output row of a lane's
-// r-th accumulator: the f64 form returns rows l/16 + 4r, the f32 form 4(l/16) + r
-// (both measured on gfx950).
-template <typename T> struct Mf;
-template <> struct Mf<double> {
-  using V = og_d4;
-  static __device__ __forceinline__ V step(double a, double b, V c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int kk, int r) { return kk + 4 * r; }
-  static __device__ __forceinline__ int kk_of(int row) { return row & 3; }
-  static __device__ __forceinline__ int r_of(int row) { return row >> 2; }
-};
-template <> struct Mf<float> {
-  using V = og_f4;
-  static __device__ __forceinline__ V step(float a, float b, V c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int kk, int r) { return 4 * kk + r; }
-  static __device__ __forceinline__ int kk_of(int row) { return row >> 2; }
-  static __device__ __forceinline__ int r_of(int row) { return row & 3; }
-};
-
 // The adjoint for the many-alpha edges (one spin), on the matrix cores:
 //   lr(n, k, a) = sum_x conj(uT(k, x, n)) phi'(k, x, a)          (long_range.f90:943-961)
 // as a GEMM per k (M = bands, N = the 2 nalpha real columns, K = x) in the precision

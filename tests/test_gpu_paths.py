@@ -77,6 +77,33 @@ def test_action_matches_oracle(name):
             assert err < 1e-5, (name, back, err)
 
 
+@pytest.mark.parametrize("spec", [
+    dict(nb=1, kmesh=(1, 1, 1), xmesh=(1, 1, 1), seed=71),                     # one of everything
+    dict(nb=3, kmesh=(2, 1, 1), xmesh=(31, 1, 1), lc=1, seed=72, xi_eV=2.0),   # a point short of a 32-point tile
+    dict(nb=4, kmesh=(3, 1, 1), xmesh=(32, 4, 1), seed=73),                    # whole FP64 workgroups of x
+    dict(nb=5, kmesh=(1, 2, 1), xmesh=(43, 3, 1), lc=1, seed=74),              # a point past one
+    dict(nb=17, kmesh=(2, 2, 1), xmesh=(13, 5, 1), lc=1, seed=75, lmax=4),     # 25 projectors: two tiles of 16
+    dict(nb=64, kmesh=(5, 2, 2), xmesh=(257, 1, 1), seed=76),                  # whole multiplet units; FP32 tile + 1
+    dict(nb=65, kmesh=(3, 5, 5), xmesh=(5, 14, 1), seed=77, lmin=1, lmax=2),   # two units per k, more than partials
+    dict(nb=18, kmesh=(3, 4, 5), xmesh=(5, 6, 7), nspn=2, seed=78),            # two spins: strided columns of phi
+], ids=lambda d: f"nb{d['nb']}x{np.prod(d['xmesh'])}")
+def test_action_at_tile_edges(spec):
+    """Bands around the four-band steps and 64-band units, x meshes around the wave and
+    workgroup tiles, projectors around 16: the bars of the other action tests."""
+    inp = synth.make_inputs(**spec)
+    P = to_problem(inp)
+    with core.OceanGPU.from_inputs(inp) as g:
+        psi = _rand(g.shape, 5)
+        for prec, tol in ((core.FP64, 1e-12), (core.MIXED, 1e-5)):
+            g.set_precision(prec)
+            for back in (False, True):
+                err = relerr(g.xact(psi, backwards=back), orc.xact(P, psi, backwards=back))
+                print("  precision", prec, "backwards", back, "relerr", err, flush=True)
+                assert err < tol
+            hf = (0, 0, 0, 0, 1, 0)  # the multiplet term alone
+            assert relerr(g.xact(psi, hflag=hf), orc.xact(P, psi, hflag=hf)) < 1e-12
+
+
 @pytest.mark.parametrize("spec", [dict(nb=8, kmesh=(8, 8, 8), xmesh=(3, 3, 3), lc=0, seed=61),
                                   dict(nb=5, kmesh=(8, 8, 8), xmesh=(5, 1, 1), lc=1, seed=62, xi_eV=2.0)])
 def test_cube8_transform_every_strip_width(spec):
