@@ -117,10 +117,8 @@ struct ActArgs {
   const double* allow;
   const double2* cproj;       // [s][k][p][n]
   double2* apart;             // [nm][a*P+p] multiplet partials
-  double2* amp;               // [a*P+p]
   const double2* Kmat;        // (na P)^2
   double2* hmult;             // [a*P+p]
-  int* mcount;                // reduction arrival counter (rests at 0)
   const double2* S;           // [a][b] over the na0 alphas of one right-hand side
   double mul;                 // inter_scale / (N_k celvol)
   int nb, nk, nx, na, ns, P, nj;
@@ -486,6 +484,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 // F_+ = FFTW_BACKWARD (exp +2 pi i), F_- = FFTW_FORWARD, k3 fastest
 // (Modules/FFT_wrapper.f90:67-72, :185-215).  One pencil per thread; edge classes
 // LMAX = 8, 16 and 24 (radix 2 for powers of two up to 16, direct sums otherwise).
+// FP32 took as long as FP64 although it moves half the bytes: instructions bound it, most
+// of them index arithmetic (two run-time divisions per pencil and a shift, a multiply
+// and two adds per element), and, in small problems and with many amplitudes, the
+// workgroups of the multiplet reduction in its grid.  With linear tile strides, divisions
+// by multiplication, halved direct sums and reduction workgroups that do not wait for
+// each other, per launch between events, us (before -> after):
+//   512 k points, 2 048 columns: FP64 18.2 -> 15.3, FP32 16.9 -> 13.0
+//   512 k points, 12 000 columns, 192 amplitudes: FP64 54.8 -> 45.9, FP32 47.7 -> 27.4
+//   64 k points, 864 columns, FP64: 12.6 -> 7.1
 // ---------------------------------------------------------------------------
 template <int L>
 __device__ __forceinline__ constexpr int bitrev(int i) {
@@ -494,17 +501,125 @@ __device__ __forceinline__ constexpr int bitrev(int i) {
   return r;
 }
 
-// LDS index of tile element e with one pad slot every 8 elements: pencils along
-// the fastest k dimension start 8G elements apart, which without the pad would
-// land on the same LDS banks.
-__device__ __forceinline__ int lidx(int e) { return e + (e >> 3); }
+// n / d for the small tile indices, from r = 1 / d rounded to FP32: (n + 1/2) / d is at
+// least 1 / (2 d) away from a whole number, more than its rounding error for n < 2^21
+// (three instructions; a division by a run-time value takes about thirty, and every
+// pencil of every pass needs one or two).
+__device__ __forceinline__ int qdiv(int n, float r) { return (int)(((float)n + 0.5f) * r); }
 
-// One pass of length-L pencils along the k dimension of stride S, over the G
-// columns of the strip: out[m] = sum_j v[j] w^(j m), w = exp(sign 2 pi i / L),
-// tw[m] = w^m from LDS.  Power-of-two L: radix-2 decimation in time on data
-// loaded in bit-reversed order; otherwise the direct sum.  ld(k, g) / st(k, g, v)
-// move one element, so the first pass reads HBM straight into the pencil
-// registers and the last writes HBM from them.
+// The strip in LDS: element (k1, k2, k3, g) at k1 P1 + k2 P2 + k3 G + g.  An even K3
+// gets one more group of G per (k1, k2) row, so that the pencils of neighbouring rows
+// along k3 start on different banks (P2 / G is odd); every stride is linear, so a
+// pencil's addresses are one sum each.
+__host__ __device__ __forceinline__ int tile_pad(int K3, int G) { return (K3 & 1) ? 0 : G; }
+__host__ __device__ __forceinline__ size_t tile_size(int K1, int K2, int K3, int G) {
+  return (size_t)K1 * K2 * (K3 * G + tile_pad(K3, G));
+}
+
+// Pencil q of a pass along one dimension of the LDS tile: q + (q / D) M is the LDS
+// index of its first element and st the stride.
+template <typename T2>
+struct LdsPencil {
+  T2* p;
+  int st;
+  __device__ __forceinline__ T2 ld(int j) const { return p[j * st]; }
+  __device__ __forceinline__ void put(int j, T2 v) const { p[j * st] = v; }
+};
+template <typename T2>
+struct LdsPass {
+  T2* base;
+  float rD;
+  int M, st;
+  __device__ __forceinline__ LdsPencil<T2> at(int q) const { return {base + q + qdiv(q, rD) * M, st}; }
+};
+
+// Pencil q = r G + g of the phi columns in HBM, its rows starting at r * k0 with stride ks;
+// columns past the strip's gcnt repeat the last one and are not written back.
+template <typename T2>
+struct HbmPencil {
+  T2* p;
+  size_t st;
+  bool ok;
+  __device__ __forceinline__ T2 ld(int j) const { return p[j * st]; }
+  __device__ __forceinline__ void put(int j, T2 v) const { if (ok) p[j * st] = v; }
+};
+template <typename T2>
+struct HbmPass {
+  T2* base;
+  size_t ld;
+  float rG;
+  int G, gcnt, k0, ks;
+  __device__ __forceinline__ HbmPencil<T2> at(int q) const {
+    const int r = qdiv(q, rG), g = q - r * G;
+    return {base + (size_t)(r * k0) * ld + min(g, gcnt - 1), ks * ld, g < gcnt};
+  }
+};
+
+// W of the pencils along k1 (q = lo G + g, lo = (k2, k3)): wl holds W(x, :) of the strip's
+// x points, the strip's column g belonging to x (off + g) / na.
+template <typename T>
+struct WPencil {
+  const T* p;
+  int st;
+  __device__ __forceinline__ T ld(int j) const { return p[j * st]; }
+};
+template <typename T>
+struct WPass {
+  const T* wl;
+  float rG, rna;
+  int G, gcnt, off, nk, st;
+  __device__ __forceinline__ WPencil<T> at(int q) const {
+    const int lo = qdiv(q, rG), g = q - lo * G;
+    return {wl + qdiv(off + min(g, gcnt - 1), rna) * nk + lo, st};
+  }
+};
+
+// The OBF form's phi columns along k3: multiplied by the phase phs(k, x) as they are read,
+// by its conjugate as they are written; both forms scale by inv on the way out.
+template <typename T2, bool PHS>
+struct PhiPencil {
+  using T = typename Scalar<T2>::T;
+  HbmPencil<T2> h;
+  const T2* ph;
+  T inv;
+  __device__ __forceinline__ T2 ld(int j) const {
+    const T2 v = h.ld(j);
+    if constexpr (PHS) return cmul(v, ph[j]);
+    else return v;
+  }
+  __device__ __forceinline__ void put(int j, T2 v) const {
+    if (!h.ok) return;
+    if constexpr (PHS) {
+      const T2 p = ph[j];
+      v = cmake<T2>(v.x * p.x + v.y * p.y, v.y * p.x - v.x * p.y);
+    }
+    h.p[j * h.st] = cmake<T2>(v.x * inv, v.y * inv);
+  }
+};
+template <typename T2, bool PHS>
+struct PhiPass {
+  using T = typename Scalar<T2>::T;
+  HbmPass<T2> h;
+  const T2* phs;  // phs(0, x) of the strip's first x
+  float rna;
+  int off, nk, K3;
+  T inv;
+  __device__ __forceinline__ PhiPencil<T2, PHS> at(int q) const {
+    const T2* ph = nullptr;
+    if constexpr (PHS) {
+      const int r = qdiv(q, h.rG), g = q - r * h.G;
+      ph = phs + (size_t)qdiv(off + min(g, h.gcnt - 1), rna) * nk + r * K3;
+    }
+    return {h.at(q), ph, inv};
+  }
+};
+
+// One pass of length-L pencils along one k dimension, over the G columns of the strip:
+// out[m] = sum_j v[j] w^(j m), w = exp(sign 2 pi i / L), tw[m] = w^m from LDS.
+// Power-of-two L: radix-2 decimation in time on data loaded in bit-reversed order;
+// otherwise the direct sum.  src and dst give a pencil's accessor (LdsPass, HbmPass),
+// so the first pass reads HBM straight into the pencil registers and the last writes
+// HBM from them.
 // cos and sin of 2 pi m / 16, correctly rounded (c1 = cos(pi/8), s1 = sin(pi/8),
 // r = sqrt(2)/2): the power-of-two twiddles
 #define OG_C1 0.92387953251128674
@@ -533,46 +648,6 @@ __device__ __forceinline__ T2 tw_mul(int m, T2 v) {
   return cmake<T2>(c * v.x - sn * v.y, c * v.y + sn * v.x);
 }
 
-template <typename T2, int L, int SIGN, typename Ld, typename St>
-__device__ __forceinline__ void dft_pass(const T2* __restrict__ tw, int G, int nk, int S, Ld ld, St st) {
-  const int npen = (G * nk) / L;
-  for (int q = threadIdx.x; q < npen; q += blockDim.x) {
-    const int g = q % G, r = q / G;
-    const int base = (r / S) * (S * L) + (r % S);
-    T2 v[L];
-    if constexpr ((L & (L - 1)) == 0) {
-#pragma unroll
-      for (int j = 0; j < L; ++j) v[bitrev<L>(j)] = ld(base + j * S, g);
-#pragma unroll
-      for (int len = 2; len <= L; len <<= 1) {
-        const int half = len / 2, step = L / len;
-#pragma unroll
-        for (int i = 0; i < L; i += len) {
-#pragma unroll
-          for (int j = 0; j < half; ++j) {
-            const T2 t = tw_mul<SIGN, L>(j * step, v[i + j + half]);
-            const T2 u = v[i + j];
-            v[i + j] = cmake<T2>(u.x + t.x, u.y + t.y);
-            v[i + j + half] = cmake<T2>(u.x - t.x, u.y - t.y);
-          }
-        }
-      }
-#pragma unroll
-      for (int m = 0; m < L; ++m) st(base + m * S, g, v[m]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < L; ++j) v[j] = ld(base + j * S, g);
-#pragma unroll
-      for (int m = 0; m < L; ++m) {
-        T2 acc = cmake<T2>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; ++j) cfma(acc, v[j], tw[(j * m) % L]);
-        st(base + m * S, g, acc);
-      }
-    }
-  }
-}
-
 // In-register radix-2 DFT of L (a power of two) values given in bit-reversed order;
 // the result is in natural order.
 template <int SIGN, int L, typename T2>
@@ -593,79 +668,140 @@ __device__ __forceinline__ void fft_regs(T2 (&v)[L]) {
   }
 }
 
-// The last forward pass, the W product and the first backward pass fused along one
-// k dimension: each thread keeps its pencil in registers through F_+, W and F_-, so
-// the W product costs no LDS round trip (the 3-D transform is separable: the
-// backward passes may run in the reverse dimension order).
-template <typename T2, int L, typename Ld, typename St, typename Wf>
-__device__ __forceinline__ void dft_pass_w(const T2* __restrict__ twp, const T2* __restrict__ twm, int G, int nk,
-                                           int S, Ld ld, St st, Wf wf) {
-  using T = typename Scalar<T2>::T;
-  const int npen = (G * nk) / L;
+// DFT of L values, L not a power of two, by direct sums over the pairs j, L - j:
+// w^(jm) v_j + w^(-jm) v_(L-j) = c (v_j + v_(L-j)) + i s (v_j - v_(L-j)), and outputs m and
+// L - m share both sums: four multiply-adds for each of the (L/2)^2 pairs instead of
+// four for each of the L^2 terms.  tw[m] = (c, s) of m (s carries the sign), in LDS.
+template <int L, typename T2>
+__device__ __forceinline__ void dft_regs(const T2* __restrict__ tw, T2 (&v)[L]) {
+  constexpr int H = (L - 1) / 2;
+  T2 a[H + 1], b[H + 1];
+#pragma unroll
+  for (int j = 1; j <= H; ++j) {
+    a[j] = cmake<T2>(v[j].x + v[L - j].x, v[j].y + v[L - j].y);
+    b[j] = cmake<T2>(v[j].x - v[L - j].x, v[j].y - v[L - j].y);
+  }
+  const T2 v0 = v[0], vh = v[L / 2];  // vh: the unpaired middle value of an even L
+  T2 sum = v0, alt = v0;
+#pragma unroll
+  for (int j = 1; j <= H; ++j) {
+    sum.x += a[j].x; sum.y += a[j].y;
+    alt.x += (j & 1) ? -a[j].x : a[j].x;
+    alt.y += (j & 1) ? -a[j].y : a[j].y;
+  }
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    T2 e = v0;
+    if constexpr ((L & 1) == 0) {
+      e.x += (m & 1) ? -vh.x : vh.x;
+      e.y += (m & 1) ? -vh.y : vh.y;
+    }
+    T2 o = cmake<T2>(0, 0);
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      const T2 w = tw[(j * m) % L];
+      e.x = fma(w.x, a[j].x, e.x); e.y = fma(w.x, a[j].y, e.y);
+      o.x = fma(-w.y, b[j].y, o.x); o.y = fma(w.y, b[j].x, o.y);
+    }
+    v[m] = cmake<T2>(e.x + o.x, e.y + o.y);
+    v[L - m] = cmake<T2>(e.x - o.x, e.y - o.y);
+  }
+  v[0] = sum;
+  if constexpr ((L & 1) == 0) {
+    v[0] = cmake<T2>(sum.x + vh.x, sum.y + vh.y);
+    constexpr bool neg = ((L / 2) & 1) != 0;
+    v[L / 2] = cmake<T2>(alt.x + (neg ? -vh.x : vh.x), alt.y + (neg ? -vh.y : vh.y));
+  }
+}
+
+template <typename T2, int L, int SIGN, typename Src, typename Dst>
+__device__ __forceinline__ void dft_pass(const T2* __restrict__ tw, int npen, const Src& src, const Dst& dst) {
   for (int q = threadIdx.x; q < npen; q += blockDim.x) {
-    const int g = q % G, r = q / G;
-    const int base = (r / S) * (S * L) + (r % S);
-    T2 v[L], u[L];
+    const auto sp = src.at(q);
+    const auto dp = dst.at(q);
+    T2 v[L];
     if constexpr ((L & (L - 1)) == 0) {
 #pragma unroll
-      for (int j = 0; j < L; ++j) v[bitrev<L>(j)] = ld(base + j * S, g);
-      fft_regs<1, L>(v);
+      for (int j = 0; j < L; ++j) v[bitrev<L>(j)] = sp.ld(j);
+      fft_regs<SIGN, L>(v);
 #pragma unroll
-      for (int m = 0; m < L; ++m) {
-        const T w = wf(base + m * S, g);
-        u[bitrev<L>(m)] = cmake<T2>(v[m].x * w, v[m].y * w);
-      }
-      fft_regs<-1, L>(u);
-#pragma unroll
-      for (int m = 0; m < L; ++m) st(base + m * S, g, u[m]);
+      for (int m = 0; m < L; ++m) dp.put(m, v[m]);
     } else {
 #pragma unroll
-      for (int j = 0; j < L; ++j) v[j] = ld(base + j * S, g);
+      for (int j = 0; j < L; ++j) v[j] = sp.ld(j);
+      dft_regs<L>(tw, v);
 #pragma unroll
-      for (int m = 0; m < L; ++m) {
-        T2 acc = cmake<T2>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; ++j) cfma(acc, v[j], twp[(j * m) % L]);
-        const T w = wf(base + m * S, g);
-        u[m] = cmake<T2>(acc.x * w, acc.y * w);
-      }
-#pragma unroll
-      for (int m = 0; m < L; ++m) {
-        T2 acc = cmake<T2>(0, 0);
-#pragma unroll
-        for (int j = 0; j < L; ++j) cfma(acc, u[j], twm[(j * m) % L]);
-        st(base + m * S, g, acc);
-      }
+      for (int m = 0; m < L; ++m) dp.put(m, v[m]);
     }
   }
 }
 
-template <typename T2, int LMAX, typename Ld, typename St, typename Wf>
-__device__ __forceinline__ void dft_run_w(const T2* twp, const T2* twm, int G, int nk, int L, int S, Ld ld, St st,
-                                          Wf wf) {
+// The last forward pass, the W product and the first backward pass fused along one
+// k dimension: each thread keeps its pencil in registers through F_+, W and F_-, so
+// the W product costs no LDS round trip (the 3-D transform is separable: the
+// backward passes may run in the reverse dimension order).
+template <typename T2, int L, typename Acc, typename Wf>
+__device__ __forceinline__ void dft_pass_w(const T2* __restrict__ twp, const T2* __restrict__ twm, int npen,
+                                           const Acc& acc_, const Wf& wf) {
+  using T = typename Scalar<T2>::T;
+  for (int q = threadIdx.x; q < npen; q += blockDim.x) {
+    const auto p = acc_.at(q);
+    const auto wp = wf.at(q);
+    T2 v[L], u[L];
+    if constexpr ((L & (L - 1)) == 0) {
+#pragma unroll
+      for (int j = 0; j < L; ++j) v[bitrev<L>(j)] = p.ld(j);
+      fft_regs<1, L>(v);
+#pragma unroll
+      for (int m = 0; m < L; ++m) {
+        const T w = wp.ld(m);
+        u[bitrev<L>(m)] = cmake<T2>(v[m].x * w, v[m].y * w);
+      }
+      fft_regs<-1, L>(u);
+#pragma unroll
+      for (int m = 0; m < L; ++m) p.put(m, u[m]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < L; ++j) v[j] = p.ld(j);
+      dft_regs<L>(twp, v);
+#pragma unroll
+      for (int m = 0; m < L; ++m) {
+        const T w = wp.ld(m);
+        u[m] = cmake<T2>(v[m].x * w, v[m].y * w);
+      }
+      dft_regs<L>(twm, u);
+#pragma unroll
+      for (int m = 0; m < L; ++m) p.put(m, u[m]);
+    }
+  }
+}
+
+template <typename T2, int LMAX, typename Acc, typename Wf>
+__device__ __forceinline__ void dft_run_w(const T2* twp, const T2* twm, int npen, int L, const Acc& acc,
+                                          const Wf& wf) {
   switch (L) {
-    case 1: dft_pass_w<T2, 1>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 2: dft_pass_w<T2, 2>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 3: dft_pass_w<T2, 3>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 4: dft_pass_w<T2, 4>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 5: dft_pass_w<T2, 5>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 6: dft_pass_w<T2, 6>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 7: dft_pass_w<T2, 7>(twp, twm, G, nk, S, ld, st, wf); break;
-    case 8: dft_pass_w<T2, 8>(twp, twm, G, nk, S, ld, st, wf); break;
+    case 1: dft_pass_w<T2, 1>(twp, twm, npen, acc, wf); break;
+    case 2: dft_pass_w<T2, 2>(twp, twm, npen, acc, wf); break;
+    case 3: dft_pass_w<T2, 3>(twp, twm, npen, acc, wf); break;
+    case 4: dft_pass_w<T2, 4>(twp, twm, npen, acc, wf); break;
+    case 5: dft_pass_w<T2, 5>(twp, twm, npen, acc, wf); break;
+    case 6: dft_pass_w<T2, 6>(twp, twm, npen, acc, wf); break;
+    case 7: dft_pass_w<T2, 7>(twp, twm, npen, acc, wf); break;
+    case 8: dft_pass_w<T2, 8>(twp, twm, npen, acc, wf); break;
     default:
       if constexpr (LMAX > 8) {
         switch (L) {
-          case 9: dft_pass_w<T2, 9>(twp, twm, G, nk, S, ld, st, wf); break;
-          case 10: dft_pass_w<T2, 10>(twp, twm, G, nk, S, ld, st, wf); break;
-          case 12: dft_pass_w<T2, 12>(twp, twm, G, nk, S, ld, st, wf); break;
-          case 16: dft_pass_w<T2, 16>(twp, twm, G, nk, S, ld, st, wf); break;
+          case 9: dft_pass_w<T2, 9>(twp, twm, npen, acc, wf); break;
+          case 10: dft_pass_w<T2, 10>(twp, twm, npen, acc, wf); break;
+          case 12: dft_pass_w<T2, 12>(twp, twm, npen, acc, wf); break;
+          case 16: dft_pass_w<T2, 16>(twp, twm, npen, acc, wf); break;
           default:
             if constexpr (LMAX > 16) {
               switch (L) {
-                case 15: dft_pass_w<T2, 15>(twp, twm, G, nk, S, ld, st, wf); break;
-                case 18: dft_pass_w<T2, 18>(twp, twm, G, nk, S, ld, st, wf); break;
-                case 20: dft_pass_w<T2, 20>(twp, twm, G, nk, S, ld, st, wf); break;
-                case 24: dft_pass_w<T2, 24>(twp, twm, G, nk, S, ld, st, wf); break;
+                case 15: dft_pass_w<T2, 15>(twp, twm, npen, acc, wf); break;
+                case 18: dft_pass_w<T2, 18>(twp, twm, npen, acc, wf); break;
+                case 20: dft_pass_w<T2, 20>(twp, twm, npen, acc, wf); break;
+                case 24: dft_pass_w<T2, 24>(twp, twm, npen, acc, wf); break;
                 default: break;  // rejected on the host
               }
             }
@@ -676,31 +812,31 @@ __device__ __forceinline__ void dft_run_w(const T2* twp, const T2* twm, int G, i
   }
 }
 
-template <typename T2, int LMAX, int SIGN, typename Ld, typename St>
-__device__ __forceinline__ void dft_run(const T2* tw, int G, int nk, int L, int S, Ld ld, St st) {
+template <typename T2, int LMAX, int SIGN, typename Src, typename Dst>
+__device__ __forceinline__ void dft_run(const T2* tw, int npen, int L, const Src& src, const Dst& dst) {
   switch (L) {
-    case 1: dft_pass<T2, 1, SIGN>(tw, G, nk, S, ld, st); break;
-    case 2: dft_pass<T2, 2, SIGN>(tw, G, nk, S, ld, st); break;
-    case 3: dft_pass<T2, 3, SIGN>(tw, G, nk, S, ld, st); break;
-    case 4: dft_pass<T2, 4, SIGN>(tw, G, nk, S, ld, st); break;
-    case 5: dft_pass<T2, 5, SIGN>(tw, G, nk, S, ld, st); break;
-    case 6: dft_pass<T2, 6, SIGN>(tw, G, nk, S, ld, st); break;
-    case 7: dft_pass<T2, 7, SIGN>(tw, G, nk, S, ld, st); break;
-    case 8: dft_pass<T2, 8, SIGN>(tw, G, nk, S, ld, st); break;
+    case 1: dft_pass<T2, 1, SIGN>(tw, npen, src, dst); break;
+    case 2: dft_pass<T2, 2, SIGN>(tw, npen, src, dst); break;
+    case 3: dft_pass<T2, 3, SIGN>(tw, npen, src, dst); break;
+    case 4: dft_pass<T2, 4, SIGN>(tw, npen, src, dst); break;
+    case 5: dft_pass<T2, 5, SIGN>(tw, npen, src, dst); break;
+    case 6: dft_pass<T2, 6, SIGN>(tw, npen, src, dst); break;
+    case 7: dft_pass<T2, 7, SIGN>(tw, npen, src, dst); break;
+    case 8: dft_pass<T2, 8, SIGN>(tw, npen, src, dst); break;
     default:
       if constexpr (LMAX > 8) {
         switch (L) {
-          case 9: dft_pass<T2, 9, SIGN>(tw, G, nk, S, ld, st); break;
-          case 10: dft_pass<T2, 10, SIGN>(tw, G, nk, S, ld, st); break;
-          case 12: dft_pass<T2, 12, SIGN>(tw, G, nk, S, ld, st); break;
-          case 16: dft_pass<T2, 16, SIGN>(tw, G, nk, S, ld, st); break;
+          case 9: dft_pass<T2, 9, SIGN>(tw, npen, src, dst); break;
+          case 10: dft_pass<T2, 10, SIGN>(tw, npen, src, dst); break;
+          case 12: dft_pass<T2, 12, SIGN>(tw, npen, src, dst); break;
+          case 16: dft_pass<T2, 16, SIGN>(tw, npen, src, dst); break;
           default:
             if constexpr (LMAX > 16) {
               switch (L) {
-                case 15: dft_pass<T2, 15, SIGN>(tw, G, nk, S, ld, st); break;
-                case 18: dft_pass<T2, 18, SIGN>(tw, G, nk, S, ld, st); break;
-                case 20: dft_pass<T2, 20, SIGN>(tw, G, nk, S, ld, st); break;
-                case 24: dft_pass<T2, 24, SIGN>(tw, G, nk, S, ld, st); break;
+                case 15: dft_pass<T2, 15, SIGN>(tw, npen, src, dst); break;
+                case 18: dft_pass<T2, 18, SIGN>(tw, npen, src, dst); break;
+                case 20: dft_pass<T2, 20, SIGN>(tw, npen, src, dst); break;
+                case 24: dft_pass<T2, 24, SIGN>(tw, npen, src, dst); break;
                 default: break;  // rejected on the host
               }
             }
@@ -711,9 +847,8 @@ __device__ __forceinline__ void dft_run(const T2* tw, int G, int nk, int L, int 
   }
 }
 
-__device__ void mred_tail(const double2* __restrict__ apart, double2* __restrict__ amp,
-                          const double2* __restrict__ K, double2* __restrict__ hmult, int* counter,
-                          int np, int nj, int nj0, double mul, int r, int nred, double2* lds);
+__device__ void mred_rows(const double2* __restrict__ apart, const double2* __restrict__ K,
+                          double2* __restrict__ hmult, int np, int nj, int nj0, double mul, int r, double2* lds);
 
 // Strip of G consecutive phi columns (c = x*na + a) per workgroup, all nk rows:
 //   pass 1 (K3, F_+): HBM -> registers -> LDS, with W(x, :) staged beside it
@@ -731,8 +866,7 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
   // the reduction workgroups come first so that they are dispatched first
   const int nred = A.nred, nfft = A.nfft;
   if (blk < nred) {
-    mred_tail(A.apart, A.amp, A.Kmat, A.hmult, A.mcount, A.nm, A.nj, A.na0 * A.P, A.mul, blk, nred,
-              reinterpret_cast<double2*>(smem));
+    mred_rows(A.apart, A.Kmat, A.hmult, A.nm, A.nj, A.na0 * A.P, A.mul, blk, reinterpret_cast<double2*>(smem));
     return;
   }
   const int nk = A.nk, ncol = A.ncol, na = A.na, G = A.G, ldphi = A.ldphi;
@@ -741,8 +875,8 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
   const T* W = A.W;
   // twiddles: [dim][sign][m], dims ordered (K3, K2, K1), 2 * LMAX per dim
   T2* twl = reinterpret_cast<T2*>(smem);
-  T2* lds = twl + 6 * LMAX;                               // [k][g], padded
-  T* wl = reinterpret_cast<T*>(lds + lidx(nk * G - 1) + 1);  // W(x, :) of the strip
+  T2* lds = twl + 6 * LMAX;                               // [k][g], rows padded (tile_pad)
+  T* wl = reinterpret_cast<T*>(lds + tile_size(K1, K2, K3, G));  // W(x, :) of the strip
   const int Ks[3] = {K3, K2, K1};
   // the LDS twiddle table serves the direct sums of non-power-of-two edges only
   const bool direct = ((K1 & (K1 - 1)) | (K2 & (K2 - 1)) | (K3 & (K3 - 1))) != 0;
@@ -772,28 +906,13 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
 #pragma unroll
   for (int i = 0; i < kWR; ++i) wr[i] = wsrc[min((int)threadIdx.x + i * (int)blockDim.x, nwl - 1)];
   __syncthreads();  // twiddles
-  T2* __restrict__ gphi = phi + c0;
-  auto ld_hbm = [&](int k, int g) -> T2 {
-    const int gc = min(g, gcnt - 1);
-    T2 v = gphi[(size_t)k * ldphi + gc];
-    if constexpr (PHS) v = cmul(v, A.phs[(size_t)((c0 + gc) / na) * nk + k]);
-    return g < gcnt ? v : cmake<T2>(0, 0);
-  };
-  auto ld_lds = [&](int k, int g) -> T2 { return lds[lidx(k * G + g)]; };
-  auto st_lds = [&](int k, int g, T2 v) { lds[lidx(k * G + g)] = v; };
-  auto w_at = [&](int k, int g) -> T { return wl[((c0 + min(g, gcnt - 1)) / na - xlo) * nk + k]; };
-  const T inv = (T)1 / (T)nk;
-  auto st_hbm = [&](int k, int g, T2 v) {
-    if (g < gcnt) {
-      if constexpr (PHS) {
-        const T2 p = A.phs[(size_t)((c0 + g) / na) * nk + k];
-        v = cmake<T2>(v.x * p.x + v.y * p.y, v.y * p.x - v.x * p.y);
-      }
-      v.x *= inv; v.y *= inv;
-      gphi[(size_t)k * ldphi + g] = v;
-    }
-  };
-  dft_run<T2, LMAX, 1>(twl + 0 * LMAX, G, nk, K3, 1, ld_hbm, st_lds);
+  const int pad = tile_pad(K3, G), P2 = K3 * G + pad, P1 = K2 * P2, n = nk * G;
+  const float rG = 1.0f / (float)G, rG3 = 1.0f / (float)(K3 * G), rna = 1.0f / (float)na;
+  const int off = c0 - xlo * na;
+  const PhiPass<T2, PHS> hbm{{phi + c0, (size_t)ldphi, rG, G, gcnt, K3, 1},
+                             PHS ? A.phs + (size_t)xlo * nk : nullptr, rna, off, nk, K3, (T)1 / (T)nk};
+  const LdsPass<T2> l3{lds, rG, P2 - G, G}, l2{lds, rG3, P1 - K3 * G, P2}, l1{lds, rG3, pad, P1};
+  dft_run<T2, LMAX, 1>(twl + 0 * LMAX, n / K3, K3, hbm, l3);
 #pragma unroll
   for (int i = 0; i < kWR; ++i) {
     const int idx = threadIdx.x + i * blockDim.x;
@@ -801,14 +920,15 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
   }
   for (int idx = threadIdx.x + kWR * blockDim.x; idx < nwl; idx += blockDim.x) wl[idx] = wsrc[idx];
   __syncthreads();
-  dft_run<T2, LMAX, 1>(twl + 2 * LMAX, G, nk, K2, K3, ld_lds, st_lds);
+  dft_run<T2, LMAX, 1>(twl + 2 * LMAX, n / K2, K2, l2, l2);
   __syncthreads();
   // K1: F_+, W, F_- in registers
-  dft_run_w<T2, LMAX>(twl + 4 * LMAX, twl + 5 * LMAX, G, nk, K1, K2 * K3, ld_lds, st_lds, w_at);
+  dft_run_w<T2, LMAX>(twl + 4 * LMAX, twl + 5 * LMAX, n / K1, K1, l1,
+                      WPass<T>{wl, rG, rna, G, gcnt, off, nk, K2 * K3});
   __syncthreads();
-  dft_run<T2, LMAX, -1>(twl + 3 * LMAX, G, nk, K2, K3, ld_lds, st_lds);
+  dft_run<T2, LMAX, -1>(twl + 3 * LMAX, n / K2, K2, l2, l2);
   __syncthreads();
-  dft_run<T2, LMAX, -1>(twl + 1 * LMAX, G, nk, K3, 1, ld_lds, st_hbm);
+  dft_run<T2, LMAX, -1>(twl + 1 * LMAX, n / K3, K3, l3, hbm);
 }
 
 template <typename T2, int LMAX, bool PHS = false>
@@ -858,21 +978,17 @@ __global__ __launch_bounds__(256) void k_fft_fwd(const ActArgs<T2> A) {
   if ((nfft & 7) == 0) b = (b & 7) * (nfft >> 3) + (b >> 3);
   const int c0 = b * G;
   const int gcnt = min(G, ncol - c0);
-  T2* __restrict__ gphi = A.phi + c0;
-  auto ld_hbm = [&](int k, int g) -> T2 {
-    const T2 v = gphi[(size_t)k * ldphi + min(g, gcnt - 1)];
-    return g < gcnt ? v : cmake<T2>(0, 0);
-  };
-  auto ld_lds = [&](int k, int g) -> T2 { return lds[lidx(k * G + g)]; };
-  auto st_lds = [&](int k, int g, T2 v) { lds[lidx(k * G + g)] = v; };
-  auto st_hbm = [&](int k, int g, T2 v) {
-    if (g < gcnt) gphi[(size_t)k * ldphi + g] = v;
-  };
-  dft_run<T2, LMAX, 1>(twl + 0 * LMAX, G, nk, A.K3, 1, ld_hbm, st_lds);
+  const int K1 = A.K1, K2 = A.K2, K3 = A.K3;
+  const int pad = tile_pad(K3, G), P2 = K3 * G + pad, P1 = K2 * P2, n = nk * G;
+  const float rG = 1.0f / (float)G, rG3 = 1.0f / (float)(K3 * G);
+  const HbmPass<T2> h3{A.phi + c0, (size_t)ldphi, rG, G, gcnt, K3, 1};
+  const HbmPass<T2> h1{A.phi + c0, (size_t)ldphi, rG, G, gcnt, 1, K2 * K3};
+  const LdsPass<T2> l3{lds, rG, P2 - G, G}, l2{lds, rG3, P1 - K3 * G, P2}, l1{lds, rG3, pad, P1};
+  dft_run<T2, LMAX, 1>(twl + 0 * LMAX, n / K3, K3, h3, l3);
   __syncthreads();
-  dft_run<T2, LMAX, 1>(twl + 1 * LMAX, G, nk, A.K2, A.K3, ld_lds, st_lds);
+  dft_run<T2, LMAX, 1>(twl + 1 * LMAX, n / K2, K2, l2, l2);
   __syncthreads();
-  dft_run<T2, LMAX, 1>(twl + 2 * LMAX, G, nk, A.K1, A.K2 * A.K3, ld_lds, st_hbm);
+  dft_run<T2, LMAX, 1>(twl + 2 * LMAX, n / K1, K1, l1, h1);
 }
 
 // Q[k][x] += coef * Im sum_a conj(PY(k,x,a)) PX(k,x,a); one thread per (k, x), each
@@ -929,92 +1045,55 @@ __global__ __launch_bounds__(1024) void k_mred(
   mred_matvec(K, amp, hmult, nj, nj0, mul);
 }
 
-// Reduction run by nred extra workgroups of another kernel's grid: workgroup r sums
-// amplitudes [r*kRedPerBlock, ...) over the np <= kMultBlocks partials into amp
-// (global), one load per thread and a fixed-order tree; the last workgroup to finish
-// (device-scope counter) applies K, four rows per wave at a time with all their loads
-// in flight.  The counter returns to zero for the next launch.  Loads are batched
-// throughout: the whole tail is a few memory latencies, so it hides under the kernel
-// it rides on.
+// Reduction run by extra workgroups of another kernel's grid: workgroup r forms
+// kRedPerBlock rows of h.  Every workgroup sums the np partials of all nj0 amplitudes of
+// its rows' right-hand side (64 x 64 to 64 x 192 values, from L2) and applies its rows of
+// K to them, so that no workgroup waits for another: with the amplitudes shared out
+// over the workgroups and K applied by the last to arrive, the chain of partials,
+// counter, amplitudes and K was the longest workgroup of a small problem's transform.
+// The four waves of a workgroup sum 16 partials each, pairwise; their sums are added in
+// order.
 constexpr int kRedPerBlock = 4;
 
-__device__ void mred_tail(const double2* __restrict__ apart, double2* __restrict__ amp,
-                          const double2* __restrict__ K, double2* __restrict__ hmult, int* counter,
-                          int np, int nj, int nj0, double mul, int r, int nred, double2* lds) {
-  static_assert(kMultBlocks * kRedPerBlock == kBlock, "one partial per thread");
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  {
-    const int j = r * kRedPerBlock + (threadIdx.x & 3), m = threadIdx.x >> 2;
-    double2 v = make_double2(0.0, 0.0);
-    if (j < nj && m < np) v = apart[(size_t)m * nj + j];
+// LDS of one reduction workgroup of nw waves
+constexpr size_t mred_lds(int nj0, int nw) { return (size_t)nj0 * nw * sizeof(double2); }
+
+__device__ void mred_rows(const double2* __restrict__ apart, const double2* __restrict__ K,
+                          double2* __restrict__ hmult, int np, int nj, int nj0, double mul, int r, double2* lds) {
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  const int i0 = r * kRedPerBlock, jb = i0 - i0 % nj0;  // nj0 is a multiple of the four rows
+  constexpr int MW = kMultBlocks / (kBlock / 64), B = 8;
+  for (int j = lane; j < nj0; j += 64) {
+    double2 a = make_double2(0.0, 0.0);
+#pragma unroll 1
+    for (int m0 = wid * MW; m0 < min(wid * MW + MW, np); m0 += B) {
+      double2 v[B];
 #pragma unroll
-    for (int off = 4; off < 64; off <<= 1) {
-      v.x += __shfl_xor(v.x, off, 64);
-      v.y += __shfl_xor(v.y, off, 64);
+      for (int q = 0; q < B; ++q) v[q] = apart[(size_t)min(m0 + q, np - 1) * nj + jb + j];
+#pragma unroll
+      for (int q = 0; q < B; ++q)
+        if (m0 + q >= np) v[q] = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int d = 1; d < B; d <<= 1)
+#pragma unroll
+        for (int q = 0; q < B; q += 2 * d) { v[q].x += v[q + d].x; v[q].y += v[q + d].y; }
+      a.x += v[0].x; a.y += v[0].y;
     }
-    if (lane < kRedPerBlock) lds[wid * kRedPerBlock + lane] = v;
-    __syncthreads();
-    if (threadIdx.x < kRedPerBlock && j < nj) {
-      double2 a = make_double2(0.0, 0.0);
-      for (int q = 0; q < nw; ++q) {
-        a.x += lds[q * kRedPerBlock + threadIdx.x].x;
-        a.y += lds[q * kRedPerBlock + threadIdx.x].y;
-      }
-      amp[j] = a;
-    }
-  }
-  __threadfence();
-  __syncthreads();
-  __shared__ int is_last;
-  if (threadIdx.x == 0) is_last = (atomicAdd(counter, 1) == nred - 1);
-  __syncthreads();
-  if (!is_last) return;
-  __threadfence();
-  for (int j = threadIdx.x; j < nj; j += blockDim.x) {
-    // other workgroups (possibly on other XCDs) wrote amp: device-scope loads
-    const double ax = __hip_atomic_load(&amp[j].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const double ay = __hip_atomic_load(&amp[j].y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    lds[j] = make_double2(ax, ay);
+    lds[wid * nj0 + j] = a;
   }
   __syncthreads();
-  // K is block diagonal over right-hand sides (blocks of nj0): each row sums its own
-  // block, and a pass of R rows runs over the columns of the blocks they touch
-  // four rows per pass: eight took the transform kernel this rides on to 198 VGPRs
-  // (two waves per SIMD) from 79
-  constexpr int R = 4;
-  for (int i0 = wid * R; i0 < nj; i0 += nw * R) {
-    double v[2 * R];
-#pragma unroll
-    for (int q = 0; q < 2 * R; ++q) v[q] = 0.0;
-    const int iend = min(i0 + R, nj) - 1;
-    const int c_lo = i0 - i0 % nj0, c_hi = iend - iend % nj0 + nj0;
-    int rb[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) rb[q] = (min(i0 + q, nj - 1)) / nj0;
-    for (int c0 = c_lo; c0 < c_hi; c0 += 64) {
-      const int j = c0 + lane;
-      const int jc = min(j, nj - 1);
-      double2 kv[R];
-#pragma unroll
-      for (int q = 0; q < R; ++q) kv[q] = K[(size_t)min(i0 + q, nj - 1) * nj + jc];
-      const double2 a = lds[jc];
-      if (j < c_hi) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          if (j / nj0 != rb[q]) continue;
-          v[2 * q] = fma(kv[q].x, a.x, v[2 * q]); v[2 * q] = fma(-kv[q].y, a.y, v[2 * q]);
-          v[2 * q + 1] = fma(kv[q].x, a.y, v[2 * q + 1]); v[2 * q + 1] = fma(kv[q].y, a.x, v[2 * q + 1]);
-        }
-      }
+  for (int i = i0 + wid; i < min(i0 + kRedPerBlock, nj); i += nw) {
+    double2 acc = make_double2(0.0, 0.0);
+    for (int j = lane; j < nj0; j += 64) {
+      const double2 kv = K[(size_t)i * nj + jb + j];
+      double2 a = lds[j];
+      for (int q = 1; q < nw; ++q) { a.x += lds[q * nj0 + j].x; a.y += lds[q * nj0 + j].y; }
+      cfma(acc, kv, a);
     }
-    int owner = 0;
-    const double tot = wave_multi_sum<double, 2 * R>(v, lane, &owner);
-    if ((lane & (64 / (2 * R) - 1)) == 0) {
-      const int q = owner >> 1;
-      if (i0 + q < nj) reinterpret_cast<double*>(hmult + i0 + q)[owner & 1] = tot * mul;
-    }
+    acc.x = wave_sum(acc.x);
+    acc.y = wave_sum(acc.y);
+    if (lane == 0) hmult[i] = make_double2(acc.x * mul, acc.y * mul);
   }
-  if (threadIdx.x == 0) atomicExch(counter, 0);
 }
 
 // ---------------------------------------------------------------------------

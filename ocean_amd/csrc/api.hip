@@ -189,8 +189,8 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   a.u = u; a.uT = uT; a.phi = phi; a.W = W;
   a.psi = in; a.out = out;
   a.energy = h->energy; a.allow = h->allow;
-  a.cproj = h->cproj; a.apart = h->apart; a.amp = h->amp; a.Kmat = h->Kmat; a.hmult = h->hmult;
-  a.mcount = h->mcount; a.S = h->Smat;
+  a.cproj = h->cproj; a.apart = h->apart; a.Kmat = h->Kmat; a.hmult = h->hmult;
+  a.S = h->Smat;
   a.mul = h->d.inter_scale / ((double)nk * h->d.celvol);
   a.nb = nb; a.nk = nk; a.nx = nx; a.na = na; a.ns = ns; a.P = h->P; a.nj = na * h->P; a.na0 = h->na0;
   a.ldu = bs ? bs->ldu : h->ldu;
@@ -218,11 +218,14 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   // transform
   a.ncol = nx * na;
   const int cap = (int)(57344 / sizeof(T2)) / nk;
-  // default strip: 2048 elements; stacked right-hand sides in FP32 on a 512-point
-  // k mesh take twice that (measured: six polarisations 173.3 -> 172.0 us, three
-  // 127.2 -> 125.8 us per action; one right-hand side and L2,3 are not helped)
+  // default strip: 2048 elements, one pencil of eight per thread and pass (twice that at
+  // 512 k points, 12 000 columns: FP32 25.2 -> 39.3 us, FP64 43 -> 71)
   int Gdef = std::min((256 * 8) / nk, cap);
-  if (sizeof(T) == 4 && h->nrhs > 1 && nk >= 512) Gdef = std::min(2 * Gdef, cap);
+  // a short vector's strips are narrowed to one per compute unit, but not below 64-byte
+  // row segments: 864 columns at 64 k points, 27 strips of 32 columns 8.8 us, 108 of 8 or
+  // 216 of 4 columns 6.9 us
+  const int Gfill = (((a.ncol + h->ncu - 1) / h->ncu) + 3) & ~3;
+  Gdef = std::min(Gdef, std::max(Gfill, (int)(64 / sizeof(T2))));
   int G = t.G > 0 ? t.G : Gdef;
   G = std::max(1, std::min(std::min(G, std::max(cap, 1)), a.ncol));
   a.G = G;
@@ -230,10 +233,10 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   a.nred = (lr && fg) ? (a.nj + og::kRedPerBlock - 1) / og::kRedPerBlock : 0;
   a.K1 = h->km[0]; a.K2 = h->km[1]; a.K3 = h->km[2];
   g.lmax = edge_class(h->km);
-  const size_t tile = (size_t)nk * G;
-  g.sm_fft = (6 * (size_t)g.lmax + tile + tile / 8 + 1) * sizeof(T2) +
-             (size_t)((G - 1) / na + 2) * nk * sizeof(T);
-  g.sm_fft = std::max(g.sm_fft, (size_t)a.nj * sizeof(double2));
+  // x points of a strip: a strip that divides nalpha, or the reverse, starts on one
+  const int xs = na % G == 0 ? 1 : G % na == 0 ? G / na : (G - 1) / na + 2;
+  g.sm_fft = (6 * (size_t)g.lmax + og::tile_size(a.K1, a.K2, a.K3, G)) * sizeof(T2) + (size_t)xs * nk * sizeof(T);
+  if (a.nred) g.sm_fft = std::max(g.sm_fft, og::mred_lds(h->na0 * h->P, kBlock / 64));
   if (g.sm_fft > h->lds_max || g.sm_proj > h->lds_max) return OCEAN_GPU_ERR_ARG;  // k mesh or bands too large
   g.nblk_fft = a.nred + a.nfft;
   // adjoint: x-splits, phi' chunk and reduction rounds sharing one LDS area
@@ -317,6 +320,7 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
     OG_CHECK(hipGetLastError());
     if (ev) OG_CHECK(hipEventRecord(ev[1], h->stream));
     if (g.lmax == 8) {
+      OG_TRY(lds_opt_in(og::k_fft_w<T2, 8>, g.sm_fft));
       og::k_fft_w<T2, 8><<<g.nblk_fft, kBlock, g.sm_fft, h->stream>>>(a);
     } else if (g.lmax == 16) {
       OG_TRY(lds_opt_in(og::k_fft_w<T2, 16>, g.sm_fft));
@@ -408,6 +412,7 @@ int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev,
       h->obf_beta, h->ldb, h->obf_f, h->phi64, h->ldphi, nk, nx, no);
   OG_CHECK(hipGetLastError());
   if (g.lmax == 8) {
+    OG_TRY(lds_opt_in(og::k_fft_w<double2, 8, true>, g.sm_fft));
     og::k_fft_w<double2, 8, true><<<g.nblk_fft, kBlock, g.sm_fft, h->stream>>>(a);
   } else if (g.lmax == 16) {
     OG_TRY(lds_opt_in(og::k_fft_w<double2, 16, true>, g.sm_fft));
@@ -1178,7 +1183,6 @@ int ocean_gpu_destroy(ocean_gpu_handle* h) {
   dfree(h->w_i0); dfree(h->w_w0); dfree(h->w_w1);
   dfree(h->obf_u); dfree(h->obf_uT); dfree(h->obf_f); dfree(h->obf_fT); dfree(h->obf_phs); dfree(h->obf_beta);
   dfree(h->cproj); dfree(h->Kmat); dfree(h->apart); dfree(h->hmult); dfree(h->Smat);
-  dfree(h->amp); dfree(h->mcount);
   dfree(h->energy); dfree(h->allow); dfree(h->red); dfree(h->scal); dfree(h->tmp_in); dfree(h->tmp_out);
   for (auto& v : h->vecs) dfree(v);
   if (h->host_pin) (void)hipHostFree(h->host_pin);
@@ -1463,11 +1467,7 @@ int ocean_gpu_load_mult(ocean_gpu_handle* h, const double* mpcr, const double* m
   for (int a = 0; a < na; ++a)
     for (int b = 0; b < na; ++b) S[a * na + b] = make_double2(somelr[(size_t)b * na + a], someli[(size_t)b * na + a]);
   dfree(h->cproj); dfree(h->Kmat); dfree(h->apart); dfree(h->hmult); dfree(h->Smat);
-  dfree(h->amp); dfree(h->mcount);
   OG_TRY(dmalloc(&h->cproj, c.size()));
-  OG_TRY(dmalloc(&h->amp, (size_t)njt));
-  OG_TRY(dmalloc(&h->mcount, (size_t)1));
-  OG_CHECK(hipMemset(h->mcount, 0, sizeof(int)));
   OG_TRY(dmalloc(&h->Kmat, Kd.size()));
   OG_TRY(dmalloc(&h->apart, (size_t)og::kMultBlocks * njt));
   OG_TRY(dmalloc(&h->hmult, (size_t)njt));
@@ -2569,9 +2569,9 @@ int grad_t(H* h, int nE, const double2* xs, const double2* ys, const std::vector
         if (rc) break;
         if ((rc = lds_opt_in(og::k_proj<T2, NA>, g.sm_proj))) break;
         og::k_proj<T2, NA><<<g.nblk_proj, tl.proj, g.sm_proj, h->stream>>>(a);
-        const size_t tile = (size_t)h->nk * a.G;
-        const size_t smf = (3 * (size_t)g.lmax + tile + tile / 8 + 1) * sizeof(T2);
+        const size_t smf = (3 * (size_t)g.lmax + og::tile_size(a.K1, a.K2, a.K3, a.G)) * sizeof(T2);
         if (g.lmax == 8) {
+          if ((rc = lds_opt_in(og::k_fft_fwd<T2, 8>, smf))) break;
           og::k_fft_fwd<T2, 8><<<a.nfft, kBlock, smf, h->stream>>>(a);
         } else if (g.lmax == 16) {
           if ((rc = lds_opt_in(og::k_fft_fwd<T2, 16>, smf))) break;
@@ -2806,6 +2806,7 @@ int launch_tables(const Tables& tb, hipStream_t st, int stages) {
   }
   if (stages & 2) {
     if (tb.lmax == 8) {
+      OG_TRY(lds_opt_in(og::k_fft_w_batch<T2, 8>, tb.sm[1]));
       og::k_fft_w_batch<T2, 8><<<tb.nblk[1], kBlock, tb.sm[1], st>>>(A, tb.off + (np + 1), np);
     } else if (tb.lmax == 16) {
       OG_TRY(lds_opt_in(og::k_fft_w_batch<T2, 16>, tb.sm[1]));

@@ -236,9 +236,7 @@ struct ocean_gpu_handle {
   double2* cproj = nullptr; // [s][k][p][n]
   double2* Kmat = nullptr;  // (P*na)^2, h_i = sum_j K[i*(P*na)+j] a_j, i=(a*P+p)
   double2* apart = nullptr; // [kMultBlocks][a*P+p] multiplet projection partials
-  double2* amp = nullptr;   // [a*P+p]   summed over k
   double2* hmult = nullptr; // [a*P+p]   = mul K amp
-  int* mcount = nullptr;    // arrival counter of the reduction workgroups (rests at 0)
   double2* Smat = nullptr;  // [a][b]
   int have_so = 0;
 

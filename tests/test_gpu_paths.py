@@ -130,6 +130,28 @@ def test_cube8_transform_every_strip_width(spec):
                     assert np.array_equal(o, outs[0])
 
 
+@pytest.mark.parametrize("kmesh,lc,lmax", [((7, 6, 3), 0, 3), ((5, 3, 7), 1, 3), ((6, 5, 2), 1, 2), ((3, 7, 6), 0, 4)])
+def test_transform_odd_edges_every_strip_width(kmesh, lc, lmax):
+    """Direct sums at 3, 5, 6 and 7 points in each position, padded (even k3) and unpadded
+    tile rows, strips that do and do not divide the alphas (ragged at the end), and the
+    reduction rows of 4 to 25 projectors: the bars of the other action tests, and the
+    widths agree bit for bit."""
+    inp = synth.make_inputs(nb=9, kmesh=kmesh, xmesh=(5, 3, 2), lc=lc, seed=81, lmax=lmax, xi_eV=2.0 if lc else 0.0)
+    P = to_problem(inp)
+    with core.OceanGPU.from_inputs(inp) as g:
+        psi = _rand(g.shape, 6)
+        for prec, tol in ((core.FP64, 1e-12), (core.MIXED, 1e-5)):
+            g.set_precision(prec)
+            ref = orc.xact(P, psi)
+            outs = []
+            for G in (0, 1, 3, 4, 6, 8, 12):
+                g.set_tiles(256, 512, G, -1)
+                outs.append(g.xact(psi))
+            assert relerr(outs[0], ref) < tol
+            for o in outs[1:]:
+                assert np.array_equal(o, outs[0])
+
+
 @pytest.mark.parametrize("name", ["k16", "l23_x512_nb72", "k24"])
 def test_haydock_matches_oracle(name):
     inp = synth.make_inputs(**dict(WIDE, **EDGES)[name])
