@@ -273,6 +273,12 @@ bool adj_mf(const H* h, int flags, const Tiles& t) {
   return t.adj_mf != 0;
 }
 
+// The matrix-core adjoint's tile: 64 bands on four waves, or, where that grid would leave
+// compute units idle, half the bands on twice the waves.  The rule looks at the problem
+// alone, so that a batch sums in the same order as its members on their own.
+bool adj_small(const H* h) { return ((h->nb + 63) / 64) * h->nk < h->ncu; }
+int adj_lr_blocks(const H* h) { return (adj_small(h) ? (h->nb + 31) / 32 : (h->nb + 63) / 64) * h->nk; }
+
 // The device state of one precision form.
 template <typename T2> struct StateOf;
 template <> struct StateOf<double2> {
@@ -352,12 +358,10 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
     // 24 alphas (several right-hand sides on one spin) have the matrix-core adjoint only
     if (NA > 12 && !mf) return OCEAN_GPU_ERR_UNSUPPORTED;
     if (mf) {
-      // the deep load ring where two workgroups per CU hold the whole grid
-      const int nwg = ((h->nb + 63) / 64) * h->nk;
-      if (nwg <= 2 * h->ncu)
-        og::k_adj_lr<T2, NA, true><<<nwg, 256, 0, h->stream>>>(a);
+      if (adj_small(h))
+        og::k_adj_lr<T2, NA, 2, 8><<<adj_lr_blocks(h), 512, 0, h->stream>>>(a);
       else
-        og::k_adj_lr<T2, NA, false><<<nwg, 256, 0, h->stream>>>(a);
+        og::k_adj_lr<T2, NA, 4, 4><<<adj_lr_blocks(h), 256, 0, h->stream>>>(a);
     }
   }
   if constexpr (NA <= 12) {
@@ -2724,9 +2728,10 @@ using B = ocean_gpu_batch;
 // Device tables of one group for one set of (in, out) vectors.
 struct Tables {
   void* args = nullptr;  // og::ActArgs<T2>[np]
-  int* off = nullptr;    // [4][np + 1] first workgroup of each problem: proj, fft, adj, matrix-core lr
+  int* off = nullptr;    // [5][np + 1] first workgroup of each problem: proj, fft, adj, matrix-core
+                         // adjoint of 64 and of 32 bands
   int np = 0;
-  int nblk[4] = {0, 0, 0, 0};
+  int nblk[5] = {0, 0, 0, 0, 0};
   size_t sm[3] = {0, 0, 0};
   int threads[3] = {256, kBlock, 512};
   int lmax = 8;
@@ -2756,7 +2761,7 @@ int build_tables(const B* b, const B::Group& g, const std::vector<const double2*
                  const std::vector<double2*>& out, const Tiles& t, Tables& tb) {
   const int np = (int)g.idx.size();
   std::vector<og::ActArgs<T2>> host((size_t)np);
-  std::vector<int> off((size_t)4 * (np + 1), 0);
+  std::vector<int> off((size_t)5 * (np + 1), 0);
   tb = Tables{};
   tb.np = np;
   tb.lmax = g.lmax;
@@ -2772,17 +2777,17 @@ int build_tables(const B* b, const B::Group& g, const std::vector<const double2*
     off[(np + 1) + q + 1] = off[(np + 1) + q] + ge.nblk_fft;
     off[2 * (np + 1) + q + 1] = off[2 * (np + 1) + q] + ge.nblk_adj;
     // many alphas on one spin: the matrix-core adjoint, as in xact_t
-    int nlr = 0;
+    int nlr[2] = {0, 0};
     if (adj_mf<T2, NA>(h, f, t)) {
-      nlr = ((h->nb + 63) / 64) * h->nk;
+      nlr[adj_small(h)] = adj_lr_blocks(h);
       off[2 * (np + 1) + q + 1] = off[2 * (np + 1) + q];
     }
-    off[3 * (np + 1) + q + 1] = off[3 * (np + 1) + q] + nlr;
+    for (int i = 0; i < 2; ++i) off[(3 + i) * (np + 1) + q + 1] = off[(3 + i) * (np + 1) + q] + nlr[i];
     tb.sm[0] = std::max(tb.sm[0], ge.sm_proj);
     tb.sm[1] = std::max(tb.sm[1], ge.sm_fft);
     tb.sm[2] = std::max(tb.sm[2], ge.sm_adj);
   }
-  for (int i = 0; i < 4; ++i) tb.nblk[i] = off[(size_t)i * (np + 1) + np];
+  for (int i = 0; i < 5; ++i) tb.nblk[i] = off[(size_t)i * (np + 1) + np];
   tb.threads[0] = t.proj;
   tb.threads[2] = t.adj;
   OG_CHECK(hipMalloc(&tb.args, sizeof(og::ActArgs<T2>) * (size_t)np));
@@ -2819,7 +2824,9 @@ int launch_tables(const Tables& tb, hipStream_t st, int stages) {
   if (stages & 4) {
     if constexpr (NA >= 6) {
       if (tb.nblk[3] > 0)
-        og::k_adj_lr_batch<T2, NA><<<tb.nblk[3], 256, 0, st>>>(A, tb.off + 3 * (np + 1), np);
+        og::k_adj_lr_batch<T2, NA, 4, 4><<<tb.nblk[3], 256, 0, st>>>(A, tb.off + 3 * (np + 1), np);
+      if (tb.nblk[4] > 0)
+        og::k_adj_lr_batch<T2, NA, 2, 8><<<tb.nblk[4], 512, 0, st>>>(A, tb.off + 4 * (np + 1), np);
     }
     if constexpr (NA <= 12) {
       if (tb.nblk[2] > 0) {

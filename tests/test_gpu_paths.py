@@ -130,6 +130,26 @@ def test_cube8_transform_every_strip_width(spec):
                     assert np.array_equal(o, outs[0])
 
 
+@pytest.mark.parametrize("nb,kmesh,x", [(1, (1, 1, 1), 1), (31, (2, 1, 2), 33), (33, (3, 1, 1), 47), (64, (2, 2, 1), 96),
+                                        (65, (8, 8, 2), 67), (7, (8, 8, 4), 17)])
+def test_l23_adjoint_tiles(nb, kmesh, x):
+    """Twelve alphas: the 32-band tiles of small grids and the 64-band ones of grids of 256
+    workgroups and more, bands and x points around their edges, odd FP32 rows (their last
+    pair ends past the row); 24 alphas as two right-hand sides."""
+    inp = synth.make_inputs(nb=nb, kmesh=kmesh, xmesh=(x, 1, 1), lc=1, seed=91, xi_eV=3.0)
+    P = to_problem(inp)
+    with core.OceanGPU.from_inputs(inp) as g, core.OceanGPU.from_inputs(inp, nrhs=2) as g2:
+        psi = [_rand(g.shape, 7 + i) for i in range(2)]
+        ref = [orc.xact(P, p) for p in psi]
+        for prec, tol in ((core.FP64, 1e-12), (core.MIXED, 1e-5)):
+            g.set_precision(prec)
+            g2.set_precision(prec)
+            assert relerr(g.xact(psi[0]), ref[0]) < tol
+            got = g2.xact(np.asfortranarray(np.concatenate(psi, axis=2)))
+            for i in range(2):
+                assert relerr(got[:, :, 12 * i:12 * i + 12], ref[i]) < tol
+
+
 @pytest.mark.parametrize("kmesh,lc,lmax", [((7, 6, 3), 0, 3), ((5, 3, 7), 1, 3), ((6, 5, 2), 1, 2), ((3, 7, 6), 0, 4)])
 def test_transform_odd_edges_every_strip_width(kmesh, lc, lmax):
     """Direct sums at 3, 5, 6 and 7 points in each position, padded (even k3) and unpadded
