@@ -101,6 +101,58 @@ __device__ __noinline__ void gm_finish(const GmFin F) {
   __syncthreads();
 }
 
+// A Haydock iteration fused into the action (OCEAN_hay_ab_twoterm, OCEAN2/OCEAN_haydock.f90:
+// 824-938).  The recursion's vectors stay as they are before their division by b: vector
+// psi_i is the stored one times inv(i - 1) = 1 / b(i - 1).  The transform's grid has one
+// more workgroup that finishes b(i - 1) from the partials of |h|^2; the adjoint's
+// epilogue scales H psi, subtracts b(i - 1) psi_(i-1) and writes the partials of <h|psi>;
+// k_hay2 (vec.hpp) takes a(i) from them, subtracts a(i) psi and writes the partials of
+// |h|^2.  As three passes over the vectors of their own after the action these steps
+// took 14.5 us of a 135 us iteration at 131 072 elements and 10.6 of 34 at 4 096.
+// Scalars of right-hand side q at s + q stride: a(0:niter), imag a, b, inv (n1 each), part1
+// [np1][2], part2 [kRedBlocks].  The iteration number is `it`, or *itp where one captured
+// iteration is replayed; the adjoint then copies it to itp[1] for k_hay2, which advances
+// itp[0].
+struct HayFuse {
+  double* s = nullptr;  // nullptr: no recursion
+  const double2* old = nullptr;
+  int* itp = nullptr;
+  int it = 0, n1 = 0, np1 = 0, stride = 0;
+};
+struct HayScal { double sc, so, mb; };  // of psi, of old, -b(i - 1)
+
+__device__ __forceinline__ int hay_it(const HayFuse& F) { return F.itp ? F.itp[0] : F.it; }
+__device__ __forceinline__ HayScal hay_scal(const HayFuse& F, int it, int q) {
+  if (F.s == nullptr) return {1.0, 0.0, 0.0};
+  const double* s = F.s + (size_t)q * F.stride + 2 * F.n1;
+  return {s[F.n1 + it - 1], s[F.n1 + max(it - 2, 0)], -s[it - 1]};
+}
+// h = r - b psi_old of one element, and its term of <h|psi>
+__device__ __forceinline__ double2 hay_elem(const HayScal& c, double2 pv, double2 ov, double2& r) {
+  r.x = fma(c.mb, ov.x * c.so, r.x);
+  r.y = fma(c.mb, ov.y * c.so, r.y);
+  return make_double2(fma(r.y, pv.y, r.x * pv.x), fma(-r.y, pv.x, r.x * pv.y));
+}
+// partial `idx` of right-hand side q: wave q of the workgroup sums n terms
+__device__ __forceinline__ void hay_part(const HayFuse& F, const double2* t, int n, int q, int idx) {
+  const int lane = threadIdx.x & 63;
+  double x = 0.0, y = 0.0;
+  for (int e = lane; e < n; e += 64) { x += t[e].x; y += t[e].y; }
+  x = wave_sum(x);
+  y = wave_sum(y);
+  double* p = F.s + (size_t)q * F.stride + 4 * F.n1 + 2 * idx;
+  if (lane == 0) { p[0] = x; p[1] = y; }
+}
+// b(j) = sqrt(|h|^2) and 1 / b(j) of every right-hand side (one workgroup)
+__device__ __forceinline__ void hay_fin(const HayFuse& F, int j, int R) {
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  for (int q = threadIdx.x >> 6; q < R; q += nw) {
+    double* s = F.s + (size_t)q * F.stride;
+    const double b = sqrt(wave_sum_parts(s + 4 * F.n1 + 2 * F.np1, kRedBlocks, 1, 0, lane));
+    if (lane == 0) { s[2 * F.n1 + j] = b; s[3 * F.n1 + j] = 1.0 / b; }
+  }
+}
+
 // Everything one problem's action kernels read: pointers into its device state,
 // its sizes and its launch geometry.  Passed by value to the single-problem
 // kernels; the batched kernels read an array of them, one per problem.
@@ -138,6 +190,8 @@ struct ActArgs {
                               // enqueued ahead)
   int axmy;                   // 1: the adjoint writes c psi - H psi instead of H psi
   double2 axmy_c;             // c = E + i gamma of a GMRES step (OCEAN_psi_axmy)
+  HayFuse hay;                // hay.s != nullptr: a Haydock iteration rides on the action
+  int nfin;                   // 1: the transform's grid finishes the previous iteration's b
   GmFin fin;                  // fin.c != nullptr: workgroup 0 of the projection first runs
                               // the previous GMRES residual step's finish
 };
@@ -869,6 +923,11 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
     mred_rows(A.apart, A.Kmat, A.hmult, A.nm, A.nj, A.na0 * A.P, A.mul, blk, reinterpret_cast<double2*>(smem));
     return;
   }
+  if (blk < nred + A.nfin) {
+    const int it = hay_it(A.hay);
+    if (it >= 2) hay_fin(A.hay, it - 1, A.na / A.na0);
+    return;
+  }
   const int nk = A.nk, ncol = A.ncol, na = A.na, G = A.G, ldphi = A.ldphi;
   const int K1 = A.K1, K2 = A.K2, K3 = A.K3;
   T2* phi = A.phi;
@@ -893,7 +952,7 @@ __device__ __forceinline__ void fft_body(const ActArgs<T2>& A, int blk) {
   // Workgroups are dispatched round-robin over the 8 XCDs; remap so that
   // consecutive column strips (which share 128-B lines) run on the same XCD and
   // therefore hit the same L2.
-  int b = blk - nred;
+  int b = blk - nred - A.nfin;
   if ((nfft & 7) == 0) b = (b & 7) * (nfft >> 3) + (b >> 3);
   const int c0 = b * G;
   const int gcnt = min(G, ncol - c0);
@@ -1113,7 +1172,7 @@ __device__ void mred_rows(const double2* __restrict__ apart, const double2* __re
 // One workgroup per k; threads (n, xs) with n fastest.  JR alphas per reduction
 // round through LDS (the reduction buffer reuses the phi' staging area).
 // ---------------------------------------------------------------------------
-template <typename T2, int NA>
+template <typename T2, int NA, bool HAY>
 __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int nb = A.nb, nk = A.nk, nx = A.nx, na = A.na, ns = A.ns, P = A.P;
@@ -1145,18 +1204,28 @@ __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
   const int nel = na * nb;
   const int na0 = A.na0;
   // epilogue operands of the first kEP elements owned by this thread
-  constexpr int kEP = 2;
-  double2 e_psi[kEP], e_en[kEP];
+  constexpr int kEP = HAY ? 1 : 2;  // (a recursion holds more per element)
+  const int it = HAY ? hay_it(A.hay) : 0;
+  HayScal hs0 = {1.0, 0.0, 0.0};
+  double2 e_psi[kEP], e_en[kEP], e_old[kEP];
   double e_m[kEP];
+  auto operands = [&]() {
 #pragma unroll
-  for (int i = 0; i < kEP; ++i) {
-    const int e = min(t + i * bd, nel - 1);
-    const int a = e / nb, nn = e - a * nb;
-    const size_t off = ((size_t)a * nk + k) * nb + nn;
-    e_psi[i] = psi[off];
-    e_en[i] = energy[off];
-    e_m[i] = allow[off];
-  }
+    for (int i = 0; i < kEP; ++i) {
+      const int e = min(t + i * bd, nel - 1);
+      const int a = e / nb, nn = e - a * nb;
+      const size_t off = ((size_t)a * nk + k) * nb + nn;
+      e_psi[i] = psi[off];
+      e_en[i] = energy[off];
+      e_m[i] = allow[off];
+    }
+  };
+  // Beside a recursion's own operands these cost registers: a second workgroup per CU was
+  // lost with all of them held through the stream (a batch of FP32 problems 92 -> 127
+  // us).  So the recursion's come behind it, in FP64 the others too (50.6 against 51.7 us
+  // at 512 k points and 64 bands; FP32 31.7 against 31.2).
+  constexpr bool kPre = !HAY || sizeof(T2) == 8;
+  if constexpr (kPre) operands();
 
   const int astep = (ns == 2) ? 2 : 1;
   const int acnt = (ns == 2) ? na / 2 : na;
@@ -1266,9 +1335,18 @@ __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
       }
     }
   }
+  if constexpr (HAY) {
+    if constexpr (!kPre) operands();
+    hs0 = hay_scal(A.hay, it, 0);
+#pragma unroll
+    for (int i = 0; i < kEP; ++i) {
+      const int e = min(t + i * bd, nel - 1), a = e / nb;
+      e_old[i] = A.hay.old[((size_t)a * nk + k) * nb + e - a * nb];
+    }
+  }
   __syncthreads();
   const bool back = (flags & F_BACK) != 0;
-  auto finish = [&](int e, double2 pv, double2 ev, double am) {
+  auto finish = [&](int e, double2 pv, double2 ev, double am, double2 ov) {
     const int a = e / nb, nn = e - a * nb;
     const size_t off = ((size_t)a * nk + k) * nb + nn;
     double2 inter = res[e];
@@ -1283,38 +1361,51 @@ __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
         cfma(inter, sab, psi[((size_t)(a0 + b) * nk + k) * nb + nn]);
       }
     }
+    HayScal hs = hs0;
+    if constexpr (HAY) {
+      if (a >= na0) hs = hay_scal(A.hay, it, a / na0);
+      pv.x *= hs.sc; pv.y *= hs.sc;
+      inter.x *= hs.sc; inter.y *= hs.sc;
+    }
     double2 r = inter;
     if (flags & F_E0) {
       if (back) ev.y = -ev.y;
       r.x = ev.x * pv.x - ev.y * pv.y + inter.x;
       r.y = ev.x * pv.y + ev.y * pv.x + inter.y;
     }
+    if constexpr (HAY) res[e] = hay_elem(hs, pv, ov, r);
     out[off] = axmy_epilogue(A, pv, r);
   };
 #pragma unroll
   for (int i = 0; i < kEP; ++i)
-    if (t + i * bd < nel) finish(t + i * bd, e_psi[i], e_en[i], e_m[i]);
+    if (t + i * bd < nel) finish(t + i * bd, e_psi[i], e_en[i], e_m[i], e_old[i]);
   for (int e = t + kEP * bd; e < nel; e += bd) {
     const int a = e / nb, nn = e - a * nb;
     const size_t off = ((size_t)a * nk + k) * nb + nn;
-    finish(e, psi[off], energy[off], allow[off]);
+    finish(e, psi[off], energy[off], allow[off], HAY ? A.hay.old[off] : make_double2(0.0, 0.0));
+  }
+  if constexpr (HAY) {
+    __syncthreads();
+    if ((t >> 6) < (bd >> 6))  // whole waves: at least four, as bd > 256
+      for (int q = t >> 6; q < na / na0; q += bd >> 6) hay_part(A.hay, res + q * na0 * nb, na0 * nb, q, k);
+    if (A.hay.itp && blk == 0 && t == 0) A.hay.itp[1] = it;
   }
 }
 
 // One problem: one workgroup per k.
-template <typename T2, int NA>
+template <typename T2, int NA, bool HAY>
 __global__ __launch_bounds__(512) void k_adj(const ActArgs<T2> A) {
   if (skipped(A)) return;
-  adj_body<T2, NA>(A, blockIdx.x);
+  adj_body<T2, NA, HAY>(A, blockIdx.x);
 }
 
-template <typename T2, int NA>
+template <typename T2, int NA, bool HAY>
 __global__ __launch_bounds__(512) void k_adj_batch(const ActArgs<T2>* __restrict__ As,
                                                    const int* __restrict__ off, int np) {
   const int p = find_problem(off, np, blockIdx.x);
   const ActArgs<T2> A = As[p];
   if (skipped(A)) return;
-  adj_body<T2, NA>(A, blockIdx.x - off[p]);
+  adj_body<T2, NA, HAY>(A, blockIdx.x - off[p]);
 }
 
 }  // namespace og

@@ -180,7 +180,7 @@ int mult_blocks(const H* h, int nw) {
 template <typename T2, int NA>
 int make_args(const H* h, const double2* in, double2* out, int flags, const Tiles& t, const T2* u,
               const T2* uT, T2* phi, const typename og::Scalar<T2>::T* W, og::ActArgs<T2>& a,
-              Geom<T2>& g, const BandSide* bs = nullptr) {
+              Geom<T2>& g, const BandSide* bs = nullptr, const og::HayFuse* hay = nullptr) {
   using T = typename og::Scalar<T2>::T;
   const int nb = h->nb, nk = h->nk, na = h->na, ns = h->ns;
   const int nx = bs ? bs->nx : h->nx;
@@ -238,7 +238,11 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   g.sm_fft = (6 * (size_t)g.lmax + og::tile_size(a.K1, a.K2, a.K3, G)) * sizeof(T2) + (size_t)xs * nk * sizeof(T);
   if (a.nred) g.sm_fft = std::max(g.sm_fft, og::mred_lds(h->na0 * h->P, kBlock / 64));
   if (g.sm_fft > h->lds_max || g.sm_proj > h->lds_max) return OCEAN_GPU_ERR_ARG;  // k mesh or bands too large
-  g.nblk_fft = a.nred + a.nfft;
+  if (hay) {
+    a.hay = *hay;
+    a.nfin = 1;
+  }
+  g.nblk_fft = a.nred + a.nfin + a.nfft;
   // adjoint: x-splits, phi' chunk and reduction rounds sharing one LDS area
   if (nb > t.adj) return OCEAN_GPU_ERR_ARG;
   const int XS = std::max(1, t.adj / nb);
@@ -279,6 +283,11 @@ bool adj_mf(const H* h, int flags, const Tiles& t) {
 bool adj_small(const H* h) { return ((h->nb + 63) / 64) * h->nk < h->ncu; }
 int adj_lr_blocks(const H* h) { return (adj_small(h) ? (h->nb + 31) / 32 : (h->nb + 63) / 64) * h->nk; }
 
+// Partials of <h|psi> that the adjoint of a Haydock iteration writes (where the tile has
+// the VALU form instead it writes the first nk, and the rest stay zero).
+int hay_parts(const H* h) { return h->ns == 1 && na_tmpl(h->na) == h->na && h->na >= 6 ? std::max(h->nk, adj_lr_blocks(h)) : h->nk; }
+size_t hay_scalars(const H* h, size_t n1) { return 4 * n1 + 2 * (size_t)hay_parts(h) + kRedBlocks; }
+
 // The device state of one precision form.
 template <typename T2> struct StateOf;
 template <> struct StateOf<double2> {
@@ -306,11 +315,11 @@ Tiles tiles_for(const H* h) {
 template <typename T2, int NA>
 int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* phi,
            const typename og::Scalar<T2>::T* W, hipEvent_t* ev, const int* skip, const double2* axmy,
-           const og::GmFin* fin) {
+           const og::GmFin* fin, const og::HayFuse* hay) {
   og::ActArgs<T2> a;
   Geom<T2> g;
   const Tiles tl = tiles_for<T2>(h);
-  OG_TRY((make_args<T2, NA>(h, in, out, flags, tl, u, uT, phi, W, a, g)));
+  OG_TRY((make_args<T2, NA>(h, in, out, flags, tl, u, uT, phi, W, a, g, nullptr, hay)));
   a.skip = skip;
   if (axmy) {
     a.axmy = 1;
@@ -337,9 +346,16 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
     }
     OG_CHECK(hipGetLastError());
     if (ev) OG_CHECK(hipEventRecord(ev[2], h->stream));
-  } else if (ev) {
-    OG_CHECK(hipEventRecord(ev[1], h->stream));
-    OG_CHECK(hipEventRecord(ev[2], h->stream));
+  } else {
+    // no transform to ride on
+    if (hay && hay->it >= 2) {
+      og::k_hay_fin<<<1, kBlock, 0, h->stream>>>(*hay, hay->it - 1, h->nrhs);
+      OG_CHECK(hipGetLastError());
+    }
+    if (ev) {
+      OG_CHECK(hipEventRecord(ev[1], h->stream));
+      OG_CHECK(hipEventRecord(ev[2], h->stream));
+    }
   }
   if ((flags & og::F_FG) && !(flags & og::F_LR)) {
     const int nm = mult_blocks(h, kBlock / 64);
@@ -366,8 +382,9 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
   }
   if constexpr (NA <= 12) {
     if (!mf) {
-      OG_TRY(lds_opt_in(og::k_adj<T2, NA>, g.sm_adj));
-      og::k_adj<T2, NA><<<g.nblk_adj, g.adj_threads, g.sm_adj, h->stream>>>(a);
+      const auto kernel = hay ? og::k_adj<T2, NA, true> : og::k_adj<T2, NA, false>;
+      OG_TRY(lds_opt_in(kernel, g.sm_adj));
+      kernel<<<g.nblk_adj, g.adj_threads, g.sm_adj, h->stream>>>(a);
     }
   }
   OG_CHECK(hipGetLastError());
@@ -388,16 +405,16 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
 // the x side (both obf products and the transform), adj = the adjoint.
 template <int NA>
 int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev, const int* skip,
-               const double2* axmy) {
+               const double2* axmy, const og::HayFuse* hay) {
   flags &= ~og::F_FG;
   og::ActArgs<double2> a, ab;
   Geom<double2> g, gb;
   const Tiles tl = tiles_for<double2>(h);
-  OG_TRY((make_args<double2, NA>(h, in, out, flags, tl, nullptr, nullptr, h->phi64, h->W64, a, g)));
+  OG_TRY((make_args<double2, NA>(h, in, out, flags, tl, nullptr, nullptr, h->phi64, h->W64, a, g, nullptr, hay)));
   a.phs = h->obf_phs;
   const BandSide bs{h->no, h->ldu_o, h->ldT_o, h->ldb};
   OG_TRY((make_args<double2, NA>(h, in, out, flags, tl, h->obf_u, h->obf_uT, h->obf_beta, nullptr, ab, gb,
-                                 &bs)));
+                                 &bs, hay)));
   a.skip = skip;
   ab.skip = skip;
   if (axmy) {
@@ -433,8 +450,9 @@ int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev,
     OG_CHECK(hipEventRecord(ev[2], h->stream));
     OG_CHECK(hipEventRecord(ev[3], h->stream));
   }
-  OG_TRY(lds_opt_in(og::k_adj<double2, NA>, gb.sm_adj));
-  og::k_adj<double2, NA><<<gb.nblk_adj, gb.adj_threads, gb.sm_adj, h->stream>>>(ab);
+  const auto kernel = hay ? og::k_adj<double2, NA, true> : og::k_adj<double2, NA, false>;
+  OG_TRY(lds_opt_in(kernel, gb.sm_adj));
+  kernel<<<gb.nblk_adj, gb.adj_threads, gb.sm_adj, h->stream>>>(ab);
   OG_CHECK(hipGetLastError());
   if (ev) OG_CHECK(hipEventRecord(ev[4], h->stream));
   return OCEAN_GPU_OK;
@@ -443,20 +461,21 @@ int xact_obf_t(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev,
 // skip (nullable): every kernel returns at once while *skip != 0; axmy (nullable):
 // out = c in - H in with c = *axmy, formed in the adjoint's epilogue.
 int xact_dev(H* h, const double2* in, double2* out, int flags, hipEvent_t* ev = nullptr,
-             const int* skip = nullptr, const double2* axmy = nullptr, const og::GmFin* fin = nullptr) {
+             const int* skip = nullptr, const double2* axmy = nullptr, const og::GmFin* fin = nullptr,
+             const og::HayFuse* hay = nullptr) {
   const int acnt = (h->ns == 2) ? h->na / 2 : h->na;
   const int NA = na_tmpl(acnt);
   const bool mixed = (h->precision == OCEAN_GPU_MIXED);
   if (h->obf_on && (flags & og::F_LR)) {
     if (mixed || h->ns != 1) return OCEAN_GPU_ERR_STATE;
-    if (NA == 4 && h->na == 4) return xact_obf_t<4>(h, in, out, flags, ev, skip, axmy);
-    if (NA == 12 && h->na == 12) return xact_obf_t<12>(h, in, out, flags, ev, skip, axmy);
+    if (NA == 4 && h->na == 4) return xact_obf_t<4>(h, in, out, flags, ev, skip, axmy, hay);
+    if (NA == 12 && h->na == 12) return xact_obf_t<12>(h, in, out, flags, ev, skip, axmy, hay);
     return OCEAN_GPU_ERR_ARG;
   }
 #define OG_DISPATCH(NAV)                                                              \
   if (NA == NAV)                                                                      \
-    return mixed ? xact_t<float2, NAV>(h, in, out, flags, h->u32, h->uT32, h->phi32, h->W32, ev, skip, axmy, fin) \
-                 : xact_t<double2, NAV>(h, in, out, flags, h->u64, h->uT64, h->phi64, h->W64, ev, skip, axmy, fin);
+    return mixed ? xact_t<float2, NAV>(h, in, out, flags, h->u32, h->uT32, h->phi32, h->W32, ev, skip, axmy, fin, hay) \
+                 : xact_t<double2, NAV>(h, in, out, flags, h->u64, h->uT64, h->phi64, h->W64, ev, skip, axmy, fin, hay);
   OG_DISPATCH(2)
   OG_DISPATCH(4)
   OG_DISPATCH(6)
@@ -1747,13 +1766,12 @@ int haydock_run(H* h, const double* psi0_re, const double* psi0_im, int niter, c
   const size_t nv = h->nvec();
   const size_t n1 = (size_t)niter + 1;
   constexpr int kConvBlocks = 64;
-  OG_TRY(ensure_scal(h, 3 * n1 + 3 * (size_t)kRedBlocks + 2 * n1 + 4 * (size_t)kConvBlocks));
+  const size_t ns = hay_scalars(h, n1);
+  OG_TRY(ensure_scal(h, ns + 2 * n1 + 4 * (size_t)kConvBlocks));
   double* da = h->scal;
   double* dai = da + n1;
   double* db = dai + n1;
-  double* part1 = db + n1;
-  double* part2 = part1 + 2 * kRedBlocks;
-  double* conv = part2 + kRedBlocks;      // [iter][relArea, maxDiff]
+  double* conv = da + ns;                 // [iter][relArea, maxDiff]
   double* cpart = conv + 2 * n1;
   double2 *v0 = nullptr, *v1 = nullptr, *v2 = nullptr;
   OG_TRY(dmalloc(&v0, nv));
@@ -1785,15 +1803,21 @@ int haydock_run(H* h, const double* psi0_re, const double* psi0_im, int niter, c
   };
   if (rc == 0) {
     og::k_fill<<<grid_for(nv), kBlock, 0, h->stream>>>(old, make_double2(0.0, 0.0), nv);
-    og::k_fill_d<<<grid_for(5 * n1), kBlock, 0, h->stream>>>(da, 0.0, 3 * n1);
+    og::k_fill_d<<<grid_for(ns), kBlock, 0, h->stream>>>(da, 0.0, ns);
+    og::k_fill_d<<<1, 64, 0, h->stream>>>(da + 3 * n1, 1.0, 1);  // psi_1 is normalised
     og::k_fill_d<<<grid_for(2 * n1), kBlock, 0, h->stream>>>(conv, 0.0, 2 * n1);
+    og::HayFuse hf;
+    hf.s = da;
+    hf.n1 = (int)n1;
+    hf.np1 = hay_parts(h);
     for (int it = 1; it <= niter && rc == 0 && !stop; ++it) {
-      rc = xact_dev(h, psi, hv, f);
+      hf.old = old;
+      hf.it = it;
+      rc = xact_dev(h, psi, hv, f, nullptr, nullptr, nullptr, nullptr, &hf);
       if (rc) break;
-      og::k_hay1<<<kRedBlocks, kBlock, 0, h->stream>>>(hv, old, psi, db + (it - 1), nv, part1);
-      og::k_hay2<<<kRedBlocks, kBlock, 0, h->stream>>>(hv, psi, part1, kRedBlocks, nv, da + (it - 1),
-                                                      dai + (it - 1), part2);
-      og::k_hay3<<<kRedBlocks, kBlock, 0, h->stream>>>(hv, part2, kRedBlocks, nv, db + it);
+      og::k_hay2<<<kRedBlocks, kBlock, 0, h->stream>>>(og::HayArgs{hf, hv, psi, nv});
+      // b(it) is finished by the next iteration's transform; now where it is needed now
+      if (it == niter || ex) og::k_hay_fin<<<1, kBlock, 0, h->stream>>>(hf, it, 1);
       if (ex && it > ex->spacing) {
         const int nb = std::min(kConvBlocks, std::max(1, (ex->ne + kBlock - 1) / kBlock));
         og::k_conv_part<<<nb, kBlock, 0, h->stream>>>(da, db, dai, it, it - ex->spacing, ex->kpref, ex->gam,
@@ -1867,46 +1891,35 @@ int ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const do
   const int R = h->nrhs;
   const size_t nv = h->nvec(), nv0 = h->nvec0();
   const size_t n1 = (size_t)niter + 1;
-  const size_t nscal = 3 * n1 + 3 * (size_t)kRedBlocks;  // a, ai, b, part1 (2 kRedBlocks), part2
+  const size_t nscal = hay_scalars(h, n1);
   double2* V[3] = {nullptr, nullptr, nullptr};
   double* S = nullptr;
-  int* dcount = nullptr;  // [0] iteration number, [1] its copy for the third step
-  og::HayArgs* dhay[3] = {nullptr, nullptr, nullptr};
   int rc = OCEAN_GPU_OK;
   for (int i = 0; i < 3 && rc == 0; ++i) rc = dmalloc(&V[i], nv);
   if (rc == 0) rc = dmalloc(&S, (size_t)R * nscal);
-  if (rc == 0) rc = dmalloc(&dcount, (size_t)2);
-  for (int i = 0; i < 3 && rc == 0; ++i) rc = dmalloc(&dhay[i], (size_t)R);
   if (rc == 0) rc = put_planes(h, psi0_re, psi0_im, V[0], nv);
   // rotation r of an iteration: (psi, old, hv) = (V0, V1, V2), (V2, V0, V1), (V1, V2, V0)
   const int rot[3][3] = {{0, 1, 2}, {2, 0, 1}, {1, 2, 0}};
-  for (int r = 0; r < 3 && rc == 0; ++r) {
-    std::vector<og::HayArgs> ha((size_t)R);
-    for (int q = 0; q < R; ++q) {
-      double* sq = S + (size_t)q * nscal;
-      ha[q] = og::HayArgs{V[rot[r][2]] + q * nv0, V[rot[r][1]] + q * nv0, V[rot[r][0]] + q * nv0,
-                          sq + 3 * n1, sq + 3 * n1 + 2 * kRedBlocks, sq, sq + n1, sq + 2 * n1, nv0};
-    }
-    if (hipMemcpy(dhay[r], ha.data(), sizeof(og::HayArgs) * R, hipMemcpyHostToDevice) != hipSuccess)
-      rc = OCEAN_GPU_ERR_HIP;
-  }
-  // psi_old = 0, coefficients 0 (b_0 = 0), iteration 1
+  og::HayFuse hf;
+  hf.s = S;
+  hf.n1 = (int)n1;
+  hf.np1 = hay_parts(h);
+  hf.stride = (int)nscal;
+  // psi_old = 0, coefficients 0 (b_0 = 0), psi_1 normalised
   if (rc == 0) {
     og::k_fill<<<grid_for(nv), kBlock, 0, h->stream>>>(V[1], make_double2(0.0, 0.0), nv);
     og::k_fill_d<<<grid_for((size_t)R * nscal), kBlock, 0, h->stream>>>(S, 0.0, (size_t)R * nscal);
-    const int init[2] = {1, 0};
-    if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(dcount, init, sizeof(init), hipMemcpyHostToDevice, h->stream) != hipSuccess ||
-        hipStreamSynchronize(h->stream) != hipSuccess)
-      rc = OCEAN_GPU_ERR_HIP;
+    for (int q = 0; q < R; ++q) og::k_fill_d<<<1, 64, 0, h->stream>>>(S + q * nscal + 3 * n1, 1.0, 1);
+    if (hipGetLastError() != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
   }
   for (int it = 1; it <= niter && rc == 0; ++it) {
     const int r = (it - 1) % 3;
-    rc = xact_dev(h, V[rot[r][0]], V[rot[r][2]], f);
+    hf.old = V[rot[r][1]];
+    hf.it = it;
+    rc = xact_dev(h, V[rot[r][0]], V[rot[r][2]], f, nullptr, nullptr, nullptr, nullptr, &hf);
     if (rc) break;
-    og::k_hay1_batch<<<R * kRedBlocks, kBlock, 0, h->stream>>>(dhay[r], dcount);
-    og::k_hay2_batch<<<R * kRedBlocks, kBlock, 0, h->stream>>>(dhay[r], dcount);
-    og::k_hay3_batch<<<R * kRedBlocks, kBlock, 0, h->stream>>>(dhay[r], dcount);
+    og::k_hay2<<<R * kRedBlocks, kBlock, 0, h->stream>>>(og::HayArgs{hf, V[rot[r][2]], V[rot[r][0]], nv0});
+    if (it == niter) og::k_hay_fin<<<1, kBlock, 0, h->stream>>>(hf, it, R);
     if (hipGetLastError() != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
   }
   if (rc == 0 && hipStreamSynchronize(h->stream) != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
@@ -1930,9 +1943,7 @@ int ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const do
     if (niter_done) niter_done[q] = done;
   }
   for (auto& v : V) dfree(v);
-  for (auto& d : dhay) dfree(d);
   dfree(S);
-  dfree(dcount);
   return rc ? rc : rc_nan;
 }
 
@@ -2717,7 +2728,7 @@ struct ocean_gpu_batch {
   std::vector<H*> hs;
   std::vector<Group> groups;
   hipStream_t stream = nullptr;
-  int* dcount = nullptr;  // [0] Haydock iteration number, [1] its copy for the third step
+  int* dcount = nullptr;  // [0] Haydock iteration number, [1] its copy for k_hay2
   double t_last = 0.0;    // ms per batched action (all problems) of the last timed call
 };
 
@@ -2735,6 +2746,7 @@ struct Tables {
   size_t sm[3] = {0, 0, 0};
   int threads[3] = {256, kBlock, 512};
   int lmax = 8;
+  bool hay = false;      // a Haydock iteration rides on the actions
   void release() {
     if (args) (void)hipFree(args);
     if (off) (void)hipFree(off);
@@ -2758,13 +2770,14 @@ int group_call(const B::Group& g, F&& f) {
 
 template <typename T2, int NA>
 int build_tables(const B* b, const B::Group& g, const std::vector<const double2*>& in,
-                 const std::vector<double2*>& out, const Tiles& t, Tables& tb) {
+                 const std::vector<double2*>& out, const Tiles& t, Tables& tb, const og::HayArgs* hay) {
   const int np = (int)g.idx.size();
   std::vector<og::ActArgs<T2>> host((size_t)np);
   std::vector<int> off((size_t)5 * (np + 1), 0);
   tb = Tables{};
   tb.np = np;
   tb.lmax = g.lmax;
+  tb.hay = hay != nullptr;
   for (int q = 0; q < np; ++q) {
     const H* h = b->hs[g.idx[q]];
     const int f = flags_of(h, 0, nullptr);
@@ -2772,7 +2785,8 @@ int build_tables(const B* b, const B::Group& g, const std::vector<const double2*
     OG_TRY(check_ready(h, f));
     Geom<T2> ge;
     OG_TRY((make_args<T2, NA>(h, in[q], out[q], f, t, StateOf<T2>::u(h), StateOf<T2>::uT(h),
-                              StateOf<T2>::phi(h), StateOf<T2>::W(h), host[q], ge)));
+                              StateOf<T2>::phi(h), StateOf<T2>::W(h), host[q], ge, nullptr,
+                              hay ? &hay[g.idx[q]].f : nullptr)));
     off[q + 1] = off[q] + ge.nblk_proj;
     off[(np + 1) + q + 1] = off[(np + 1) + q] + ge.nblk_fft;
     off[2 * (np + 1) + q + 1] = off[2 * (np + 1) + q] + ge.nblk_adj;
@@ -2830,8 +2844,9 @@ int launch_tables(const Tables& tb, hipStream_t st, int stages) {
     }
     if constexpr (NA <= 12) {
       if (tb.nblk[2] > 0) {
-        OG_TRY(lds_opt_in(og::k_adj_batch<T2, NA>, tb.sm[2]));
-        og::k_adj_batch<T2, NA><<<tb.nblk[2], tb.threads[2], tb.sm[2], st>>>(A, tb.off + 2 * (np + 1), np);
+        const auto kernel = tb.hay ? og::k_adj_batch<T2, NA, true> : og::k_adj_batch<T2, NA, false>;
+        OG_TRY(lds_opt_in(kernel, tb.sm[2]));
+        kernel<<<tb.nblk[2], tb.threads[2], tb.sm[2], st>>>(A, tb.off + 2 * (np + 1), np);
       }
     } else if (tb.nblk[2] > 0) {
       return OCEAN_GPU_ERR_UNSUPPORTED;  // 24 alphas: the matrix-core adjoint only
@@ -2842,9 +2857,9 @@ int launch_tables(const Tables& tb, hipStream_t st, int stages) {
 }
 
 int group_build(const B* b, const B::Group& g, const std::vector<const double2*>& in,
-                const std::vector<double2*>& out, const Tiles& t, Tables& tb) {
+                const std::vector<double2*>& out, const Tiles& t, Tables& tb, const og::HayArgs* hay = nullptr) {
   return group_call(g, [&](auto na, auto t2) {
-    return build_tables<decltype(t2), decltype(na)::value>(b, g, in, out, t, tb);
+    return build_tables<decltype(t2), decltype(na)::value>(b, g, in, out, t, tb, hay);
   });
 }
 
@@ -3129,7 +3144,6 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
   for (H* h : b->hs)
     if (h->nrhs != 1) return OCEAN_GPU_ERR_UNSUPPORTED;
   const size_t n1 = (size_t)niter + 1;
-  const size_t nscal = 3 * n1 + 3 * (size_t)kRedBlocks;
   std::vector<double2*> V((size_t)3 * n, nullptr);
   std::vector<double*> Sd((size_t)n, nullptr);
   int rc = OCEAN_GPU_OK;
@@ -3137,7 +3151,7 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
     H* h = b->hs[q];
     if (!psi_re[q] || !psi_im[q] || !real_a[q] || !real_b[q]) rc = OCEAN_GPU_ERR_ARG;
     for (int i = 0; i < 3 && rc == 0; ++i) rc = dmalloc(&V[(size_t)3 * q + i], h->nvec());
-    if (rc == 0) rc = dmalloc(&Sd[q], nscal);
+    if (rc == 0) rc = dmalloc(&Sd[q], hay_scalars(h, n1));
     if (rc == 0) rc = put_planes(h, psi_re[q], psi_im[q], V[(size_t)3 * q], h->nvec());
   }
   // rotation r of an iteration: (psi, old, hv) = (V0, V1, V2), (V2, V0, V1), (V1, V2, V0)
@@ -3154,15 +3168,19 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
       double2* hv = V[(size_t)3 * q + rot[r][2]];
       in_all[q] = psi;
       out_all[q] = hv;
-      double* s = Sd[q];
-      ha[q] = og::HayArgs{hv, old, psi, s + 3 * n1, s + 3 * n1 + 2 * kRedBlocks, s, s + n1, s + 2 * n1,
-                          b->hs[q]->nvec()};
+      og::HayFuse hf;
+      hf.s = Sd[q];
+      hf.old = old;
+      hf.itp = b->dcount;
+      hf.n1 = (int)n1;
+      hf.np1 = hay_parts(b->hs[q]);
+      ha[q] = og::HayArgs{hf, hv, psi, b->hs[q]->nvec()};
     }
     for (size_t gi = 0; gi < b->groups.size() && rc == 0; ++gi) {
       std::vector<const double2*> in;
       std::vector<double2*> out;
       group_vectors(b->groups[gi], in_all, out_all, in, out);
-      rc = group_build(b, b->groups[gi], in, out, b->groups[gi].tiles, tabs[r][gi]);
+      rc = group_build(b, b->groups[gi], in, out, b->groups[gi].tiles, tabs[r][gi], ha.data());
     }
     if (rc == 0) rc = dmalloc(&dhay[r], (size_t)n);
     if (rc == 0 && hipMemcpy(dhay[r], ha.data(), sizeof(og::HayArgs) * n, hipMemcpyHostToDevice) != hipSuccess)
@@ -3173,7 +3191,9 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
     for (int q = 0; q < n; ++q) {
       og::k_fill<<<grid_for(b->hs[q]->nvec()), kBlock, 0, b->stream>>>(V[(size_t)3 * q + 1], make_double2(0.0, 0.0),
                                                                        b->hs[q]->nvec());
-      og::k_fill_d<<<grid_for(3 * n1), kBlock, 0, b->stream>>>(Sd[q], 0.0, 3 * n1);
+      const size_t nscal = hay_scalars(b->hs[q], n1);
+      og::k_fill_d<<<grid_for(nscal), kBlock, 0, b->stream>>>(Sd[q], 0.0, nscal);
+      og::k_fill_d<<<1, 64, 0, b->stream>>>(Sd[q] + 3 * n1, 1.0, 1);  // psi_1 is normalised
     }
     const int init[2] = {1, 0};
     if (hipGetLastError() != hipSuccess ||
@@ -3183,9 +3203,7 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
   }
   auto enqueue_iter = [&](int r) -> int {
     for (size_t gi = 0; gi < b->groups.size(); ++gi) OG_TRY(group_launch(b->groups[gi], tabs[r][gi], b->stream, 7));
-    og::k_hay1_batch<<<n * kRedBlocks, kBlock, 0, b->stream>>>(dhay[r], b->dcount);
     og::k_hay2_batch<<<n * kRedBlocks, kBlock, 0, b->stream>>>(dhay[r], b->dcount);
-    og::k_hay3_batch<<<n * kRedBlocks, kBlock, 0, b->stream>>>(dhay[r], b->dcount);
     OG_CHECK(hipGetLastError());
     return OCEAN_GPU_OK;
   };
@@ -3208,6 +3226,10 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
   for (int c = 0; c < cycles && rc == 0; ++c)
     if (hipGraphLaunch(exec, b->stream) != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
   for (int r = 0; r < rem && rc == 0; ++r) rc = enqueue_iter(r);
+  if (rc == 0) {
+    og::k_hay_fin_batch<<<n, kBlock, 0, b->stream>>>(dhay[0], niter);  // the last b
+    if (hipGetLastError() != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
+  }
   if (rc == 0 && (hipEventRecord(e1, b->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess))
     rc = OCEAN_GPU_ERR_HIP;
   if (rc == 0) {

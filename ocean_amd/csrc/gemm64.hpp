@@ -120,7 +120,9 @@ __device__ __forceinline__ void adj_lr_body(const ActArgs<T2>& A, int bx, int k)
   constexpr int AS = 64 * W / BN, APW = (NA + AS - 1) / AS;
   const int nl = threadIdx.x % BN, n = n0 + nl, nn = min(n, nb - 1);
   const int a0 = BN == 64 ? w : (int)threadIdx.x / BN;
-  double2 pv[APW], ev[APW];
+  const bool hay = A.hay.s != nullptr;
+  const int it = hay_it(A.hay);
+  double2 pv[APW], ev[APW], ov[APW];
   double am[APW];
 #pragma unroll
   for (int j = 0; j < APW; ++j) {
@@ -129,6 +131,7 @@ __device__ __forceinline__ void adj_lr_body(const ActArgs<T2>& A, int bx, int k)
     pv[j] = A.psi[off];
     ev[j] = A.energy[off];
     am[j] = A.allow[off];
+    ov[j] = hay ? A.hay.old[off] : make_double2(0.0, 0.0);
   }
   V acc[NT][MT];
 #pragma unroll
@@ -267,18 +270,22 @@ __device__ __forceinline__ void adj_lr_body(const ActArgs<T2>& A, int bx, int k)
     }
   }
   if (so) __syncthreads();
-  if (n >= nb) return;
+  double2 dt[APW];
 #pragma unroll
   for (int j = 0; j < APW; ++j) {
     const int a = a0 + AS * j;
-    if (a >= NA) break;
+    dt[j] = make_double2(0.0, 0.0);
+    if (a >= NA || n >= nb) continue;
     double2 inter = res[j];
     inter.x *= am[j];
     inter.y *= am[j];
+    const int ar = a % na0, ab = a - ar;
     if (so) {
-      const int ar = a % na0, ab = a - ar;
       for (int b = 0; b < na0; ++b) cfma(inter, Ss[ar * na0 + b], Ps[(ab + b) * BN + nl]);
     }
+    const HayScal hs = hay_scal(A.hay, it, a / na0);
+    pv[j].x *= hs.sc; pv[j].y *= hs.sc;
+    inter.x *= hs.sc; inter.y *= hs.sc;
     double2 r = inter;
     if (flags & F_E0) {
       double2 e = ev[j];
@@ -286,7 +293,18 @@ __device__ __forceinline__ void adj_lr_body(const ActArgs<T2>& A, int bx, int k)
       r.x = e.x * pv[j].x - e.y * pv[j].y + inter.x;
       r.y = e.x * pv[j].y + e.y * pv[j].x + inter.y;
     }
+    if (hay) dt[j] = hay_elem(hs, pv[j], ov[j], r);
     A.out[((size_t)a * nk + k) * nb + n] = axmy_epilogue(A, pv[j], r);
+  }
+  if (hay) {
+    __syncthreads();  // psi and S of the spin-orbit term have been read
+#pragma unroll
+    for (int j = 0; j < APW; ++j)
+      if (a0 + AS * j < NA) Ps[(a0 + AS * j) * BN + nl] = dt[j];
+    __syncthreads();
+    const int nbb = (nb + BN - 1) / BN;
+    for (int q = w; q < NA / na0; q += W) hay_part(A.hay, Ps + q * na0 * BN, na0 * BN, q, k * nbb + bx);
+    if (A.hay.itp && k == 0 && bx == 0 && threadIdx.x == 0) A.hay.itp[1] = it;
   }
 }
 

@@ -4,6 +4,7 @@
 // Reductions are deterministic: a fixed grid of kRedBlocks workgroups writes
 // partials, and every consumer sums them in the same order.
 #pragma once
+#include "action.hpp"
 #include "common.hpp"
 
 namespace og {
@@ -113,175 +114,83 @@ __global__ void k_fill_d(double* __restrict__ dst, double v, size_t n) {
 }
 
 // ---------------------------------------------------------------------------
-// Haydock two-term step (OCEAN_hay_ab_twoterm, OCEAN2/OCEAN_haydock.f90:824-938)
-// split into three streaming passes with device-resident scalars:
-//   hay1: h -= b(i-1) old ; partial <h|psi>
-//   hay2: a(i-1) = Re<h|psi> ; h -= a(i-1) psi ; partial <h|h>
-//   hay3: b(i) = sqrt(<h|h>) ; h *= 1/b(i)
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_hay1(double2* __restrict__ h, const double2* __restrict__ old,
-                                                  const double2* __restrict__ psi,
-                                                  const double* __restrict__ bprev, size_t n,
-                                                  double* __restrict__ part) {
-  __shared__ double lds[8 * 2];
-  const double mb = -bprev[0];
-  double v[2] = {0.0, 0.0};
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    double2 a = h[i];
-    const double2 o = old[i];
-    a.x += mb * o.x; a.y += mb * o.y;
-    h[i] = a;
-    const double2 b = psi[i];
-    v[0] = fma(a.x, b.x, v[0]); v[0] = fma(a.y, b.y, v[0]);
-    v[1] = fma(a.x, b.y, v[1]); v[1] = fma(-a.y, b.x, v[1]);
-  }
-  block_sum<2>(v, lds);
-  if (threadIdx.x == 0) { part[2 * blockIdx.x] = v[0]; part[2 * blockIdx.x + 1] = v[1]; }
-}
-
-__global__ __launch_bounds__(kBlock) void k_hay2(double2* __restrict__ h, const double2* __restrict__ psi,
-                                                  const double* __restrict__ part1, int nblk, size_t n,
-                                                  double* __restrict__ a_out, double* __restrict__ ai_out,
-                                                  double* __restrict__ part2) {
-  __shared__ double lds[8];
-  __shared__ double s_a;
-  if (threadIdx.x < 64) {
-    const double ar = wave_sum_parts(part1, nblk, 2, 0, threadIdx.x);
-    const double ai = wave_sum_parts(part1, nblk, 2, 1, threadIdx.x);
-    if (threadIdx.x == 0) {
-      s_a = ar;
-      if (blockIdx.x == 0) { a_out[0] = ar; ai_out[0] = ai; }
-    }
-  }
-  __syncthreads();
-  const double ma = -s_a;
-  double v[1] = {0.0};
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    double2 a = h[i];
-    const double2 p = psi[i];
-    a.x += ma * p.x; a.y += ma * p.y;
-    h[i] = a;
-    v[0] = fma(a.x, a.x, v[0]); v[0] = fma(a.y, a.y, v[0]);
-  }
-  block_sum<1>(v, lds);
-  if (threadIdx.x == 0) part2[blockIdx.x] = v[0];
-}
-
-__global__ __launch_bounds__(kBlock) void k_hay3(double2* __restrict__ h, const double* __restrict__ part2,
-                                                  int nblk, size_t n, double* __restrict__ b_out) {
-  __shared__ double s_inv;
-  if (threadIdx.x < 64) {
-    const double b = sqrt(wave_sum_parts(part2, nblk, 1, 0, threadIdx.x));
-    if (threadIdx.x == 0) {
-      s_inv = 1.0 / b;
-      if (blockIdx.x == 0) b_out[0] = b;
-    }
-  }
-  __syncthreads();
-  const double inv = s_inv;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    double2 a = h[i];
-    a.x *= inv; a.y *= inv;
-    h[i] = a;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same three passes for many independent recursions in one launch each.
-// Every problem gets kRedBlocks workgroups and the same partition as the
-// single-problem kernels, so a batched recursion reproduces each problem's
-// stand-alone coefficients bit for bit.  The iteration number lives on the
-// device so that one captured iteration replays unchanged: k_hay1_batch and
-// k_hay2_batch read it from itp[0]; the first workgroup of k_hay2_batch copies it to
-// itp[1], which k_hay3_batch reads while its first workgroup advances itp[0] (no
-// workgroup of k_hay3_batch reads itp[0], and the next k_hay1_batch runs after it).
+// The Haydock two-term step's own pass, the rest of which rides on the action (HayFuse):
+//   a(i) = Re<h|psi> from the adjoint's partials; h -= a(i) psi; partials of |h|^2
+// h and psi are the stored vectors, n elements per right-hand side; the workgroup lb of
+// kRedBlocks always takes the same elements.  The first elements are in flight while
+// the partials are summed.
 // ---------------------------------------------------------------------------
 struct HayArgs {
-  double2* h;            // H psi on entry, psi_{i+1} on exit
-  const double2* old;    // psi_{i-1}
-  const double2* psi;    // psi_i
-  double* part1;         // [2 kRedBlocks]
-  double* part2;         // [kRedBlocks]
-  double* a;             // real_a(0:niter)
-  double* ai;            // imag_a(0:niter)
-  double* b;             // real_b(0:niter)
+  HayFuse f;
+  double2* h;
+  const double2* psi;
   size_t n;
 };
 
-__global__ __launch_bounds__(kBlock) void k_hay1_batch(const HayArgs* __restrict__ As, const int* __restrict__ itp) {
+__device__ __forceinline__ void hay2_body(const HayArgs& A, int q, int lb, int it) {
+  constexpr int U = 2;
   __shared__ double lds[8 * 2];
-  const HayArgs A = As[blockIdx.x / kRedBlocks];
-  const int lb = blockIdx.x % kRedBlocks;
-  const int it = *itp;
-  const double mb = -A.b[it - 1];
-  double v[2] = {0.0, 0.0};
-  for (size_t i = (size_t)lb * blockDim.x + threadIdx.x; i < A.n; i += (size_t)kRedBlocks * blockDim.x) {
-    double2 a = A.h[i];
-    const double2 o = A.old[i];
-    a.x += mb * o.x; a.y += mb * o.y;
-    A.h[i] = a;
-    const double2 b = A.psi[i];
-    v[0] = fma(a.x, b.x, v[0]); v[0] = fma(a.y, b.y, v[0]);
-    v[1] = fma(a.x, b.y, v[1]); v[1] = fma(-a.y, b.x, v[1]);
-  }
-  block_sum<2>(v, lds);
-  if (threadIdx.x == 0) { A.part1[2 * lb] = v[0]; A.part1[2 * lb + 1] = v[1]; }
-}
-
-__global__ __launch_bounds__(kBlock) void k_hay2_batch(const HayArgs* __restrict__ As, int* __restrict__ itp) {
-  __shared__ double lds[8];
   __shared__ double s_a;
-  const HayArgs A = As[blockIdx.x / kRedBlocks];
-  const int lb = blockIdx.x % kRedBlocks;
-  const int it = itp[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) itp[1] = it;
-  if (threadIdx.x < 64) {
-    const double ar = wave_sum_parts(A.part1, kRedBlocks, 2, 0, threadIdx.x);
-    const double ai = wave_sum_parts(A.part1, kRedBlocks, 2, 1, threadIdx.x);
-    if (threadIdx.x == 0) {
-      s_a = ar;
-      if (lb == 0) { A.a[it - 1] = ar; A.ai[it - 1] = ai; }
-    }
+  double* s = A.f.s + (size_t)q * A.f.stride;
+  const int n1 = A.f.n1, np1 = A.f.np1;
+  const double* part1 = s + 4 * n1;
+  double* part2 = s + 4 * n1 + 2 * np1;
+  double2* h = A.h + (size_t)q * A.n;
+  const double2* psi = A.psi + (size_t)q * A.n;
+  const size_t n = A.n, st = (size_t)kRedBlocks * blockDim.x;
+  size_t i = (size_t)lb * blockDim.x + threadIdx.x;
+  double2 hv[U], pv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const size_t e = min(i + u * st, n - 1);
+    hv[u] = h[e];
+    pv[u] = psi[e];
+  }
+  const double sc = s[3 * n1 + it - 1];
+  double p[2] = {0.0, 0.0};
+  for (int m = threadIdx.x; m < np1; m += blockDim.x) { p[0] += part1[2 * m]; p[1] += part1[2 * m + 1]; }
+  block_sum<2>(p, lds);
+  if (threadIdx.x == 0) {
+    s_a = p[0];
+    if (lb == 0) { s[it - 1] = p[0]; s[n1 + it - 1] = p[1]; }
   }
   __syncthreads();
   const double ma = -s_a;
   double v[1] = {0.0};
-  for (size_t i = (size_t)lb * blockDim.x + threadIdx.x; i < A.n; i += (size_t)kRedBlocks * blockDim.x) {
-    double2 a = A.h[i];
-    const double2 p = A.psi[i];
-    a.x += ma * p.x; a.y += ma * p.y;
-    A.h[i] = a;
-    v[0] = fma(a.x, a.x, v[0]); v[0] = fma(a.y, a.y, v[0]);
-  }
-  block_sum<1>(v, lds);
-  if (threadIdx.x == 0) A.part2[lb] = v[0];
-}
-
-__global__ __launch_bounds__(kBlock) void k_hay3_batch(const HayArgs* __restrict__ As, int* __restrict__ itp) {
-  __shared__ double s_inv;
-  const HayArgs A = As[blockIdx.x / kRedBlocks];
-  const int lb = blockIdx.x % kRedBlocks;
-  const int it = itp[1];
-  if (blockIdx.x == 0 && threadIdx.x == 0) itp[0] = it + 1;
-  if (threadIdx.x < 64) {
-    const double b = sqrt(wave_sum_parts(A.part2, kRedBlocks, 1, 0, threadIdx.x));
-    if (threadIdx.x == 0) {
-      s_inv = 1.0 / b;
-      if (lb == 0) A.b[it] = b;
+  for (; i < n; i += U * st) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t e = i + u * st;
+      if (e < n) {
+        const double2 a = make_double2(fma(ma, pv[u].x * sc, hv[u].x), fma(ma, pv[u].y * sc, hv[u].y));
+        h[e] = a;
+        v[0] = fma(a.x, a.x, v[0]); v[0] = fma(a.y, a.y, v[0]);
+      }
+      const size_t en = min(e + U * st, n - 1);
+      hv[u] = h[en];
+      pv[u] = psi[en];
     }
   }
-  __syncthreads();
-  const double inv = s_inv;
-  for (size_t i = (size_t)lb * blockDim.x + threadIdx.x; i < A.n; i += (size_t)kRedBlocks * blockDim.x) {
-    double2 a = A.h[i];
-    a.x *= inv; a.y *= inv;
-    A.h[i] = a;
-  }
+  block_sum<1>(v, lds);
+  if (threadIdx.x == 0) part2[lb] = v[0];
 }
 
+// one problem, all its right-hand sides
+__global__ __launch_bounds__(kBlock) void k_hay2(const HayArgs A) {
+  hay2_body(A, blockIdx.x / kRedBlocks, blockIdx.x % kRedBlocks, A.f.it);
+}
+__global__ __launch_bounds__(kBlock) void k_hay_fin(const HayFuse F, int j, int R) { hay_fin(F, j, R); }
+
+// Many problems of one right-hand side each, with the same partition as on their own, so a
+// batched recursion reproduces each problem's stand-alone coefficients bit for bit.
+__global__ __launch_bounds__(kBlock) void k_hay2_batch(const HayArgs* __restrict__ As, int* __restrict__ itp) {
+  const int it = itp[1];
+  if (blockIdx.x == 0 && threadIdx.x == 0) itp[0] = it + 1;
+  hay2_body(As[blockIdx.x / kRedBlocks], 0, blockIdx.x % kRedBlocks, it);
+}
+__global__ __launch_bounds__(kBlock) void k_hay_fin_batch(const HayArgs* __restrict__ As, int j) {
+  hay_fin(As[blockIdx.x].f, j, 1);
+}
 
 // ---------------------------------------------------------------------------
 // Continued fraction with the square-root terminator (write_core,
