@@ -218,6 +218,11 @@ int  ocean_gpu_profile_xact(ocean_gpu_handle* h, int32_t in, int32_t out, int32_
 int  ocean_gpu_haydock(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im,
                        int32_t niter, double* real_a, double* real_b, double* imag_a,
                        int32_t* niter_done);
+/* ocean_gpu_haydock with psi0 interleaved, (re, im) per element (as
+ * ocean_gpu_haydock_multi_z and ocean_gpu_batch_haydock_z take theirs): a program that
+ * holds complex vectors need not split them into planes. */
+int  ocean_gpu_haydock_z(ocean_gpu_handle* h, const double* psi0, int32_t niter, double* real_a,
+                         double* real_b, double* imag_a, int32_t* niter_done);
 
 /* The same recursion with the reference's early exit (sys%earlyExit,
  * OCEAN2/OCEAN_haydock.f90:272-291): after each iteration past `spacing`, relArea
@@ -241,6 +246,8 @@ int  ocean_gpu_haydock_early(ocean_gpu_handle* h, const double* psi0_re, const d
 int  ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im,
                              int32_t niter, double* real_a, double* real_b, double* imag_a,
                              int32_t* niter_done);
+int  ocean_gpu_haydock_multi_z(ocean_gpu_handle* h, const double* psi0, int32_t niter, double* real_a,
+                               double* real_b, double* imag_a, int32_t* niter_done);
 
 /* Non-Hermitian (bi-Lanczos) Haydock recursion: the reference's complex_haydock
  * branch, OCEAN_haydock_nonHerm_do (OCEAN2/OCEAN_haydock.f90:53-160) with
@@ -347,6 +354,9 @@ int  ocean_gpu_batch_last_ms(ocean_gpu_batch* b, double* ms);
 int  ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, const double* const* psi_im,
                              int32_t niter, double* const* real_a, double* const* real_b,
                              double* const* imag_a, int32_t* niter_done);
+int  ocean_gpu_batch_haydock_z(ocean_gpu_batch* b, const double* const* psi0, int32_t niter,
+                               double* const* real_a, double* const* real_b, double* const* imag_a,
+                               int32_t* niter_done);
 
 /* GMRES of all problems at once (as ocean_gpu_gmres per problem; energies, starting
  * vectors and kpref per problem, the solver settings shared): each problem's

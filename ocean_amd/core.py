@@ -86,6 +86,10 @@ _SIGS = {
     "ocean_gpu_xact_vec_repeat": (C.c_int, [_H, C.c_int32, C.c_int32, C.c_int32]),
     "ocean_gpu_profile_xact": (C.c_int, [_H, C.c_int32, C.c_int32, C.c_int32]),
     "ocean_gpu_haydock": (C.c_int, [_H, _DP, _DP, C.c_int32, _DP, _DP, _DP, _IP]),
+    "ocean_gpu_haydock_z": (C.c_int, [_H, _DP, C.c_int32, _DP, _DP, _DP, _IP]),
+    "ocean_gpu_haydock_multi_z": (C.c_int, [_H, _DP, C.c_int32, _DP, _DP, _DP, _IP]),
+    "ocean_gpu_batch_haydock_z": (C.c_int, [_H, C.POINTER(_DP), C.c_int32, C.POINTER(_DP), C.POINTER(_DP),
+                                            C.POINTER(_DP), _IP]),
     "ocean_gpu_haydock_early": (C.c_int, [_H, _DP, _DP, C.c_int32, C.c_int32, C.c_double, C.c_double,
                                           C.c_double, C.c_double, C.c_double, C.c_int32, _DP, _DP,
                                           _DP, _IP]),
@@ -154,6 +158,16 @@ def _planes(z, shape=None, name="array"):
     if shape is not None:
         _need(z, shape, name)
     return (np.asfortranarray(z.real, dtype=np.float64), np.asfortranarray(z.imag, dtype=np.float64))
+
+
+def _interleaved(z, shape, name):
+    """z in the library's interleaved order, without a copy where it is already held so."""
+    _need(z, shape, name)
+    return np.asfortranarray(z, dtype=np.complex128)
+
+
+def _pz(z):
+    return z.ctypes.data_as(_DP)
 
 
 def _need(a, shape, name):
@@ -570,13 +584,12 @@ class OceanGPU:
         With return_status the library's code is not raised: (a, b, ai, niter_done, rc)
         (rc = -1 and niter_done = the failing iteration on a NaN, as the reference's
         OCEAN_hay_ab_twoterm, OCEAN2/OCEAN_haydock.f90:912-920)."""
-        pr, pi = _planes(psi0, self.shape, "psi0")
+        z = _interleaved(psi0, self.shape, "psi0")
         a = np.zeros(niter + 1)
         b = np.zeros(niter + 1)
         ai = np.zeros(niter + 1)
         done = C.c_int32()
-        rc = _lib().ocean_gpu_haydock(self.h, _p(pr), _p(pi), niter, _p(a), _p(b), _p(ai),
-                                      C.byref(done))
+        rc = _lib().ocean_gpu_haydock_z(self.h, _pz(z), niter, _p(a), _p(b), _p(ai), C.byref(done))
         if return_status:
             return a, b, ai, done.value, rc
         _chk(rc, "haydock")
@@ -603,13 +616,17 @@ class OceanGPU:
         (a, b, ai, niter_done[nrhs], rc)."""
         z = np.asarray(psi0s)
         if z.shape == (self.nrhs,) + self.shape0:
-            z = np.concatenate(list(z), axis=2)
-        pr, pi = _planes(z, self.shape, "psi0s")
+            out = np.empty(self.shape, np.complex128, order="F")
+            na = self.shape0[2]
+            for r in range(self.nrhs):
+                out[:, :, r * na:(r + 1) * na] = z[r]
+            z = out
+        z = _interleaved(z, self.shape, "psi0s")
         R, n1 = self.nrhs, niter + 1
         a, b, ai = np.zeros(R * n1), np.zeros(R * n1), np.zeros(R * n1)
         done = np.zeros(R, np.int32)
-        rc = _lib().ocean_gpu_haydock_multi(self.h, _p(pr), _p(pi), niter, _p(a), _p(b), _p(ai),
-                                            done.ctypes.data_as(_IP))
+        rc = _lib().ocean_gpu_haydock_multi_z(self.h, _pz(z), niter, _p(a), _p(b), _p(ai),
+                                              done.ctypes.data_as(_IP))
         a, b, ai = a.reshape(R, n1), b.reshape(R, n1), ai.reshape(R, n1)
         if return_status:
             return a, b, ai, done, rc
@@ -731,9 +748,8 @@ class OceanBatch:
         n = len(self.problems)
         if len(psi0s) != n:
             raise ValueError("one starting vector per problem")
-        planes = [_planes(p, g.shape, "psi0") for p, g in zip(psi0s, self.problems)]
-        pr = (_DP * n)(*[_p(x[0]) for x in planes])
-        pi = (_DP * n)(*[_p(x[1]) for x in planes])
+        z = [_interleaved(p, g.shape, "psi0") for p, g in zip(psi0s, self.problems)]
+        pz = (_DP * n)(*[_pz(x) for x in z])
         A = [np.zeros(niter + 1) for _ in range(n)]
         Bv = [np.zeros(niter + 1) for _ in range(n)]
         AI = [np.zeros(niter + 1) for _ in range(n)]
@@ -741,7 +757,7 @@ class OceanBatch:
         pb = (_DP * n)(*[_p(x) for x in Bv])
         pai = (_DP * n)(*[_p(x) for x in AI])
         done = np.zeros(n, np.int32)
-        rc = _lib().ocean_gpu_batch_haydock(self.b, pr, pi, niter, pa, pb, pai, done.ctypes.data_as(_IP))
+        rc = _lib().ocean_gpu_batch_haydock_z(self.b, pz, niter, pa, pb, pai, done.ctypes.data_as(_IP))
         _chk(rc, "batch_haydock")
         ms = C.c_double()
         _chk(_lib().ocean_gpu_batch_last_ms(self.b, C.byref(ms)), "batch_last_ms")

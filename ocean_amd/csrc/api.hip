@@ -4,6 +4,7 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 
@@ -71,17 +72,74 @@ int ensure_pin(H* h, size_t ndouble) {
   return OCEAN_GPU_OK;
 }
 
-// host planes (n) -> device interleaved complex
-int put_planes(H* h, const double* re, const double* im, double2* dst, size_t n) {
+// Device workspace of n elements in one piece: a solve's vectors one by one cost an
+// allocation and a synchronising free each (206 of each at a GMRES depth of 100).  Up to
+// kKeepWs bytes stay with their owner until it is destroyed; more goes back after the
+// call (give_ws).
+constexpr size_t kKeepWs = (size_t)256 << 20;
+
+int take_ws(double2** ws, size_t* have, size_t n) {
+  if (*have >= n) return OCEAN_GPU_OK;
+  dfree(*ws);
+  *have = 0;
+  OG_TRY(dmalloc(ws, n));
+  *have = n;
+  return OCEAN_GPU_OK;
+}
+void give_ws(double2** ws, size_t* have) {
+  if (*have * sizeof(double2) <= kKeepWs) return;
+  dfree(*ws);
+  *have = 0;
+}
+
+// A host vector: planes (step 1, im may be null) or interleaved (im = re + 1, step 2).
+struct HostVec {
+  const double* re;
+  const double* im;
+  size_t step;
+};
+HostVec interleaved(const double* z) { return {z, z + 1, 2}; }
+
+// host vector (n) -> device interleaved complex, through pinned memory; a vector of
+// several MB is staged by four threads, each part on its way as soon as it is there
+int put_vec(H* h, const HostVec& v, double2* dst, size_t n) {
   OG_TRY(ensure_pin(h, 2 * n));
   double* p = h->host_pin;
-  for (size_t i = 0; i < n; ++i) {
-    p[2 * i] = re[i];
-    p[2 * i + 1] = im ? im[i] : 0.0;
+  auto fill = [&](size_t a, size_t b) {
+    if (v.step == 2) {
+      std::memcpy(p + 2 * a, v.re + 2 * a, (b - a) * sizeof(double2));
+      return;
+    }
+    for (size_t i = a; i < b; ++i) {
+      p[2 * i] = v.re[i];
+      p[2 * i + 1] = v.im ? v.im[i] : 0.0;
+    }
+  };
+  constexpr int T = 4;
+  std::thread th[T];
+  const int parts = n >= (size_t)1 << 18 ? T : 1;
+  auto at = [&](int t) { return n * t / parts; };
+  for (int t = 1; t < parts; ++t) {
+    try {
+      th[t] = std::thread(fill, at(t), at(t + 1));
+    } catch (const std::system_error&) {  // no thread to be had: this one fills the part below
+    }
   }
-  OG_CHECK(hipMemcpyAsync(dst, p, n * sizeof(double2), hipMemcpyHostToDevice, h->stream));
+  int rc = OCEAN_GPU_OK;
+  for (int t = 0; t < parts; ++t) {
+    if (th[t].joinable()) th[t].join();
+    else fill(at(t), at(t + 1));
+    if (rc == 0 && hipMemcpyAsync(dst + at(t), p + 2 * at(t), (at(t + 1) - at(t)) * sizeof(double2),
+                                  hipMemcpyHostToDevice, h->stream) != hipSuccess)
+      rc = OCEAN_GPU_ERR_HIP;
+  }
+  OG_TRY(rc);
   OG_CHECK(hipStreamSynchronize(h->stream));
   return OCEAN_GPU_OK;
+}
+
+int put_planes(H* h, const double* re, const double* im, double2* dst, size_t n) {
+  return put_vec(h, {re, im, 1}, dst, n);
 }
 
 int get_planes(H* h, const double2* src, double* re, double* im, size_t n) {
@@ -1208,6 +1266,8 @@ int ocean_gpu_destroy(ocean_gpu_handle* h) {
   dfree(h->cproj); dfree(h->Kmat); dfree(h->apart); dfree(h->hmult); dfree(h->Smat);
   dfree(h->energy); dfree(h->allow); dfree(h->red); dfree(h->scal); dfree(h->tmp_in); dfree(h->tmp_out);
   for (auto& v : h->vecs) dfree(v);
+  if (h->pin_ctl) (void)hipHostFree(h->pin_ctl);
+  dfree(h->ws);
   if (h->host_pin) (void)hipHostFree(h->host_pin);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -1758,8 +1818,8 @@ struct EarlyExit {
   int ne = 0;
 };
 
-int haydock_run(H* h, const double* psi0_re, const double* psi0_im, int niter, const EarlyExit* ex,
-                double* real_a, double* real_b, double* imag_a, int32_t* niter_done) {
+int haydock_run(H* h, const HostVec& psi0, int niter, const EarlyExit* ex, double* real_a,
+                double* real_b, double* imag_a, int32_t* niter_done) {
   if (h->nrhs != 1) return OCEAN_GPU_ERR_UNSUPPORTED;  // ocean_gpu_haydock_multi
   const int f = flags_of(h, 0, nullptr);
   OG_TRY(check_ready(h, f));
@@ -1773,11 +1833,9 @@ int haydock_run(H* h, const double* psi0_re, const double* psi0_im, int niter, c
   double* db = dai + n1;
   double* conv = da + ns;                 // [iter][relArea, maxDiff]
   double* cpart = conv + 2 * n1;
-  double2 *v0 = nullptr, *v1 = nullptr, *v2 = nullptr;
-  OG_TRY(dmalloc(&v0, nv));
-  if (dmalloc(&v1, nv) || dmalloc(&v2, nv)) { dfree(v0); dfree(v1); return OCEAN_GPU_ERR_NOMEM; }
-  int rc = put_planes(h, psi0_re, psi0_im, v0, nv);
-  double2 *psi = v0, *old = v1, *hv = v2;
+  OG_TRY(take_ws(&h->ws, &h->ws_n, 3 * nv));
+  double2 *psi = h->ws, *old = psi + nv, *hv = old + nv;
+  int rc = put_vec(h, psi0, psi, nv);
   int done = niter;
   // early exit: the convergence figures are formed on the device every iteration
   // and read back every kCheck iterations; the reference's decision is replayed in
@@ -1838,7 +1896,7 @@ int haydock_run(H* h, const double* psi0_re, const double* psi0_im, int niter, c
         hipStreamSynchronize(h->stream) != hipSuccess)
       rc = OCEAN_GPU_ERR_HIP;
   }
-  dfree(v0); dfree(v1); dfree(v2);
+  give_ws(&h->ws, &h->ws_n);
   if (rc) return rc;
   for (int i = 0; i < done; ++i)
     if (hb[i] != hb[i]) { done = i + 1; rc = OCEAN_GPU_ERR_NAN; break; }
@@ -1859,7 +1917,13 @@ extern "C" {
 int ocean_gpu_haydock(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im, int32_t niter,
                       double* real_a, double* real_b, double* imag_a, int32_t* niter_done) {
   if (!h || !psi0_re || !psi0_im || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
-  return haydock_run(h, psi0_re, psi0_im, niter, nullptr, real_a, real_b, imag_a, niter_done);
+  return haydock_run(h, {psi0_re, psi0_im, 1}, niter, nullptr, real_a, real_b, imag_a, niter_done);
+}
+
+int ocean_gpu_haydock_z(ocean_gpu_handle* h, const double* psi0, int32_t niter, double* real_a, double* real_b,
+                        double* imag_a, int32_t* niter_done) {
+  if (!h || !psi0 || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+  return haydock_run(h, interleaved(psi0), niter, nullptr, real_a, real_b, imag_a, niter_done);
 }
 
 int ocean_gpu_haydock_early(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im, int32_t niter,
@@ -1875,29 +1939,31 @@ int ocean_gpu_haydock_early(ocean_gpu_handle* h, const double* psi0_re, const do
   ex.el = el;
   ex.eh = eh;
   ex.ne = ne;
-  return haydock_run(h, psi0_re, psi0_im, niter, &ex, real_a, real_b, imag_a, niter_done);
+  return haydock_run(h, {psi0_re, psi0_im, 1}, niter, &ex, real_a, real_b, imag_a, niter_done);
 }
+
+}  // extern "C"
+
+namespace {
 
 // The recursions of every right-hand side of the handle at once: one action over the
 // stacked vector per iteration (each u stream serves all nrhs right-hand sides), then
 // the three-term steps of OCEAN_hay_ab_twoterm (OCEAN2/OCEAN_haydock.f90:824-938) per
 // right-hand side in one launch each, with the fixed-order reductions of the
 // one-right-hand-side recursion.
-int ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im, int32_t niter,
-                            double* real_a, double* real_b, double* imag_a, int32_t* niter_done) {
-  if (!h || !psi0_re || !psi0_im || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+int haydock_multi_run(H* h, const HostVec& psi0, int niter, double* real_a, double* real_b, double* imag_a,
+                      int32_t* niter_done) {
   const int f = flags_of(h, 0, nullptr);
   OG_TRY(check_ready(h, f));
   const int R = h->nrhs;
   const size_t nv = h->nvec(), nv0 = h->nvec0();
   const size_t n1 = (size_t)niter + 1;
   const size_t nscal = hay_scalars(h, n1);
-  double2* V[3] = {nullptr, nullptr, nullptr};
-  double* S = nullptr;
-  int rc = OCEAN_GPU_OK;
-  for (int i = 0; i < 3 && rc == 0; ++i) rc = dmalloc(&V[i], nv);
-  if (rc == 0) rc = dmalloc(&S, (size_t)R * nscal);
-  if (rc == 0) rc = put_planes(h, psi0_re, psi0_im, V[0], nv);
+  OG_TRY(ensure_scal(h, (size_t)R * nscal));
+  OG_TRY(take_ws(&h->ws, &h->ws_n, 3 * nv));
+  double* S = h->scal;
+  double2* V[3] = {h->ws, h->ws + nv, h->ws + 2 * nv};
+  int rc = put_vec(h, psi0, V[0], nv);
   // rotation r of an iteration: (psi, old, hv) = (V0, V1, V2), (V2, V0, V1), (V1, V2, V0)
   const int rot[3][3] = {{0, 1, 2}, {2, 0, 1}, {1, 2, 0}};
   og::HayFuse hf;
@@ -1942,9 +2008,24 @@ int ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const do
     }
     if (niter_done) niter_done[q] = done;
   }
-  for (auto& v : V) dfree(v);
-  dfree(S);
+  give_ws(&h->ws, &h->ws_n);
   return rc ? rc : rc_nan;
+}
+
+}  // namespace
+
+extern "C" {
+
+int ocean_gpu_haydock_multi(ocean_gpu_handle* h, const double* psi0_re, const double* psi0_im, int32_t niter,
+                            double* real_a, double* real_b, double* imag_a, int32_t* niter_done) {
+  if (!h || !psi0_re || !psi0_im || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+  return haydock_multi_run(h, {psi0_re, psi0_im, 1}, niter, real_a, real_b, imag_a, niter_done);
+}
+
+int ocean_gpu_haydock_multi_z(ocean_gpu_handle* h, const double* psi0, int32_t niter, double* real_a, double* real_b,
+                              double* imag_a, int32_t* niter_done) {
+  if (!h || !psi0 || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+  return haydock_multi_run(h, interleaved(psi0), niter, real_a, real_b, imag_a, niter_done);
 }
 
 // The non-Hermitian (bi-Lanczos) recursion of OCEAN2's complex_haydock branch
@@ -2171,12 +2252,12 @@ int ocean_gpu_spectrum(const double* real_a, const double* real_b, const double*
   double *d = nullptr;
   const size_t n1 = (size_t)niter + 1;
   OG_TRY(dmalloc(&d, 3 * n1 + 5 * ((size_t)ne + 1)));
-  std::vector<double> ia(n1, 0.0);
-  if (imag_a) std::copy(imag_a, imag_a + n1, ia.begin());
+  std::vector<double> co(3 * n1, 0.0);  // a, b, imag a in one copy
+  std::copy(real_a, real_a + n1, co.begin());
+  std::copy(real_b, real_b + n1, co.begin() + n1);
+  if (imag_a) std::copy(imag_a, imag_a + n1, co.begin() + 2 * n1);
   int rc = OCEAN_GPU_OK;
-  if (hipMemcpy(d, real_a, n1 * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d + n1, real_b, n1 * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d + 2 * n1, ia.data(), n1 * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemcpy(d, co.data(), co.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
     rc = OCEAN_GPU_ERR_HIP;
   if (rc == 0) {
     og::k_cfrac<<<(ne + 1 + 127) / 128, 128>>>(d, d + n1, d + 2 * n1, niter, kpref, gam, el, eh, ne,
@@ -2269,35 +2350,36 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   hipStream_t st = h->stream;
   // vectors: rhs, h1, x, ax, g, pcdiv, u[1..depth], au[1..depth]
   const int nfix = 6;
-  std::vector<double2*> V(nfix + 2 * depth, nullptr);
-  int rc = OCEAN_GPU_OK;
-  for (auto& p : V)
-    if (rc == 0) rc = dmalloc(&p, nv);
-  double2** dlist = nullptr;
-  double2* dcoef = nullptr;
-  double* part = nullptr;
-  if (rc == 0) rc = dmalloc(&dlist, 2 * (size_t)depth + 2);
-  if (rc == 0) rc = dmalloc(&dcoef, (size_t)depth);
-  if (rc == 0) rc = dmalloc(&part, (size_t)kRedBlocks * 4 * depth + 4 * (size_t)depth + 3 * (size_t)kRedBlocks + 16);
-  double2* dL = nullptr;
-  double* dD = nullptr;
-  double2* dC = nullptr;   // cumulative least-squares coefficients of the cycle
-  double2* dRU = nullptr;  // <rhs|U_i>
-  GmCtl* ctl = nullptr;
-  GmCtl* hctl = nullptr;
-  if (rc == 0) rc = dmalloc(&dL, (size_t)depth * (depth - 1) / 2 + 1);
-  if (rc == 0) rc = dmalloc(&dD, (size_t)depth);
-  if (rc == 0) rc = dmalloc(&dC, (size_t)depth);
-  if (rc == 0) rc = dmalloc(&dRU, (size_t)depth);
-  if (rc == 0) rc = dmalloc(&ctl, (size_t)1);
-  if (rc == 0 && hipHostMalloc((void**)&hctl, sizeof(GmCtl), hipHostMallocDefault) != hipSuccess)
-    rc = OCEAN_GPU_ERR_NOMEM;
-  auto cleanup = [&]() {
-    for (auto& p : V) dfree(p);
-    dfree(dlist); dfree(dcoef); dfree(part); dfree(dL); dfree(dD); dfree(dC); dfree(dRU); dfree(ctl);
-    if (hctl) (void)hipHostFree(hctl);
+  // one workspace: the vectors, then the tables (offsets in 16-byte elements)
+  const size_t nd = (size_t)depth, npart = (size_t)kRedBlocks * 4 * nd + 4 * nd + 3 * (size_t)kRedBlocks + 16;
+  size_t at = (nfix + 2 * nd) * nv;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 15) / 16;
+    return o;
   };
-  if (rc) { cleanup(); return rc; }
+  const size_t o_list = take((2 * nd + 2) * sizeof(double2*)), o_coef = take(nd * sizeof(double2));
+  const size_t o_part = take(npart * sizeof(double)), o_L = take((nd * (nd - 1) / 2 + 1) * sizeof(double2));
+  const size_t o_D = take(nd * sizeof(double)), o_C = take(nd * sizeof(double2)), o_RU = take(nd * sizeof(double2));
+  const size_t o_ctl = take(sizeof(GmCtl));
+  OG_TRY(take_ws(&h->ws, &h->ws_n, at));
+  if (!h->pin_ctl && hipHostMalloc(&h->pin_ctl, sizeof(GmCtl), hipHostMallocDefault) != hipSuccess) {
+    h->pin_ctl = nullptr;
+    return OCEAN_GPU_ERR_NOMEM;
+  }
+  std::vector<double2*> V(nfix + 2 * nd);
+  for (size_t i = 0; i < V.size(); ++i) V[i] = h->ws + i * nv;
+  double2** dlist = reinterpret_cast<double2**>(h->ws + o_list);
+  double2* dcoef = h->ws + o_coef;
+  double* part = reinterpret_cast<double*>(h->ws + o_part);
+  double2* dL = h->ws + o_L;
+  double* dD = reinterpret_cast<double*>(h->ws + o_D);
+  double2* dC = h->ws + o_C;    // cumulative least-squares coefficients of the cycle
+  double2* dRU = h->ws + o_RU;  // <rhs|U_i>
+  GmCtl* ctl = reinterpret_cast<GmCtl*>(h->ws + o_ctl);
+  GmCtl* hctl = static_cast<GmCtl*>(h->pin_ctl);
+  int rc = OCEAN_GPU_OK;
+  auto cleanup = [&]() { give_ws(&h->ws, &h->ws_n); };
   int* skip = &ctl->done;
   int* info = &ctl->info;
   double2 *rhs = V[0], *h1 = V[1], *x = V[2], *ax = V[3], *g = V[4], *pc = V[5];
@@ -2729,6 +2811,8 @@ struct ocean_gpu_batch {
   std::vector<Group> groups;
   hipStream_t stream = nullptr;
   int* dcount = nullptr;  // [0] Haydock iteration number, [1] its copy for k_hay2
+  double2* ws = nullptr;  // the recursions' vectors and scalars, kept up to kKeepWs bytes
+  size_t ws_n = 0;
   double t_last = 0.0;    // ms per batched action (all problems) of the last timed call
 };
 
@@ -2961,6 +3045,7 @@ int ocean_gpu_batch_destroy(ocean_gpu_batch* b) {
   if (!b) return OCEAN_GPU_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   if (b->dcount) (void)hipFree(b->dcount);
+  dfree(b->ws);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
   return OCEAN_GPU_OK;
@@ -3134,25 +3219,31 @@ int ocean_gpu_batch_last_ms(ocean_gpu_batch* b, double* ms) {
   return OCEAN_GPU_OK;
 }
 
-int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, const double* const* psi_im,
-                            int32_t niter, double* const* real_a, double* const* real_b,
-                            double* const* imag_a, int32_t* niter_done) {
-  if (!b || !psi_re || !psi_im || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+namespace {
+
+int batch_haydock_run(ocean_gpu_batch* b, const std::vector<HostVec>& psi0, int niter, double* const* real_a,
+                      double* const* real_b, double* const* imag_a, int32_t* niter_done) {
   const int n = (int)b->hs.size();
   // one recursion per problem: a problem with several right-hand sides runs
   // ocean_gpu_haydock_multi on its own
   for (H* h : b->hs)
     if (h->nrhs != 1) return OCEAN_GPU_ERR_UNSUPPORTED;
+  for (int q = 0; q < n; ++q)
+    if (!psi0[q].re || !psi0[q].im || !real_a[q] || !real_b[q]) return OCEAN_GPU_ERR_ARG;
   const size_t n1 = (size_t)niter + 1;
+  size_t tot = 0;
+  for (H* h : b->hs) tot += 3 * h->nvec() + (hay_scalars(h, n1) + 1) / 2;
+  OG_TRY(take_ws(&b->ws, &b->ws_n, tot));
   std::vector<double2*> V((size_t)3 * n, nullptr);
   std::vector<double*> Sd((size_t)n, nullptr);
   int rc = OCEAN_GPU_OK;
+  double2* at = b->ws;
   for (int q = 0; q < n && rc == 0; ++q) {
     H* h = b->hs[q];
-    if (!psi_re[q] || !psi_im[q] || !real_a[q] || !real_b[q]) rc = OCEAN_GPU_ERR_ARG;
-    for (int i = 0; i < 3 && rc == 0; ++i) rc = dmalloc(&V[(size_t)3 * q + i], h->nvec());
-    if (rc == 0) rc = dmalloc(&Sd[q], hay_scalars(h, n1));
-    if (rc == 0) rc = put_planes(h, psi_re[q], psi_im[q], V[(size_t)3 * q], h->nvec());
+    for (int i = 0; i < 3; ++i, at += h->nvec()) V[(size_t)3 * q + i] = at;
+    Sd[q] = reinterpret_cast<double*>(at);
+    at += (hay_scalars(h, n1) + 1) / 2;
+    rc = put_vec(h, psi0[q], V[(size_t)3 * q], h->nvec());
   }
   // rotation r of an iteration: (psi, old, hv) = (V0, V1, V2), (V2, V0, V1), (V1, V2, V0)
   const int rot[3][3] = {{0, 1, 2}, {2, 0, 1}, {1, 2, 0}};
@@ -3261,10 +3352,29 @@ int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, con
   for (auto& tr : tabs)
     for (auto& t : tr) t.release();
   for (int r = 0; r < 3; ++r) dfree(dhay[r]);
-  for (auto& v : V) dfree(v);
-  for (auto& s : Sd) dfree(s);
+  give_ws(&b->ws, &b->ws_n);
   return rc ? rc : rc_nan;
 }
+
+}  // namespace
+
+int ocean_gpu_batch_haydock(ocean_gpu_batch* b, const double* const* psi_re, const double* const* psi_im,
+                            int32_t niter, double* const* real_a, double* const* real_b,
+                            double* const* imag_a, int32_t* niter_done) {
+  if (!b || !psi_re || !psi_im || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+  std::vector<HostVec> v;
+  for (size_t q = 0; q < b->hs.size(); ++q) v.push_back({psi_re[q], psi_im[q], 1});
+  return batch_haydock_run(b, v, niter, real_a, real_b, imag_a, niter_done);
+}
+
+int ocean_gpu_batch_haydock_z(ocean_gpu_batch* b, const double* const* psi0, int32_t niter, double* const* real_a,
+                              double* const* real_b, double* const* imag_a, int32_t* niter_done) {
+  if (!b || !psi0 || niter <= 0 || !real_a || !real_b) return OCEAN_GPU_ERR_ARG;
+  std::vector<HostVec> v;
+  for (size_t q = 0; q < b->hs.size(); ++q) v.push_back(psi0[q] ? interleaved(psi0[q]) : HostVec{nullptr, nullptr, 2});
+  return batch_haydock_run(b, v, niter, real_a, real_b, imag_a, niter_done);
+}
+
 
 // GMRES of every problem of the batch at once: each problem's recycled solve runs on
 // its own handle's stream, driven by one of up to kGmresWorkers host threads, so the

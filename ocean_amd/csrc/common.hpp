@@ -267,6 +267,9 @@ struct ocean_gpu_handle {
   size_t scal_n = 0;
   double* host_pin = nullptr;  // pinned staging for host planes
   size_t host_pin_n = 0;
+  double2* ws = nullptr;       // the solvers' vectors, kept between calls up to kKeepWs bytes
+  size_t ws_n = 0;
+  void* pin_ctl = nullptr;     // pinned copy of the GMRES control state
   double2* tmp_in = nullptr;   // host-plane xact staging
   double2* tmp_out = nullptr;
 

@@ -1,0 +1,50 @@
+"""Host vectors and workspaces: the interleaved entry points against the ones with planes,
+vectors long enough to be staged in parts, and workspaces that other solves have used."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from ocean_amd import core, synth  # noqa: E402
+
+
+def _planes_haydock(g, psi, niter):
+    re, im = np.asfortranarray(psi.real), np.asfortranarray(psi.imag)
+    a, b, ai = (np.zeros(niter + 1) for _ in range(3))
+    done = C.c_int32()
+    rc = core._lib().ocean_gpu_haydock(g.h, core._p(re), core._p(im), niter, core._p(a), core._p(b), core._p(ai),
+                                       C.byref(done))
+    assert rc == 0 and done.value == niter
+    return a, b, ai
+
+
+# 2 560 elements; 393 216, past the 262 144 from which a vector is staged in four parts
+@pytest.mark.parametrize("nb,kmesh,xmesh,lc", [(10, (4, 4, 4), (3, 3, 2), 0), (64, (8, 8, 8), (4, 4, 4), 1)])
+def test_interleaved_and_planes_agree(nb, kmesh, xmesh, lc):
+    inp = synth.make_inputs(nb=nb, kmesh=kmesh, xmesh=xmesh, lc=lc, seed=95, xi_eV=3.0 if lc else 0.0)
+    rng = np.random.default_rng(3)
+    with core.OceanGPU.from_inputs(inp) as g:
+        z = np.asfortranarray(rng.standard_normal(g.shape) + 1j * rng.standard_normal(g.shape))
+        v = g.vec_new(z)
+        assert np.array_equal(g.vec_get(v), z)
+        want = _planes_haydock(g, inp.psi0, 3)
+        for psi in (inp.psi0, np.ascontiguousarray(inp.psi0)):  # held in the library's order, and not
+            for x, y in zip(g.haydock(psi, 3), want):
+                assert np.array_equal(x, y)
+
+
+def test_workspace_is_shared_by_the_solves():
+    """Recursions before and after a GMRES solve on the same handle (its vectors take the
+    same workspace) and another length of recursion give the same coefficients."""
+    inp = synth.make_inputs(nb=9, kmesh=(3, 2, 4), xmesh=(3, 3, 3), lc=0, seed=96)
+    with core.OceanGPU.from_inputs(inp) as g:
+        first = g.haydock(inp.psi0, 12)
+        e = np.array([3.0, 9.0])
+        rows = g.gmres(inp.psi0, e, 0.5, 13.605, 1e-12, 20)
+        g.haydock(inp.psi0, 30)
+        again = g.haydock(inp.psi0, 12)
+        assert np.array_equal(g.gmres(inp.psi0, e, 0.5, 13.605, 1e-12, 20), rows)
+        for x, y in zip(first, again):
+            assert np.array_equal(x, y)
