@@ -595,7 +595,7 @@ int dev_nrm(H* h, const double2* p, double* v) {
 // ---------------------------------------------------------------------------
 // GMRES helpers
 // ---------------------------------------------------------------------------
-// <W_i|v1>, <W_i|v2> for i < m: partials [i][4][eb].  Workgroup (row group, b) takes
+// <W_i|v1>, <W_i|v2> for i < m, row i at W + i ld: partials [i][4][eb].  Workgroup (row group, b) takes
 // eight rows of W over the elements of slice b, all its loads in flight; the 32 sums
 // reduce by one butterfly per wave and one LDS round across the waves.  The rows are
 // spread over the grid (not looped over in the workgroup), so that a short vector,
@@ -604,7 +604,7 @@ int dev_nrm(H* h, const double2* p, double* v) {
 // elements 21.4 -> 18.4 us (4.8 TB/s; 34 us at 90 rows).
 constexpr int kDotRows = 8, kDotThreads = 256;
 __global__ __launch_bounds__(kDotThreads) void k_multidot2(const int* __restrict__ skip,
-                                                      const double2* const* __restrict__ Wl, int m,
+                                                      const double2* __restrict__ W, size_t ld, int m,
                                                       const double2* __restrict__ v1,
                                                       const double2* __restrict__ v2, size_t n, int eb,
                                                       double* __restrict__ part) {
@@ -618,7 +618,7 @@ __global__ __launch_bounds__(kDotThreads) void k_multidot2(const int* __restrict
   for (int q = 0; q < 4 * R; ++q) v[q] = 0.0;
   const double2* row[R];
 #pragma unroll
-  for (int q = 0; q < R; ++q) row[q] = Wl[min(i0 + q, m - 1)];
+  for (int q = 0; q < R; ++q) row[q] = W + (size_t)min(i0 + q, m - 1) * ld;
   for (size_t e = (size_t)b * blockDim.x + threadIdx.x; e < n; e += (size_t)eb * blockDim.x) {
     const double2 b1 = v1[e], c1 = v2[e];
     double2 a[R];
@@ -658,7 +658,7 @@ int dot_slices(size_t n, int m) {
 // when the basis is about to be replaced or the solve has converged); terms with
 // C_i = 0 are skipped (their U_i may not have been formed).  skip may be null.
 __global__ __launch_bounds__(kBlock) void k_materialize(const int* __restrict__ skip,
-                                                        const double2* const* __restrict__ Ul,
+                                                        const double2* __restrict__ U, size_t ld,
                                                         const double2* __restrict__ C, int m,
                                                         double2* __restrict__ x, size_t n) {
   if (skip && *skip) return;
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(kBlock) void k_materialize(const int* __restrict__ 
       for (int q = 0; q < R; ++q) {
         ci[q] = C[min(i0 + q, m - 1)];
         const bool use = i0 + q < m && (ci[q].x != 0.0 || ci[q].y != 0.0);
-        w[q] = use ? Ul[i0 + q][e] : make_double2(0.0, 0.0);
+        w[q] = use ? U[(size_t)(i0 + q) * ld + e] : make_double2(0.0, 0.0);
       }
 #pragma unroll
       for (int q = 0; q < R; ++q) {
@@ -1059,11 +1059,12 @@ __global__ __launch_bounds__(kBlock) void k_pc_apply(GmCtl* __restrict__ c, doub
 // wave); the shares are added in LDS in order.  With the rows of an element on one
 // thread the kernel waited on m / 8 dependent rounds of loads with one wave per SIMD:
 // averages over solves of up to 80 rows at 3 120 elements 9.4 -> 5.8 us, up to 100 rows
-// at 131 072 elements 19.1 us as before (36 us at 90 rows, 5.2 TB/s).
+// at 131 072 elements 19.1 us as before; with the rows 512 bytes past a power of two apart
+// (at 2 MB they fall on the same HBM channels) 19.5 -> 17.7 us.
 constexpr int kAxThreads = 1024;
 template <int RS>
 __global__ __launch_bounds__(kAxThreads) void k_axpy_resid(GmCtl* __restrict__ c,
-                                                           const double2* const* __restrict__ AUl,
+                                                           const double2* __restrict__ AU, size_t ld,
                                                            const double2* __restrict__ coef, int m,
                                                            double2* __restrict__ ax, const double2* __restrict__ rhs,
                                                            double2* __restrict__ g, const double2* __restrict__ pc,
@@ -1090,7 +1091,7 @@ __global__ __launch_bounds__(kAxThreads) void k_axpy_resid(GmCtl* __restrict__ c
     for (int i0 = ia; i0 < ib; i0 += R) {
       double2 a[R];
 #pragma unroll
-      for (int q = 0; q < R; ++q) a[q] = AUl[min(i0 + q, ib - 1)][ec];
+      for (int q = 0; q < R; ++q) a[q] = AU[(size_t)min(i0 + q, ib - 1) * ld + ec];
 #pragma unroll
       for (int q = 0; q < R; ++q)
         if (i0 + q < ib) og::cfma(sum, coef[i0 + q], a[q]);
@@ -2350,15 +2351,18 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   hipStream_t st = h->stream;
   // vectors: rhs, h1, x, ax, g, pcdiv, u[1..depth], au[1..depth]
   const int nfix = 6;
-  // one workspace: the vectors, then the tables (offsets in 16-byte elements)
+  // one workspace: the vectors (U and AU as consecutive rows, so that the step kernels
+  // need no pointer table and recycling is one launch), then the small state (offsets in
+  // 16-byte elements)
   const size_t nd = (size_t)depth, npart = (size_t)kRedBlocks * 4 * nd + 4 * nd + 3 * (size_t)kRedBlocks + 16;
-  size_t at = (nfix + 2 * nd) * nv;
+  const size_t ld = nv + 32;  // off the power of two (see k_axpy_resid)
+  size_t at = (nfix + 2 * nd) * ld;
   auto take = [&](size_t bytes) {
     const size_t o = at;
     at += (bytes + 15) / 16;
     return o;
   };
-  const size_t o_list = take((2 * nd + 2) * sizeof(double2*)), o_coef = take(nd * sizeof(double2));
+  const size_t o_coef = take(nd * sizeof(double2));
   const size_t o_part = take(npart * sizeof(double)), o_L = take((nd * (nd - 1) / 2 + 1) * sizeof(double2));
   const size_t o_D = take(nd * sizeof(double)), o_C = take(nd * sizeof(double2)), o_RU = take(nd * sizeof(double2));
   const size_t o_ctl = take(sizeof(GmCtl));
@@ -2368,8 +2372,7 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
     return OCEAN_GPU_ERR_NOMEM;
   }
   std::vector<double2*> V(nfix + 2 * nd);
-  for (size_t i = 0; i < V.size(); ++i) V[i] = h->ws + i * nv;
-  double2** dlist = reinterpret_cast<double2**>(h->ws + o_list);
+  for (size_t i = 0; i < V.size(); ++i) V[i] = h->ws + i * ld;
   double2* dcoef = h->ws + o_coef;
   double* part = reinterpret_cast<double*>(h->ws + o_part);
   double2* dL = h->ws + o_L;
@@ -2385,8 +2388,6 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   double2 *rhs = V[0], *h1 = V[1], *x = V[2], *ax = V[3], *g = V[4], *pc = V[5];
   double2** U = &V[nfix];            // U[i], i = 0..depth-1  (reference u_matrix(i+1))
   double2** AU = &V[nfix + depth];   // AU[i]
-  std::vector<double2*> hlist(2 * depth);
-  for (int i = 0; i < depth; ++i) { hlist[i] = AU[i]; hlist[depth + i] = U[i]; }
 
   auto launched = [&]() -> int {
     if (hipGetLastError() != hipSuccess) return OCEAN_GPU_ERR_HIP;
@@ -2399,8 +2400,6 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   og::k_fill<<<1, 64, 0, st>>>(dC, make_double2(0.0, 0.0), (size_t)depth);
   rc = launched();
   if (rc == 0) rc = xact_dev(h, x, h1, f);  // h1 = H . 1
-  if (rc == 0) rc = hipMemcpy(dlist, hlist.data(), 2 * depth * sizeof(double2*), hipMemcpyHostToDevice) == hipSuccess
-                        ? OCEAN_GPU_OK : OCEAN_GPU_ERR_HIP;
 
   // A finish of a residual step that the next action's projection runs (within a
   // restart cycle the next kernel after the residual step is always that projection)
@@ -2423,8 +2422,7 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   // gated: dropped once the solve has stopped (the converged x is formed by the host's
   // ungated call after reading the state)
   auto materialise = [&](bool gated) -> int {
-    k_materialize<<<grid, kBlock, 0, st>>>(gated ? skip : nullptr, (const double2* const*)(dlist + depth), dC, depth,
-                                           x, nv);
+    k_materialize<<<grid, kBlock, 0, st>>>(gated ? skip : nullptr, U[0], ld, dC, depth, x, nv);
     k_fold_c<<<1, 64, 0, st>>>(gated ? skip : nullptr, ctl, dC, dRU, depth);
     return launched();
   };
@@ -2449,7 +2447,7 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   auto update = [&](int cur, int rit = -1, int check = 0, double2* unext = nullptr) -> int {
     const int eb = dot_slices(nv, cur);
     k_multidot2<<<eb * ((cur + kDotRows - 1) / kDotRows), kDotThreads, 0, st>>>(
-        skip, (const double2* const*)dlist, cur, AU[cur - 1], g, nv, eb, part);
+        skip, AU[0], ld, cur, AU[cur - 1], g, nv, eb, part);
     const size_t sm = ls_lds(cur, true);
     if (sm <= h->lds_max) {
       OG_TRY(lds_opt_in(k_ls_update<true>, sm));
@@ -2465,7 +2463,7 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
       const size_t epb = kAxThreads / (wide ? 16 : 4);
       const int nblk = (int)std::min<size_t>(kRedBlocks, (nv + epb - 1) / epb);
       (wide ? k_axpy_resid<16> : k_axpy_resid<4>)<<<nblk, kAxThreads, 0, st>>>(
-          ctl, (const double2* const*)dlist, dcoef, cur, ax, rhs, g, pc, unext, nv, rpart);
+          ctl, AU[0], ld, dcoef, cur, ax, rhs, g, pc, unext, nv, rpart);
       const GmFin F = fin_of(rit, check, kResU, cur, unext ? cur : -1, nblk);
       if (ride && check && unext) {
         // the next kernel is the next iteration's projection: the finish rides on it
@@ -2517,7 +2515,8 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
     } else {
       // make_recycle: au += (E - E_prev) u, then the updates over the kept basis
       const double delta = E - energies_eV[step - 1] * kEV2Hartree;
-      for (int i = 0; i < prev_iter; ++i) k_axpy_gated<<<grid, kBlock, 0, st>>>(skip, delta, 0.0, U[i], AU[i], nv);
+      const size_t nr = (size_t)prev_iter * ld;  // the rows' padding included
+      k_axpy_gated<<<grid_for(nr), kBlock, 0, st>>>(skip, delta, 0.0, U[0], AU[0], nr);
       if ((rc = axmy_xact(x, ax, E))) break;
       if ((rc = resid(0, 0))) break;
       for (int it = 1; it <= prev_iter && rc == 0; ++it) rc = update(it, 0, 0, nullptr);
