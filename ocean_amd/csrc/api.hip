@@ -2995,7 +2995,7 @@ int ocean_gpu_batch_create(ocean_gpu_handle* const* hs, int32_t n, ocean_gpu_bat
   *out = nullptr;
   B* b = new B();
   for (int i = 0; i < n; ++i) {
-    // each problem owns its multiplet scratch and counter: no handle twice
+    // each problem owns its multiplet scratch and workspaces: no handle twice
     if (!hs[i] || hs[i]->device != hs[0]->device ||
         std::find(b->hs.begin(), b->hs.end(), hs[i]) != b->hs.end()) {
       delete b;
