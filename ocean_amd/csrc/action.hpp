@@ -1169,8 +1169,9 @@ __device__ void mred_rows(const double2* __restrict__ apart, const double2* __re
 // projector rows are loaded before the u stream starts, so their latency hides
 // under it: with one k per workgroup the whole grid is resident at once and any
 // load left to the end would be paid by every workgroup together.
-// One workgroup per k; threads (n, xs) with n fastest.  JR alphas per reduction
-// round through LDS (the reduction buffer reuses the phi' staging area).
+// One workgroup per k; threads (n, xs) with n fastest, in whole waves (the threads past
+// nb XS only stage and finish).  JR alphas per reduction round through LDS (the
+// reduction buffer reuses the phi' staging area).
 // ---------------------------------------------------------------------------
 template <typename T2, int NA, bool HAY>
 __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
@@ -1386,8 +1387,8 @@ __device__ __forceinline__ void adj_body(const ActArgs<T2>& A, int blk) {
   }
   if constexpr (HAY) {
     __syncthreads();
-    if ((t >> 6) < (bd >> 6))  // whole waves: at least four, as bd > 256
-      for (int q = t >> 6; q < na / na0; q += bd >> 6) hay_part(A.hay, res + q * na0 * nb, na0 * nb, q, k);
+    // one wave per right-hand side: bd is a whole number of waves, at least one
+    for (int q = t >> 6; q < na / na0; q += bd >> 6) hay_part(A.hay, res + q * na0 * nb, na0 * nb, q, k);
     if (A.hay.itp && blk == 0 && t == 0) A.hay.itp[1] = it;
   }
 }

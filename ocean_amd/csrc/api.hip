@@ -304,7 +304,8 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   // adjoint: x-splits, phi' chunk and reduction rounds sharing one LDS area
   if (nb > t.adj) return OCEAN_GPU_ERR_ARG;
   const int XS = std::max(1, t.adj / nb);
-  g.adj_threads = nb * XS;
+  // whole waves (at most t.adj, a multiple of 64): a recursion's epilogue sums by waves
+  g.adj_threads = (nb * XS + 63) & ~63;
   const size_t resb = (size_t)na * nb * sizeof(double2);
   // two adjoint workgroups per CU while the result rows fit half the LDS; past that
   // the device's whole per-workgroup LDS (many bands at the L2,3 edge)
