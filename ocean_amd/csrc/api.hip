@@ -4,7 +4,6 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <type_traits>
 
@@ -13,6 +12,7 @@
 #include "gemm64.hpp"
 #include "obf.hpp"
 #include "setup.hpp"
+#include "staging.hpp"
 #include "vec.hpp"
 
 using og::kBlock;
@@ -115,24 +115,11 @@ int put_vec(H* h, const HostVec& v, double2* dst, size_t n) {
       p[2 * i + 1] = v.im ? v.im[i] : 0.0;
     }
   };
-  constexpr int T = 4;
-  std::thread th[T];
-  const int parts = n >= (size_t)1 << 18 ? T : 1;
-  auto at = [&](int t) { return n * t / parts; };
-  for (int t = 1; t < parts; ++t) {
-    try {
-      th[t] = std::thread(fill, at(t), at(t + 1));
-    } catch (const std::system_error&) {  // no thread to be had: this one fills the part below
-    }
-  }
-  int rc = OCEAN_GPU_OK;
-  for (int t = 0; t < parts; ++t) {
-    if (th[t].joinable()) th[t].join();
-    else fill(at(t), at(t + 1));
-    if (rc == 0 && hipMemcpyAsync(dst + at(t), p + 2 * at(t), (at(t + 1) - at(t)) * sizeof(double2),
-                                  hipMemcpyHostToDevice, h->stream) != hipSuccess)
-      rc = OCEAN_GPU_ERR_HIP;
-  }
+  auto send = [&](size_t a, size_t b) -> int {
+    OG_CHECK(hipMemcpyAsync(dst + a, p + 2 * a, (b - a) * sizeof(double2), hipMemcpyHostToDevice, h->stream));
+    return OCEAN_GPU_OK;
+  };
+  const int rc = og::stage(n, n >= (size_t)1 << 18 ? og::kStageParts : 1, fill, send);
   OG_TRY(rc);
   OG_CHECK(hipStreamSynchronize(h->stream));
   return OCEAN_GPU_OK;
