@@ -119,10 +119,11 @@ int put_vec(H* h, const HostVec& v, double2* dst, size_t n) {
     OG_CHECK(hipMemcpyAsync(dst + a, p + 2 * a, (b - a) * sizeof(double2), hipMemcpyHostToDevice, h->stream));
     return OCEAN_GPU_OK;
   };
-  const int rc = og::stage(n, n >= (size_t)1 << 18 ? og::kStageParts : 1, fill, send);
-  OG_TRY(rc);
-  OG_CHECK(hipStreamSynchronize(h->stream));
-  return OCEAN_GPU_OK;
+  auto wait = [&]() -> int {
+    OG_CHECK(hipStreamSynchronize(h->stream));
+    return OCEAN_GPU_OK;
+  };
+  return og::stage(n, n >= (size_t)1 << 18 ? og::kStageParts : 1, fill, send, wait);
 }
 
 int put_planes(H* h, const double* re, const double* im, double2* dst, size_t n) {

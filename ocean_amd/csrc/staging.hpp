@@ -11,8 +11,8 @@ namespace og {
 // first error; parts past it are filled but not sent.
 constexpr int kStageParts = 4;
 
-template <typename Fill, typename Send>
-int stage(size_t n, int parts, Fill fill, Send send) {
+template <typename Fill, typename Send, typename Wait>
+int stage(size_t n, int parts, Fill fill, Send send, Wait wait) {
   std::thread th[kStageParts];
   auto at = [&](int t) { return n * t / parts; };
   for (int t = 1; t < parts; ++t) {
@@ -27,7 +27,8 @@ int stage(size_t n, int parts, Fill fill, Send send) {
     else fill(at(t), at(t + 1));
     if (rc == 0) rc = send(at(t), at(t + 1));
   }
-  return rc;
+  const int rw = wait();
+  return rc ? rc : rw;
 }
 
 }  // namespace og

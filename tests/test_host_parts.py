@@ -33,6 +33,7 @@ int main() {
       for (int parts : {1, 4}) {
         std::vector<int> filled(n, 0), sent(n, 0);
         std::size_t next = 0;
+        int waits = 0;
         g_fail = fail;
         const int rc = og::stage(
             n, parts, [&](std::size_t a, std::size_t b) { for (; a < b; ++a) ++filled[a]; },
@@ -40,21 +41,22 @@ int main() {
               if (a != next) return 7;
               for (next = b; a < b; ++a) sent[a] += filled[a];
               return 0;
-            });
+            },
+            [&] { ++waits; return 0; });
         g_fail = false;
-        if (rc != 0 || next != n) return std::printf("rc %d, %zu of %zu\n", rc, next, n), 1;
+        if (rc != 0 || next != n || waits != 1) return std::printf("rc %d, %zu of %zu\n", rc, next, n), 1;
         for (std::size_t i = 0; i < n; ++i)
           if (filled[i] != 1 || sent[i] != 1) return std::printf("element %zu of %zu\n", i, n), 1;
       }
-  // an error ends the sending, not the filling
+  // an error ends the sending, not the filling, and what was sent is waited for
   std::vector<int> filled(8, 0);
-  int sends = 0;
+  int sends = 0, waits = 0;
   const int rc = og::stage(
       8, 4, [&](std::size_t a, std::size_t b) { for (; a < b; ++a) ++filled[a]; },
-      [&](std::size_t, std::size_t) { return ++sends == 2 ? 5 : 0; });
+      [&](std::size_t, std::size_t) { return ++sends == 2 ? 5 : 0; }, [&] { ++waits; return 6; });
   for (int f : filled)
     if (f != 1) return 1;
-  return rc == 5 && sends == 2 ? 0 : 1;
+  return rc == 5 && sends == 2 && waits == 1 ? 0 : 1;
 }
 """
 
