@@ -11,7 +11,7 @@ ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libocean_gpu.so")
 SRC = [os.path.join(HERE, "csrc", "api.hip")]
 DEPS = [os.path.join(HERE, "csrc", f) for f in ("common.hpp", "action.hpp", "vec.hpp", "obf.hpp", "gemm64.hpp", "setup.hpp",
-                                                "staging.hpp")] + \
+                                                "staging.hpp", "workspace.hpp")] + \
     [os.path.join(ROOT, "include", "ocean_gpu.h")]
 
 HIPCC_FLAGS = [

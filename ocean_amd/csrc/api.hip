@@ -14,6 +14,7 @@
 #include "setup.hpp"
 #include "staging.hpp"
 #include "vec.hpp"
+#include "workspace.hpp"
 
 using og::kBlock;
 using og::kRedBlocks;
@@ -35,16 +36,53 @@ int grid_for(size_t n) {
   return (int)std::min<size_t>(std::max<size_t>(g, 1), 4096);
 }
 
+struct HipDev {
+  static bool alloc(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();  // or the next launch would be taken to have failed
+    *p = nullptr;
+    return false;
+  }
+  static void free(void* p) { (void)hipFree(p); }  // waits for the device
+};
+
+// The vectors of a solve are one workspace of its handle (or batch), kept between calls: one
+// by one they cost an allocation and a synchronising free each (206 of each at a GMRES
+// depth of 100).  Up to kKeepWs bytes stay with one owner and up to kKeepTotal with all
+// of them (0.4 % of the device), and an allocation of this library that fails gives the
+// idle ones back first.  The pool outlives every handle: it is never destroyed.
+constexpr size_t kKeepWs = (size_t)256 << 20, kKeepTotal = (size_t)1 << 30;
+og::WorkspacePool<HipDev>& pool() {
+  static auto* p = new og::WorkspacePool<HipDev>(kKeepWs, kKeepTotal);
+  return *p;
+}
+
 template <typename T>
 int dmalloc(T** p, size_t n) {
-  *p = nullptr;
-  if (n == 0) n = 1;
-  if (hipMalloc((void**)p, n * sizeof(T)) != hipSuccess) {
-    *p = nullptr;
-    return OCEAN_GPU_ERR_NOMEM;
-  }
-  return OCEAN_GPU_OK;
+  void* q = nullptr;
+  const bool ok = pool().alloc(&q, std::max<size_t>(n, 1) * sizeof(T));
+  *p = ok ? static_cast<T*>(q) : nullptr;
+  return ok ? OCEAN_GPU_OK : OCEAN_GPU_ERR_NOMEM;
 }
+
+// One call's use of a workspace, ended on every way out.
+class WsUse {
+ public:
+  explicit WsUse(og::Workspace& w) : w_(w) {}
+  WsUse(const WsUse&) = delete;
+  WsUse& operator=(const WsUse&) = delete;
+  ~WsUse() { if (p_) pool().give(w_); }
+  int take(size_t n) {
+    if (!pool().take(w_, n * sizeof(double2))) return OCEAN_GPU_ERR_NOMEM;
+    p_ = static_cast<double2*>(w_.p);
+    return OCEAN_GPU_OK;
+  }
+  double2* get() const { return p_; }
+
+ private:
+  og::Workspace& w_;
+  double2* p_ = nullptr;
+};
 
 template <typename T>
 void dfree(T*& p) {
@@ -70,26 +108,6 @@ int ensure_pin(H* h, size_t ndouble) {
   }
   h->host_pin_n = ndouble;
   return OCEAN_GPU_OK;
-}
-
-// Device workspace of n elements in one piece: a solve's vectors one by one cost an
-// allocation and a synchronising free each (206 of each at a GMRES depth of 100).  Up to
-// kKeepWs bytes stay with their owner until it is destroyed; more goes back after the
-// call (give_ws).
-constexpr size_t kKeepWs = (size_t)256 << 20;
-
-int take_ws(double2** ws, size_t* have, size_t n) {
-  if (*have >= n) return OCEAN_GPU_OK;
-  dfree(*ws);
-  *have = 0;
-  OG_TRY(dmalloc(ws, n));
-  *have = n;
-  return OCEAN_GPU_OK;
-}
-void give_ws(double2** ws, size_t* have) {
-  if (*have * sizeof(double2) <= kKeepWs) return;
-  dfree(*ws);
-  *have = 0;
 }
 
 // A host vector: planes (step 1, im may be null) or interleaved (im = re + 1, step 2).
@@ -1257,7 +1275,7 @@ int ocean_gpu_destroy(ocean_gpu_handle* h) {
   dfree(h->energy); dfree(h->allow); dfree(h->red); dfree(h->scal); dfree(h->tmp_in); dfree(h->tmp_out);
   for (auto& v : h->vecs) dfree(v);
   if (h->pin_ctl) (void)hipHostFree(h->pin_ctl);
-  dfree(h->ws);
+  pool().drop(h->ws);
   if (h->host_pin) (void)hipHostFree(h->host_pin);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -1823,8 +1841,9 @@ int haydock_run(H* h, const HostVec& psi0, int niter, const EarlyExit* ex, doubl
   double* db = dai + n1;
   double* conv = da + ns;                 // [iter][relArea, maxDiff]
   double* cpart = conv + 2 * n1;
-  OG_TRY(take_ws(&h->ws, &h->ws_n, 3 * nv));
-  double2 *psi = h->ws, *old = psi + nv, *hv = old + nv;
+  WsUse ws(h->ws);
+  OG_TRY(ws.take(3 * nv));
+  double2 *psi = ws.get(), *old = psi + nv, *hv = old + nv;
   int rc = put_vec(h, psi0, psi, nv);
   int done = niter;
   // early exit: the convergence figures are formed on the device every iteration
@@ -1886,7 +1905,6 @@ int haydock_run(H* h, const HostVec& psi0, int niter, const EarlyExit* ex, doubl
         hipStreamSynchronize(h->stream) != hipSuccess)
       rc = OCEAN_GPU_ERR_HIP;
   }
-  give_ws(&h->ws, &h->ws_n);
   if (rc) return rc;
   for (int i = 0; i < done; ++i)
     if (hb[i] != hb[i]) { done = i + 1; rc = OCEAN_GPU_ERR_NAN; break; }
@@ -1950,9 +1968,10 @@ int haydock_multi_run(H* h, const HostVec& psi0, int niter, double* real_a, doub
   const size_t n1 = (size_t)niter + 1;
   const size_t nscal = hay_scalars(h, n1);
   OG_TRY(ensure_scal(h, (size_t)R * nscal));
-  OG_TRY(take_ws(&h->ws, &h->ws_n, 3 * nv));
+  WsUse ws(h->ws);
+  OG_TRY(ws.take(3 * nv));
   double* S = h->scal;
-  double2* V[3] = {h->ws, h->ws + nv, h->ws + 2 * nv};
+  double2* V[3] = {ws.get(), ws.get() + nv, ws.get() + 2 * nv};
   int rc = put_vec(h, psi0, V[0], nv);
   // rotation r of an iteration: (psi, old, hv) = (V0, V1, V2), (V2, V0, V1), (V1, V2, V0)
   const int rot[3][3] = {{0, 1, 2}, {2, 0, 1}, {1, 2, 0}};
@@ -1998,7 +2017,6 @@ int haydock_multi_run(H* h, const HostVec& psi0, int niter, double* real_a, doub
     }
     if (niter_done) niter_done[q] = done;
   }
-  give_ws(&h->ws, &h->ws_n);
   return rc ? rc : rc_nan;
 }
 
@@ -2355,23 +2373,24 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
   const size_t o_part = take(npart * sizeof(double)), o_L = take((nd * (nd - 1) / 2 + 1) * sizeof(double2));
   const size_t o_D = take(nd * sizeof(double)), o_C = take(nd * sizeof(double2)), o_RU = take(nd * sizeof(double2));
   const size_t o_ctl = take(sizeof(GmCtl));
-  OG_TRY(take_ws(&h->ws, &h->ws_n, at));
+  WsUse ws(h->ws);
+  OG_TRY(ws.take(at));
+  double2* const base = ws.get();
   if (!h->pin_ctl && hipHostMalloc(&h->pin_ctl, sizeof(GmCtl), hipHostMallocDefault) != hipSuccess) {
     h->pin_ctl = nullptr;
     return OCEAN_GPU_ERR_NOMEM;
   }
   std::vector<double2*> V(nfix + 2 * nd);
-  for (size_t i = 0; i < V.size(); ++i) V[i] = h->ws + i * ld;
-  double2* dcoef = h->ws + o_coef;
-  double* part = reinterpret_cast<double*>(h->ws + o_part);
-  double2* dL = h->ws + o_L;
-  double* dD = reinterpret_cast<double*>(h->ws + o_D);
-  double2* dC = h->ws + o_C;    // cumulative least-squares coefficients of the cycle
-  double2* dRU = h->ws + o_RU;  // <rhs|U_i>
-  GmCtl* ctl = reinterpret_cast<GmCtl*>(h->ws + o_ctl);
+  for (size_t i = 0; i < V.size(); ++i) V[i] = base + i * ld;
+  double2* dcoef = base + o_coef;
+  double* part = reinterpret_cast<double*>(base + o_part);
+  double2* dL = base + o_L;
+  double* dD = reinterpret_cast<double*>(base + o_D);
+  double2* dC = base + o_C;    // cumulative least-squares coefficients of the cycle
+  double2* dRU = base + o_RU;  // <rhs|U_i>
+  GmCtl* ctl = reinterpret_cast<GmCtl*>(base + o_ctl);
   GmCtl* hctl = static_cast<GmCtl*>(h->pin_ctl);
   int rc = OCEAN_GPU_OK;
-  auto cleanup = [&]() { give_ws(&h->ws, &h->ws_n); };
   int* skip = &ctl->done;
   int* info = &ctl->info;
   double2 *rhs = V[0], *h1 = V[1], *x = V[2], *ax = V[3], *g = V[4], *pc = V[5];
@@ -2585,7 +2604,6 @@ int gmres_run(H* h, const double2* rhs_dev, int nE, const double* energies_eV, d
                ? OCEAN_GPU_OK : OCEAN_GPU_ERR_HIP;
   }
   if (rc == 0 && hipStreamSynchronize(st) != hipSuccess) rc = OCEAN_GPU_ERR_HIP;
-  cleanup();
   return rc;
 }
 
@@ -2799,8 +2817,7 @@ struct ocean_gpu_batch {
   std::vector<Group> groups;
   hipStream_t stream = nullptr;
   int* dcount = nullptr;  // [0] Haydock iteration number, [1] its copy for k_hay2
-  double2* ws = nullptr;  // the recursions' vectors and scalars, kept up to kKeepWs bytes
-  size_t ws_n = 0;
+  og::Workspace ws;       // the recursions' vectors and scalars
   double t_last = 0.0;    // ms per batched action (all problems) of the last timed call
 };
 
@@ -2876,8 +2893,10 @@ int build_tables(const B* b, const B::Group& g, const std::vector<const double2*
   for (int i = 0; i < 5; ++i) tb.nblk[i] = off[(size_t)i * (np + 1) + np];
   tb.threads[0] = t.proj;
   tb.threads[2] = t.adj;
-  OG_CHECK(hipMalloc(&tb.args, sizeof(og::ActArgs<T2>) * (size_t)np));
-  if (hipMalloc((void**)&tb.off, sizeof(int) * off.size()) != hipSuccess) { tb.release(); return OCEAN_GPU_ERR_NOMEM; }
+  og::ActArgs<T2>* args = nullptr;
+  OG_TRY(dmalloc(&args, (size_t)np));
+  tb.args = args;
+  if (dmalloc(&tb.off, off.size())) { tb.release(); return OCEAN_GPU_ERR_NOMEM; }
   if (hipMemcpy(tb.args, host.data(), sizeof(og::ActArgs<T2>) * (size_t)np, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(tb.off, off.data(), sizeof(int) * off.size(), hipMemcpyHostToDevice) != hipSuccess) {
     tb.release();
@@ -2996,7 +3015,7 @@ int ocean_gpu_batch_create(ocean_gpu_handle* const* hs, int32_t n, ocean_gpu_bat
     }
     b->hs.push_back(hs[i]);
   }
-  if (hipStreamCreate(&b->stream) != hipSuccess || hipMalloc((void**)&b->dcount, 2 * sizeof(int)) != hipSuccess) {
+  if (hipStreamCreate(&b->stream) != hipSuccess || dmalloc(&b->dcount, (size_t)2)) {
     ocean_gpu_batch_destroy(b);
     return OCEAN_GPU_ERR_HIP;
   }
@@ -3033,7 +3052,7 @@ int ocean_gpu_batch_destroy(ocean_gpu_batch* b) {
   if (!b) return OCEAN_GPU_OK;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   if (b->dcount) (void)hipFree(b->dcount);
-  dfree(b->ws);
+  pool().drop(b->ws);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
   return OCEAN_GPU_OK;
@@ -3221,11 +3240,12 @@ int batch_haydock_run(ocean_gpu_batch* b, const std::vector<HostVec>& psi0, int 
   const size_t n1 = (size_t)niter + 1;
   size_t tot = 0;
   for (H* h : b->hs) tot += 3 * h->nvec() + (hay_scalars(h, n1) + 1) / 2;
-  OG_TRY(take_ws(&b->ws, &b->ws_n, tot));
+  WsUse ws(b->ws);
+  OG_TRY(ws.take(tot));
   std::vector<double2*> V((size_t)3 * n, nullptr);
   std::vector<double*> Sd((size_t)n, nullptr);
   int rc = OCEAN_GPU_OK;
-  double2* at = b->ws;
+  double2* at = ws.get();
   for (int q = 0; q < n && rc == 0; ++q) {
     H* h = b->hs[q];
     for (int i = 0; i < 3; ++i, at += h->nvec()) V[(size_t)3 * q + i] = at;
@@ -3340,7 +3360,6 @@ int batch_haydock_run(ocean_gpu_batch* b, const std::vector<HostVec>& psi0, int 
   for (auto& tr : tabs)
     for (auto& t : tr) t.release();
   for (int r = 0; r < 3; ++r) dfree(dhay[r]);
-  give_ws(&b->ws, &b->ws_n);
   return rc ? rc : rc_nan;
 }
 

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/ocean_gpu.h"
+#include "workspace.hpp"
 
 #define OG_CHECK(expr)                                                         \
   do {                                                                         \
@@ -267,8 +268,7 @@ struct ocean_gpu_handle {
   size_t scal_n = 0;
   double* host_pin = nullptr;  // pinned staging for host planes
   size_t host_pin_n = 0;
-  double2* ws = nullptr;       // the solvers' vectors, kept between calls up to kKeepWs bytes
-  size_t ws_n = 0;
+  og::Workspace ws;            // the solvers' vectors, kept between calls
   void* pin_ctl = nullptr;     // pinned copy of the GMRES control state
   double2* tmp_in = nullptr;   // host-plane xact staging
   double2* tmp_out = nullptr;

@@ -48,3 +48,30 @@ def test_workspace_is_shared_by_the_solves():
         assert np.array_equal(g.gmres(inp.psi0, e, 0.5, 13.605, 1e-12, 20), rows)
         for x, y in zip(first, again):
             assert np.array_equal(x, y)
+
+
+def test_kept_workspaces_are_bounded_over_all_handles():
+    """Eight handles whose solves take 216 MiB each: no more than 1 GiB of it stays with them
+    (one more workspace if the runtime holds on to what was freed last, and 64 MiB for
+    code and the handles' own small buffers)."""
+    hip = C.CDLL("libamdhip64.so.7")  # the runtime the library already loaded
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    inp = synth.make_inputs(nb=8, kmesh=(16, 16, 16), xmesh=(2, 2, 2), lc=1, seed=97, xi_eV=3.0)
+    gs = [core.OceanGPU.from_inputs(inp) for _ in range(8)]
+    before = free()
+    for g in gs:
+        g.gmres(inp.psi0, np.array([3.0]), 0.5, 13.605, 1e-2, 15, return_status=True)
+    used = before - free()
+    print("kept", used, flush=True)
+    assert used <= (1 << 30) + (216 << 20) + (64 << 20)
+    want = gs[0].haydock(inp.psi0, 3)
+    for g in gs[1:]:  # with and without a kept workspace
+        for x, y in zip(g.haydock(inp.psi0, 3), want):
+            assert np.array_equal(x, y)
+    for g in gs:
+        g.close()
