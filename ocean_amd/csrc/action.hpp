@@ -1070,41 +1070,10 @@ __global__ void k_wgrad(const T2* __restrict__ PX, const T2* __restrict__ PY, in
 }
 
 // h(i) = mul * sum_j K(i, j) amp(j): direct -mpm a plus exchange X a
-// (OCEAN_multiplet.f90:1812-1936); one wave per row, coalesced rows of K.  With
-// several right-hand sides K is block diagonal over blocks of nj0 amplitudes and a
-// row sums its own block only (so a NaN in one right-hand side stays there).
-__device__ __forceinline__ void mred_matvec(const double2* __restrict__ K, const double2* amp,
-                                            double2* __restrict__ hmult, int nj, int nj0, double mul) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int i = wid; i < nj; i += nw) {
-    double2 acc = make_double2(0.0, 0.0);
-    const int j0 = i - i % nj0;
-    for (int j = j0 + lane; j < j0 + nj0; j += 64) cfma(acc, K[(size_t)i * nj + j], amp[j]);
-    acc.x = wave_sum(acc.x);
-    acc.y = wave_sum(acc.y);
-    if (lane == 0) hmult[i] = make_double2(acc.x * mul, acc.y * mul);
-  }
-}
-
-// Stand-alone reduction (used when the long-range term is off): one workgroup.
-__global__ __launch_bounds__(1024) void k_mred(
-    const double2* __restrict__ apart, const double2* __restrict__ K, double2* __restrict__ hmult,
-    int np, int nj, int nj0, double mul) {
-  __shared__ double2 amp[kMaxAlpha * 64];
-  for (int j = threadIdx.x; j < nj; j += blockDim.x) {
-    double2 a = make_double2(0.0, 0.0);
-    for (int m = 0; m < np; ++m) {
-      const double2 v = apart[(size_t)m * nj + j];
-      a.x += v.x;
-      a.y += v.y;
-    }
-    amp[j] = a;
-  }
-  __syncthreads();
-  mred_matvec(K, amp, hmult, nj, nj0, mul);
-}
-
-// Reduction run by extra workgroups of another kernel's grid: workgroup r forms
+// (OCEAN_multiplet.f90:1812-1936), where amp are the summed partials.  With several
+// right-hand sides K is block diagonal over blocks of nj0 amplitudes and a row sums its own
+// block only (so a NaN in one right-hand side stays there).  Run by extra workgroups of
+// another kernel's grid, or on their own (k_mred): workgroup r forms
 // kRedPerBlock rows of h.  Every workgroup sums the np partials of all nj0 amplitudes of
 // its rows' right-hand side (64 x 64 to 64 x 192 values, from L2) and applies its rows of
 // K to them, so that no workgroup waits for another: with the amplitudes shared out
@@ -1153,6 +1122,16 @@ __device__ void mred_rows(const double2* __restrict__ apart, const double2* __re
     acc.y = wave_sum(acc.y);
     if (lane == 0) hmult[i] = make_double2(acc.x * mul, acc.y * mul);
   }
+}
+
+// The reduction on its own, where the long-range term is off and there is no transform to
+// ride on: rows of four per workgroup as there.  With all rows in one workgroup the 64 partials
+// of an amplitude were one thread's serial chain: 64 amplitudes 20.0 -> 4.0 us (and 12.8 with
+// one partial per k, before they were blocked).
+__global__ __launch_bounds__(kBlock) void k_mred(const double2* __restrict__ apart, const double2* __restrict__ K,
+                                                 double2* __restrict__ hmult, int np, int nj, int nj0, double mul) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  mred_rows(apart, K, hmult, np, nj, nj0, mul, blockIdx.x, reinterpret_cast<double2*>(smem));
 }
 
 // ---------------------------------------------------------------------------

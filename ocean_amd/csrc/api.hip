@@ -422,14 +422,13 @@ int xact_t(H* h, const double2* in, double2* out, int flags, T2* u, T2* uT, T2* 
       OG_CHECK(hipEventRecord(ev[2], h->stream));
     }
   }
-  if ((flags & og::F_FG) && !(flags & og::F_LR)) {
+  if ((flags & og::F_FG) && !(flags & og::F_LR) && h->P > 0) {
     const int nm = mult_blocks(h, kBlock / 64);
-    if (h->P > 0) {
-      og::k_mproj<NA><<<nm * ((h->P + 15) / 16) * h->ns, kBlock, 0, h->stream>>>(
-          h->cproj, in, h->allow, h->apart, h->nb, h->nk, h->na, h->ns, h->P, nm);
-      OG_CHECK(hipGetLastError());
-    }
-    og::k_mred<<<1, 1024, 0, h->stream>>>(h->apart, h->Kmat, h->hmult, nm, a.nj, h->na0 * h->P, a.mul);
+    og::k_mproj<NA><<<nm * ((h->P + 15) / 16) * h->ns, kBlock, 0, h->stream>>>(
+        h->cproj, in, h->allow, h->apart, h->nb, h->nk, h->na, h->ns, h->P, nm);
+    OG_CHECK(hipGetLastError());
+    og::k_mred<<<(a.nj + og::kRedPerBlock - 1) / og::kRedPerBlock, kBlock, og::mred_lds(h->na0 * h->P, kBlock / 64),
+                 h->stream>>>(h->apart, h->Kmat, h->hmult, nm, a.nj, h->na0 * h->P, a.mul);
     OG_CHECK(hipGetLastError());
   }
   if (ev) OG_CHECK(hipEventRecord(ev[3], h->stream));

@@ -86,3 +86,27 @@ def test_haydock_obf_at_adjoint_budget(adj):
         g.set_tiles(256, adj, 0, -1)
         a, b, _ = g.haydock(inp.psi0, N)
     _check(a, b, (ra, rb), adj)
+
+
+@pytest.mark.parametrize("kw,nrhs,n", [
+    (dict(nb=3, kmesh=(1, 1, 1), xmesh=(3, 2, 1), seed=121), 1, 5),    # one partial; the Krylov space has 6 vectors
+    (dict(nb=65, kmesh=(3, 5, 5), xmesh=(5, 14, 1), seed=122), 1, N),  # 38 partials
+    (dict(nb=9, kmesh=(8, 8, 5), xmesh=(3, 3, 1), lc=1, lmax=4, seed=123, xi_eV=2.0), 2, N),
+    (dict(nb=18, kmesh=(3, 4, 5), xmesh=(3, 3, 2), nspn=2, seed=124), 1, N)])
+def test_haydock_without_the_long_range_term(kw, nrhs, n):
+    """The multiplet term's own two kernels (no transform to ride on) and b finished on its
+    own: 1 to 64 partials, 16 and 25 projectors, two spins, two right-hand sides."""
+    inp = synth.make_inputs(**kw)
+    P = to_problem(inp, long_range=False)
+    rng = np.random.default_rng(9)
+    psis = []
+    for _ in range(nrhs):
+        z = rng.standard_normal(inp.psi0.shape) + 1j * rng.standard_normal(inp.psi0.shape)
+        psis.append(np.asfortranarray(z / np.linalg.norm(z)))
+    with core.OceanGPU.from_inputs(inp, long_range=False, nrhs=nrhs) as g:
+        a, b, _ = g.haydock_multi(psis, n)
+    for r, p in enumerate(psis):
+        ra, rb, _, ierr = orc.haydock(P, p, n)
+        assert ierr == 0
+        assert np.max(np.abs(a[r, :n] - ra[:n]) / np.abs(ra[:n])) < 1e-10
+        assert np.max(np.abs(b[r, 1:n + 1] - rb[1:n + 1]) / np.abs(rb[1:n + 1])) < 1e-10
