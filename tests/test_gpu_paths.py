@@ -230,6 +230,24 @@ def test_gmres_recycled_basis_past_the_lds_factor(nb, depth, rows):
     assert np.abs(got[:, 2] - ref[:, 2]).max() <= tol
 
 
+@pytest.mark.parametrize("nb,rows", [(8, 142), (5, 129), (1, 1)])
+def test_gmres_recycled_basis_reaches_its_rows_on_the_device(nb, rows):
+    """One unbroken cycle (no restart: the global count stays within the depth) whose basis
+    on the device passes 141 rows (the factor read from global memory), 128 rows, or
+    belongs to 32 unknowns, half a wave.  The bar of the test above."""
+    inp = synth.make_inputs(nb=nb, kmesh=(2, 2, 2), xmesh=(3, 3, 3), lc=0, seed=61)
+    P = to_problem(inp)
+    E = np.array([12.0, 12.1, 12.3, 12.5])
+    depth, ffff, gam = 256, 1e-16, 0.1
+    ref = orc.gmres_do_recycle(P, inp.psi0, E, gam, 13.605, ffff, depth, inp.kpref)
+    with core.OceanGPU.from_inputs(inp) as g:
+        got = g.gmres(inp.psi0, E, gam, 13.605, ffff, depth)
+    print(ref[:, [2, 4, 5]], got[:, [2, 4, 5]], flush=True)
+    assert rows <= got[-1, 5] <= depth
+    tol = 2 * inp.kpref * np.linalg.norm(inp.allow * inp.psi0) * np.sqrt(ffff) / (gam * core.EV2HARTREE)
+    assert np.abs(got[:, 2] - ref[:, 2]).max() <= tol
+
+
 def test_nan_in_start_vector_stops_at_first_iteration():
     inp = synth.make_inputs(nb=8, kmesh=(2, 2, 2), xmesh=(3, 3, 3), lc=0, seed=62)
     psi = inp.psi0.copy()

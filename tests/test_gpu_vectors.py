@@ -75,3 +75,40 @@ def test_kept_workspaces_are_bounded_over_all_handles():
             assert np.array_equal(x, y)
     for g in gs:
         g.close()
+
+
+def test_stacked_and_batched_planes_agree_with_interleaved():
+    """ocean_gpu_haydock_multi and ocean_gpu_batch_haydock (host planes) against their
+    interleaved forms, bit for bit; imag_a and niter_done may be null."""
+    lib, n = core._lib(), 7
+    inps = [synth.make_inputs(nb=9, kmesh=(3, 2, 4), xmesh=(3, 3, 3), lc=0, seed=98),
+            synth.make_inputs(nb=13, kmesh=(2, 2, 2), xmesh=(3, 3, 3), lc=1, seed=99, xi_eV=3.0)]
+    rng = np.random.default_rng(4)
+    with core.OceanGPU.from_inputs(inps[0], nrhs=3) as g:
+        psi = np.asfortranarray(rng.standard_normal(g.shape) + 1j * rng.standard_normal(g.shape)) / 30
+        want = g.haydock_multi(psi, n)
+        re, im = np.asfortranarray(psi.real), np.asfortranarray(psi.imag)
+        a, b, ai = (np.zeros((3, n + 1)) for _ in range(3))
+        done = np.zeros(3, np.int32)
+        assert lib.ocean_gpu_haydock_multi(g.h, core._p(re), core._p(im), n, *(x.ctypes.data_as(core._DP) for x in (a, b, ai)),
+                                           done.ctypes.data_as(core._IP)) == 0
+        assert list(done) == [n] * 3 and all(np.array_equal(x, y) for x, y in zip((a, b, ai), want))
+        assert lib.ocean_gpu_haydock_multi(g.h, core._p(re), core._p(im), n, a.ctypes.data_as(core._DP),
+                                           b.ctypes.data_as(core._DP), None, None) == 0
+        assert np.array_equal(a, want[0]) and np.array_equal(b, want[1])
+    gs = [core.OceanGPU.from_inputs(i) for i in inps]
+    bt = core.OceanBatch(gs)
+    want, _ = bt.haydock([i.psi0 for i in inps], n)
+    planes = [[np.asfortranarray(p) for p in (i.psi0.real, i.psi0.imag)] for i in inps]
+    outs = [[np.zeros(n + 1) for _ in inps] for _ in range(3)]
+    table = lambda arrays: (core._DP * 2)(*[x.ctypes.data_as(core._DP) for x in arrays])  # noqa: E731
+    pr, pi = table([p[0] for p in planes]), table([p[1] for p in planes])
+    done = np.zeros(2, np.int32)
+    assert lib.ocean_gpu_batch_haydock(bt.b, pr, pi, n, *(table(o) for o in outs), done.ctypes.data_as(core._IP)) == 0
+    assert list(done) == [n, n]
+    for q in range(2):
+        assert all(np.array_equal(o[q], w) for o, w in zip(outs, want[q]))
+    assert lib.ocean_gpu_batch_haydock(bt.b, pr, None, n, *(table(o) for o in outs), None) == 1001
+    bt.close()
+    for g in gs:
+        g.close()
