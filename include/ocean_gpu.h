@@ -420,8 +420,8 @@ int  ocean_gpu_tridiag_eigs(const double* real_a, const double* real_b, int32_t 
  * adjoint thread budget, transform strip width (0 = widest), adjoint form (1 the
  * matrix-core adjoint with its fused epilogue, 0 the VALU adjoint, -1 the default,
  * the matrix cores; it applies to many alphas on one spin)) as the handle stores
- * them (the FP32 projection runs half as many threads per x at four alphas or fewer
- * and twice as many at more). */
+ * them.  Projection and adjoint sizes are in threads; a projection wave takes 32 x
+ * points in FP64 and 64 in FP32, whose workgroups are at most 512 threads. */
 int  ocean_gpu_autotune(ocean_gpu_handle* h, int32_t reps);
 int  ocean_gpu_get_tiles(ocean_gpu_handle* h, int32_t* tiles);
 /* Sets the handle's tiles[4] as ocean_gpu_get_tiles reports them (OCEAN_GPU_ERR_ARG

@@ -515,6 +515,10 @@ __device__ __forceinline__ void proj_dispatch(const ActArgs<T2>& A, int b, int n
   proj_body<T2, NA>(A, bx, k, s, smem);
 }
 
+// Four waves per SIMD at every alpha count.  At 24 the cap makes the compiler spill 17
+// registers per lane in FP64 and 8 in FP32; three waves spill none.  us, capped -> not: 512
+// k points, 512 x, 64 bands FP64 86.5 -> 83, FP32 52 -> 50.5; 256 bands 336 -> 327, 160 ->
+// 163; 64 k points, 1000 x, 64 bands 33.0 -> 33.9, 24.8 -> 26.1.
 template <typename T2, int NA>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_proj(const ActArgs<T2> A) {
   if (skipped(A)) return;
@@ -547,6 +551,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 //   512 k points, 2 048 columns: FP64 18.2 -> 15.3, FP32 16.9 -> 13.0
 //   512 k points, 12 000 columns, 192 amplitudes: FP64 54.8 -> 45.9, FP32 47.7 -> 27.4
 //   64 k points, 864 columns, FP64: 12.6 -> 7.1
+// The FP64 24-edge class holds two arrays of 24 values: all 256 registers, 2 to 7 of them
+// spilled, and half the time of the plain sums (24 x 24 x 2 k points, 864 columns: 119 ->
+// 55; 24 x 4 x 4: 27 -> 14).
 // ---------------------------------------------------------------------------
 template <int L>
 __device__ __forceinline__ constexpr int bitrev(int i) {

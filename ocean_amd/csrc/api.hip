@@ -266,7 +266,11 @@ int make_args(const H* h, const double2* in, double2* out, int flags, const Tile
   if (t.proj < 64 || t.proj > 512 || (t.proj & 63)) return OCEAN_GPU_ERR_ARG;
   // A psi of the k (nb rounded up to the steps of four, nalpha complex) in LDS, and beside
   // it the phi tiles on their way out: contiguous rows on one spin only, and where both
-  // fit (24 alphas with more than about 340 bands: straight from the registers)
+  // fit (24 alphas with more than about 340 bands: straight from the registers).  Many bands
+  // leave fewer workgroups per CU (12 alphas FP64: four at 128 bands, two at 256, one from
+  // 384), and the ring of loads makes up for them: against staging at most 64 KB, us, 12
+  // alphas FP64: 256 bands, 512 k points, 512 x 292 -> 216; 512 bands, 64 k points, 1000 x 242 ->
+  // 124; two spins, 256 bands (six alphas each) 380 -> 395, the most that was lost
   const int nw = t.proj / 64;
   a.px = (nx + og::proj_xt<T2>() * nw - 1) / (og::proj_xt<T2>() * nw);
   g.sm_proj = ((size_t)((nb + 3) & ~3) * acnt * sizeof(T2) + 15) & ~(size_t)15;
@@ -882,7 +886,8 @@ __device__ __forceinline__ void ls_sweeps(Lf Lat, const double* fin, const doubl
 }
 
 // LDS of k_ls_update: the sums, the pivots and, where it fits, the packed factor (up to
-// 141 rows in 160 KB; past that the sweeps read L from global memory).
+// 141 rows in 160 KB; past that the sweeps read L from global memory, with four indices
+// per lane, which spills 12 registers under the 128 that 1024 threads leave).
 size_t ls_lds(int cur, bool with_L) {
   const size_t j = (size_t)cur - 1;
   return (4 * (size_t)cur + cur + (cur & 1)) * sizeof(double) + (with_L ? (j * (j - 1) / 2 + 1) * sizeof(double2) : 0);

@@ -38,7 +38,7 @@ constexpr int kMaxDim = 24;      // largest k-mesh edge handled by the LDS DFT
 
 // Tile shapes of the action kernels (defaults; the autotuner picks per batch group).
 struct Tiles {
-  int proj = 256;  // projection workgroup size (x-points per workgroup)
+  int proj = 256;  // projection threads: a wave per 32 x points in FP64, 64 in FP32 (proj_xt)
   int adj = 512;   // adjoint thread budget (x-splits = adj / nb)
   int G = 0;       // transform columns per strip, 0 = the largest that fits
   int adj_mf = -1; // many alphas on one spin: 1 the matrix-core adjoint with its fused

@@ -309,7 +309,9 @@ __device__ __forceinline__ void adj_lr_body(const ActArgs<T2>& A, int bx, int k)
 }
 
 constexpr int kAdjRing = 3;
-// waves per SIMD: FP64 tiles at three waves spill their ring (227 -> 267 us)
+// waves per SIMD: FP64 tiles at three waves spill their ring (227 -> 267 us).  24 alphas in
+// FP64 spill 34 registers at two waves and are faster with them than at one wave without:
+// 512 k points, 512 x, 64 / 128 / 256 bands 92 / 186 / 336 us against 103 / 199 / 386.
 template <typename T2, int NA> constexpr int adj_lr_waves() { return sizeof(T2) == 8 && NA <= 12 ? 4 : 2; }
 
 template <typename T2, int NA, int MT, int W>
